@@ -5,8 +5,9 @@
 // wave groups rotating between matrix work, exponentials and data movement)
 // on launches of at least kP3MinGrid of its workgroups, else attn_pp_kernel
 // (256 rows, two groups alternating between matrix work and data
-// movement), both described at the kernel; head_dim 64 runs
-// attn_fwd_kernel, described here.
+// movement), both described at the kernel; launches that leave compute units
+// idle split their keys (split_plan).  head_dim 64 runs attn_fwd_kernel,
+// described here.
 //
 // Work decomposition.  A workgroup of 8 waves owns 256 query rows (32 per
 // wave) of one (query sequence, head) pair and streams that pair's keys in
@@ -84,12 +85,11 @@ struct AttnParams {
   int Hq, kv_per_head, q_tiles, n_wg;
   int64_t q_tok, q_head, kv_tok, kv_head, o_tok, o_head;
   float scale_log2;
-  // key-split launches (attn_p3_kernel<true> + attn_combine_kernel): the
-  // per-item partial results and item records in the caller's workspace
+  // key-split launches (attn_pp_kernel<true> + attn_combine_kernel): the
+  // items' partial results in the caller's workspace
   float *part;
-  int4 *rec;
   int n_seq, n_cu;
-  // queue launches of attn_p3_kernel<false> (one workgroup per compute
+  // queue launches of attn_p3_kernel (one workgroup per compute
   // unit, items claimed from per-XCD counters): this stream's counter
   // block; null = one item per workgroup
   int *queue;
@@ -320,119 +320,141 @@ __device__ void queue_done(int *queue) {
   }
 }
 
-// One item of a key-split launch: query tile qt of sequence seq against key
-// tiles [t_lo, t_hi) (32 keys each) of its k chunks (chunk j); the items of
-// sequence seq are numbered base + j * nq + qt.
-struct SplitItem {
-  int seq, qt, j, k, nq, base, t_lo, t_hi;
+// ---- key-split launches ----------------------------------------------------
+// A launch whose query tiles leave compute units without one (a few heads,
+// short frames, a single head over a long context) splits sequences' keys
+// into chunks, one workgroup of attn_pp_kernel<true> per (query tile, chunk);
+// attn_combine_kernel then merges a tile's chunks in chunk order.  What
+// bounds such a launch is its longest workgroup, not the chip: 42 tiles of
+// 3,000-8,000 keys took 163 us on 42 of 256 units, 49 us split over 219.
+//
+// Every wave of both launches computes the same plan from cu_q / cu_k in
+// registers (no LDS, no barrier; lane i holds sequences i, i + 64, ...).
+// Keys are counted in units of kSplitUnit tiles, the key loop's unroll.  With
+// at most R * n_cu items (R = 1, and 2 when the launch has room for it) the
+// chunk length C is the smallest that fits, at least kSplitMinUnits; sequence
+// s has k_s = ceil(units_s / C) chunks of equal length (+-1 unit).  Chosen is
+// the least estimated time in units (an item costs its units and
+// kSplitItemUnits more; a unit is 2.6-3.1 us):
+//   unsplit  longest
+//   R = 1    C + kSplitFixedUnits
+//   R = 2    sum of the items' units / n_cu + C / 3 + 2 * kSplitFixedUnits
+// (the fixed part is the second launch and the partial results' traffic, C / 3
+// the unevenness of a second round).  Measured against all the alternatives
+// on 28 shapes of 6-252 tiles it took the fastest one or one within 5%: for
+// instance 168 tiles of 12,480-17,160 keys 353 us unsplit, 337 in one round
+// and 290 in two; 209 tiles of 3,000-5,000 keys 118, 130 and 130; 81 tiles of
+// 3,200-5,000 keys 112, 64 and 75.
+// Items are numbered base_s + j * nq_s + qt, so a chunk's query tiles are
+// consecutive and, numbered by xcd_remap, share their keys in one XCD's L2.
+constexpr int kSplitSeqLanes = 4;                    // sequences per lane
+constexpr int kSplitMaxSeqs = 64 * kSplitSeqLanes;   // sequences a key-split launch may have
+constexpr int kSplitUnit = 4;                        // 32-key tiles per unit
+constexpr int kSplitMinUnits = 4;                    // shortest chunk (512 keys)
+constexpr int kSplitItemUnits = 3;
+constexpr int kSplitFixedUnits = 4;
+
+struct SplitPlan {
+  int nq[kSplitSeqLanes], nu[kSplitSeqLanes], k[kSplitSeqLanes], base[kSplitSeqLanes];
+  int n_items;
 };
 
-constexpr int kSplitRows = 384;  // query rows per item (attn_p3_kernel's workgroup)
-constexpr int kSplitKeys = 32;   // keys per key tile (attn_p3_kernel's kPK)
+// One item: query tile qt of sequence seq (of nq tiles) against units
+// [u_lo, u_hi) of its keys, chunk j of k; the tile's chunk 0 is item `first`.
+struct SplitItem {
+  int seq, qt, nq, k, j, first, u_lo, u_hi;
+};
 
-// Key-split plan, computed by every workgroup of the launch in its prologue
-// (the same on each, from cu_q / cu_k alone).  Sequence s has nq_s query tiles
-// of kSplitRows rows and nkt_s key tiles; its keys split into
-// k_s = ceil(nkt_s / C) chunks of equal length (+-1 tile).  The chunk length
-// C is chosen among ceil(nkt_max / k), k = 1 .. kSplitMaxChunks, as the one
-// with the least estimated time ceil(items / n_cu) * (C + kSplitItemTiles)
-// (rounds of items over the compute units, each item's fixed cost counted
-// as kSplitItemTiles key tiles; fewer items on ties) among those with at
-// most n_items items.  Items are ranked by chunk length (longest first, ties
-// by sequence index), and a sequence's items ordered (chunk, query tile):
-// the query tiles of one chunk are consecutive, so they run at the same time
-// on one XCD and read the same keys through its L2.  Returns false when item
-// c does not exist.  scratch: 6 * kSchedMax ints of LDS, 16-byte aligned;
-// every thread must call it.
-constexpr int kSplitMaxChunks = 8;
-constexpr int kSplitItemTiles = 8;
-__device__ bool split_item(const AttnParams &p, int n_items, int c, int *scratch, SplitItem &out) {
-  const int n_seq = p.n_seq;
-  int *nq = scratch, *nkt = scratch + kSchedMax, *cost = scratch + 2 * kSchedMax;
-  int *order = scratch + 3 * kSchedMax, *items = scratch + 4 * kSchedMax, *kk = scratch + 5 * kSchedMax;
-  __shared__ int acc[3];
-  __shared__ SplitItem res;
-  const int n4 = (n_seq + 3) & ~3;
-  if (threadIdx.x == 0) {
-    acc[0] = 1;  // largest nkt (at least 1)
-    acc[1] = 0;
-    res.seq = -1;
-  }
-  __syncthreads();
-  for (int s = threadIdx.x; s < n4; s += blockDim.x) {
-    int q = 0, t = 0;
-    if (s < n_seq) {
-      const int b = s / p.Hq;
-      q = (p.cu_q[b + 1] - p.cu_q[b] + kSplitRows - 1) / kSplitRows;
-      const int kv = p.kv_per_head ? s : b;
-      t = (p.cu_k[kv + 1] - p.cu_k[kv] + kSplitKeys - 1) / kSplitKeys;
-      if (q > 0) atomicMax(&acc[0], t);
+__device__ inline int div_up(int a, int b) {
+  return static_cast<int>(static_cast<unsigned>(a + b - 1) / static_cast<unsigned>(b));
+}
+
+__device__ inline SplitPlan split_plan(const AttnParams &p) {
+  SplitPlan s;
+  const int lane = threadIdx.x & 63;
+  auto wave_total = [](int x) { return __builtin_amdgcn_readlane(wave_incl_sum(x), 63); };
+  int tiles = 0, work = 0, longest = 0;
+#pragma unroll
+  for (int i = 0; i < kSplitSeqLanes; ++i) {
+    const int sq = lane + 64 * i;
+    s.nq[i] = s.nu[i] = 0;
+    if (sq < p.n_seq) {
+      const int b = sq / p.Hq, kv = p.kv_per_head ? sq : b;
+      // (no more tiles than the launch counted, whatever cu_q holds: every
+      // item then has a slot of the workspace)
+      s.nq[i] = min(div_up(max(0, p.cu_q[b + 1] - p.cu_q[b]), 32 * kWaves), p.q_tiles);
+      s.nu[i] = div_up(max(0, p.cu_k[kv + 1] - p.cu_k[kv]), 32 * kSplitUnit);
     }
-    nq[s] = q;
-    nkt[s] = t;
+    tiles += s.nq[i];
+    work += s.nq[i] * s.nu[i];
+    longest = max(longest, s.nu[i]);
   }
-  __syncthreads();
-  // chunk length: the candidate of least estimated time
-  const int nkt_max = acc[0];
-  int C = nkt_max;
-  int64_t best = -1;
-  for (int k1 = 1; k1 <= kSplitMaxChunks; ++k1) {
-    const int cand = (nkt_max + k1 - 1) / k1;
-    if (k1 > 1 && cand == (nkt_max + k1 - 2) / (k1 - 1)) continue;  // same length as k1 - 1
-    if (threadIdx.x == 0) acc[1] = 0;
-    __syncthreads();
-    int part = 0;
-    for (int s = threadIdx.x; s < n_seq; s += blockDim.x) part += nq[s] * max(1, (nkt[s] + cand - 1) / cand);
-    if (part) atomicAdd(&acc[1], part);
-    __syncthreads();
-    const int n_it = acc[1];
-    __syncthreads();
-    if (n_it > n_items) break;  // more chunks only add items
-    const int64_t t = static_cast<int64_t>((n_it + p.n_cu - 1) / p.n_cu) * (cand + kSplitItemTiles);
-    if (best < 0 || t < best) {
-      best = t;
-      C = cand;
+  tiles = wave_total(tiles);
+  work = wave_total(work);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  auto items = [&](int C) {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < kSplitSeqLanes; ++i) n += s.nq[i] * (s.nu[i] <= C ? 1 : div_up(s.nu[i], C));
+    return wave_total(n);
+  };
+  // chunk lengths are tried in [work / G, work / (G - tiles)]: no shorter one
+  // can fit G items, and that one does (items <= work / C + tiles)
+  auto shortest = [&](int G) {
+    int lo = max(kSplitMinUnits, work / G), hi = max(lo, min(longest, div_up(work, max(1, G - tiles))));
+    while (lo < hi) {
+      const int C = (lo + hi) >> 1;
+      if (items(C) <= G) hi = C;
+      else lo = C + 1;
+    }
+    return lo;
+  };
+  int C = max(1, longest), best = longest;
+  if (tiles < p.n_cu) {
+    const int c1 = shortest(p.n_cu);
+    if (c1 + kSplitFixedUnits < best) {
+      C = c1;
+      best = c1 + kSplitFixedUnits;
     }
   }
-  for (int s = threadIdx.x; s < n4; s += blockDim.x) {
-    int k = 1, cs = -1;
-    if (s < n_seq && nq[s] > 0) {
-      k = max(1, (nkt[s] + C - 1) / C);
-      cs = (nkt[s] + k - 1) / k + 1;  // +1: fixed cost per item
+  if (p.n_wg >= 2 * p.n_cu) {
+    const int c2 = shortest(2 * p.n_cu);
+    if ((work + kSplitItemUnits * (items(c2) - tiles)) / p.n_cu + c2 / 3 + 2 * kSplitFixedUnits < best) C = c2;
+  }
+  int run = 0;
+#pragma unroll
+  for (int i = 0; i < kSplitSeqLanes; ++i) {
+    s.k[i] = s.nu[i] <= C ? 1 : div_up(s.nu[i], C);
+    const int n = s.nq[i] * s.k[i], incl = wave_incl_sum(n);
+    s.base[i] = run + incl - n;
+    run += __builtin_amdgcn_readlane(incl, 63);
+  }
+  s.n_items = run;
+  return s;
+}
+
+// Item c < n_items of the plan; uniform over the wave.
+__device__ inline SplitItem split_item(const SplitPlan &s, int c) {
+  SplitItem r{};
+#pragma unroll
+  for (int i = 0; i < kSplitSeqLanes; ++i) {
+    const uint64_t hit = __ballot(c >= s.base[i] && c < s.base[i] + s.nq[i] * s.k[i]);
+    if (hit) {
+      const int src = __builtin_ctzll(hit);
+      r.seq = src + 64 * i;
+      r.nq = __builtin_amdgcn_readlane(s.nq[i], src);
+      r.k = __builtin_amdgcn_readlane(s.k[i], src);
+      const int nu = __builtin_amdgcn_readlane(s.nu[i], src), base = __builtin_amdgcn_readlane(s.base[i], src);
+      r.j = static_cast<int>(static_cast<unsigned>(c - base) / static_cast<unsigned>(r.nq));
+      r.qt = c - base - r.j * r.nq;
+      r.first = base + r.qt;
+      r.u_lo = static_cast<int>(static_cast<unsigned>(r.j * nu) / static_cast<unsigned>(r.k));
+      r.u_hi = static_cast<int>(static_cast<unsigned>((r.j + 1) * nu) / static_cast<unsigned>(r.k));
     }
-    kk[s] = k;
-    cost[s] = cs;
-    items[s] = s < n_seq ? nq[s] * k : 0;
   }
-  __syncthreads();
-  // rank = sequences before s in (cost desc, index asc) order
-  for (int s = threadIdx.x; s < n_seq; s += blockDim.x) {
-    const int cs = cost[s];
-    int r = 0;
-    for (int t = 0; t < n_seq; ++t) r += (cost[t] > cs) || (cost[t] == cs && t < s);
-    order[r] = s;
-  }
-  __syncthreads();
-  for (int r = threadIdx.x; r < n_seq; r += blockDim.x) {
-    int base = 0;
-    for (int rr = 0; rr < r; ++rr) base += items[order[rr]];
-    const int s = order[r];
-    if (c >= base && c < base + items[s]) {
-      const int local = c - base, q = nq[s], k = kk[s];
-      res.seq = s;
-      res.j = local / q;
-      res.qt = local % q;
-      res.k = k;
-      res.nq = q;
-      res.base = base;
-      res.t_lo = static_cast<int>(static_cast<int64_t>(res.j) * nkt[s] / k);
-      res.t_hi = static_cast<int>(static_cast<int64_t>(res.j + 1) * nkt[s] / k);
-    }
-  }
-  __syncthreads();
-  out = res;
-  __syncthreads();  // the scratch is reused by the caller
-  return out.seq >= 0;
+  return r;
 }
 
 __device__ inline uint4 ldg16(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
@@ -825,7 +847,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_fwd_kernel(AttnParams p) {
 constexpr int kPK = 32;                 // keys per tile
 constexpr int kPRow = 256;              // LDS bytes per key row (128 bf16)
 constexpr int kPTileElems = kPK * 128;  // bf16 elements per tile
-static_assert(kPK == kSplitKeys, "the key-split plan counts attn_p3_kernel's key tiles");
+static_assert(kPK == 32, "the key-split plan counts tiles of 32 keys");
 
 typedef __attribute__((address_space(3))) char lds_char;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -852,11 +874,18 @@ __device__ inline void pp_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// a key-split item's partial result: per wave its lanes' 64 O^T values
+// (16 float4 per lane, lane-minor) and then per wave and lane (reference, sum)
+constexpr int kPartOFloats = kWaves * 16 * 64 * 4;
+constexpr int kPartFloats = kPartOFloats + kWaves * 64 * 2;
+
+// SPLIT: one item of a key-split launch per workgroup (see split_plan)
+template <bool SPLIT>
 __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
   constexpr int D = 128;
   __shared__ __attribute__((aligned(16))) uint16_t Ka[kPTileElems], Kb[kPTileElems], Kc[kPTileElems], Kd[kPTileElems];
   __shared__ __attribute__((aligned(16))) uint16_t Va[kPTileElems], Vb[kPTileElems], Vc[kPTileElems], Vd[kPTileElems];
-  __shared__ __attribute__((aligned(16))) int sched[4 * kSchedMax];
+  __shared__ __attribute__((aligned(16))) int sched[SPLIT ? 4 : 4 * kSchedMax];
   auto kslot = [&](auto s) -> uint16_t * {
     constexpr int S = decltype(s)::value & 3;
     if constexpr (S == 0) return Ka;
@@ -873,12 +902,24 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
   };
 
   int seq, qt;
+  SplitItem it{};
+  int slot_idx = 0;
   const int n_seq = p.n_wg / p.q_tiles;
-  if (n_seq <= kSchedMax) {
+  if constexpr (SPLIT) {
+    const SplitPlan plan = split_plan(p);
+    if (static_cast<int>(blockIdx.x) >= plan.n_items) return;
+    slot_idx = xcd_remap(blockIdx.x, plan.n_items);
+    it = split_item(plan, slot_idx);
+    seq = it.seq;
+    qt = it.qt;
+  } else if (n_seq <= kSchedMax && p.n_wg > p.n_cu) {
     if (!balanced_item(p.cu_q, p.cu_k, p.Hq, n_seq, p.kv_per_head, 32 * kWaves, xcd_remap(blockIdx.x, p.n_wg),
                        sched, seq, qt))
       return;
   } else {
+    // all workgroups run at once: no order to keep, and the list costs its
+    // barriers (228 tiles of 512 keys 24.5 us in index order, 26.6 ranked;
+    // of 6,240-17,160 keys 390 and 416)
     const int wg = xcd_remap(blockIdx.x, p.n_wg);
     seq = wg / p.q_tiles;
     qt = wg % p.q_tiles;
@@ -889,8 +930,13 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
   const int q0 = qt * 32 * kWaves;
   if (q0 >= Lq) return;
   const int kv_idx = p.kv_per_head ? seq : b;
-  const int k_begin = p.cu_k[kv_idx];
-  const int Lk = p.cu_k[kv_idx + 1] - k_begin;
+  int k_begin = p.cu_k[kv_idx];
+  int Lk = p.cu_k[kv_idx + 1] - k_begin;
+  if constexpr (SPLIT) {  // this item's chunk of the keys
+    const int lo = min(it.u_lo * kSplitUnit * kPK, Lk), hi = min(it.u_hi * kSplitUnit * kPK, Lk);
+    k_begin += lo;
+    Lk = hi - lo;
+  }
   const uint16_t *qp = p.q + static_cast<int64_t>(q_begin) * p.q_tok + h * p.q_head;
   const int64_t kv_off = static_cast<int64_t>(k_begin) * p.kv_tok + (p.kv_per_head ? 0 : h * p.kv_head);
   const uint16_t *kp = p.k + kv_off;
@@ -1201,6 +1247,21 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
     }
   }
 
+  if constexpr (SPLIT) {
+    if (it.k > 1) {
+      // this chunk's partial result, in the lane layout attn_combine_kernel reads
+      if (!wave_rows) return;
+      float *slot = p.part + static_cast<int64_t>(slot_idx) * kPartFloats;
+      float4 *po = reinterpret_cast<float4 *>(slot) + wave * 16 * 64 + lane;
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        po[j * 64] = make_float4(o[j / 4][4 * (j % 4)], o[j / 4][4 * (j % 4) + 1], o[j / 4][4 * (j % 4) + 2],
+                                 o[j / 4][4 * (j % 4) + 3]);
+      reinterpret_cast<float2 *>(slot + kPartOFloats)[wave * 64 + lane] = make_float2(m, l);
+      return;
+    }
+  }
+
   // ---- epilogue: O = O^T / l
   uint16_t *op = p.o + static_cast<int64_t>(q_begin) * p.o_tok + h * p.o_head;
   const float lt = half_sum(l);
@@ -1283,13 +1344,6 @@ constexpr int kP3Waves = 12;
 constexpr int kP3Threads = 64 * kP3Waves;
 constexpr int kP3Rows = 32 * kP3Waves;
 constexpr int kP3MinGrid = 1024;  // workgroups: four per CU
-// a key-split item's partial result: per wave its lanes' 64 O^T values
-// (16 float4 per lane, lane-minor) and then per wave and lane (r, l)
-constexpr int kPartOFloats = kP3Waves * 16 * 64 * 4;
-constexpr int kPartFloats = kPartOFloats + kP3Waves * 64 * 2;
-
-static_assert(kP3Rows == kSplitRows, "a key-split item is one attn_p3_kernel workgroup");
-
 // A sequence's last query tile holds Lq mod 384 rows -- 72 of the 4,680 of a
 // rollout's query chunk -- so in the plain work shape three of its twelve
 // waves have rows, and the tile took 82% of a full workgroup's time for 19%
@@ -1565,21 +1619,10 @@ __device__ __attribute__((always_inline)) inline void tail_item(const AttnParams
   }
 }
 
-// SPLIT: the workgroup runs item xcd_remap(blockIdx.x) of the key-split plan
-// (split_item): one query tile against one chunk of its sequence's keys.
-// An item whose sequence has one chunk writes O as the plain kernel does;
-// otherwise it writes its partial result (unnormalised O^T, the reference r
-// its probabilities were taken against -- 0, m, or the slow pass's final
-// maximum -- and the row sum l, per lane) to part slot c, and
-// attn_combine_kernel merges a query tile's chunks.  Every workgroup writes
-// its item's record (k = 0 when the item does not exist).
 // One work item of attn_p3_kernel: query tile qt (kP3Rows rows) of
-// sequence seq against all of its keys, or, in a key-split launch, against
-// the chunk of keys that `it` names.  Every wave takes every barrier of the
-// item; waves leave only after the item's last barrier.
-template <bool SPLIT>
-__device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &p, uint16_t *kv, int seq, int qt,
-                                                              const SplitItem &it) {
+// sequence seq against all of its keys.  Every wave takes every barrier of
+// the item; waves leave only after the item's last barrier.
+__device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &p, uint16_t *kv, int seq, int qt) {
   auto kslot = [&](auto s) -> uint16_t * { return kv + (decltype(s)::value & 3) * kPTileElems; };
   auto vslot = [&](auto s) -> uint16_t * { return kv + (4 + (decltype(s)::value & 3)) * kPTileElems; };
   uint16_t *const Ka = kslot(ic<0>()), *const Kb = kslot(ic<1>()), *const Kc = kslot(ic<2>()), *const Kd = kslot(ic<3>());
@@ -1590,13 +1633,8 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
   const int q0 = qt * kP3Rows;
   if (q0 >= Lq) return;
   const int kv_idx = p.kv_per_head ? seq : b;
-  int k_begin = p.cu_k[kv_idx];
-  int Lk = p.cu_k[kv_idx + 1] - k_begin;
-  if constexpr (SPLIT) {  // this item's chunk of the keys
-    const int lo = min(it.t_lo * kPK, Lk), hi = min(it.t_hi * kPK, Lk);
-    k_begin += lo;
-    Lk = hi - lo;
-  }
+  const int k_begin = p.cu_k[kv_idx];
+  const int Lk = p.cu_k[kv_idx + 1] - k_begin;
   const uint16_t *qp = p.q + static_cast<int64_t>(q_begin) * p.q_tok + h * p.q_head;
   const int64_t kv_off = static_cast<int64_t>(k_begin) * p.kv_tok + (p.kv_per_head ? 0 : h * p.kv_head);
   const uint16_t *kp = p.k + kv_off;
@@ -1615,11 +1653,9 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
   const bool wave_rows = q0 + wave_s * 32 < Lq;
   const float c = p.scale_log2;
 
-  if constexpr (!SPLIT) {
-    if (Lq - q0 <= kTailRows && (Lk + kPK - 1) / kPK >= kTailMinTiles) {
-      tail_item(p, kv, qp, kp, vp, q_begin, Lq, q0, h, Lk);
-      return;
-    }
+  if (Lq - q0 <= kTailRows && (Lk + kPK - 1) / kPK >= kTailMinTiles) {
+    tail_item(p, kv, qp, kp, vp, q_begin, Lq, q0, h, Lk);
+    return;
   }
 
   bf16x8 qr[8];
@@ -1639,7 +1675,6 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
   float m = -INFINITY, l = 0.0f;
-  float ref = 0.0f;  // the reference P was taken against (partial results of key-split items)
   const int nT = (Lk + kPK - 1) / kPK;
 
   // ---- tile copies (groups 0 and 1): buffer resources based at the tile's
@@ -1888,7 +1923,6 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
     wait_vm<0>();  // no copy may land in LDS after the workgroup ends
     // every tile's sums were rebased below 2^kHeadroom (or flagged)
     ovf = ovf || !(l < exp2f(kHeadroom));
-    ref = m;
     if (ovf) ovf_any = 1;
     __syncthreads();
     if (ovf_any) {
@@ -1931,22 +1965,6 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
         }
         __syncthreads();
       }
-      ref = m;
-    }
-  }
-
-  if constexpr (SPLIT) {
-    if (it.k > 1) {
-      // partial result of this chunk, in the lane layout attn_combine_kernel reads
-      if (!wave_rows) return;
-      float *slot = p.part + static_cast<int64_t>(xcd_remap(blockIdx.x, p.n_wg)) * kPartFloats;
-      float4 *po = reinterpret_cast<float4 *>(slot) + wave * 16 * 64 + lane;
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        po[j * 64] = make_float4(o[j / 4][4 * (j % 4)], o[j / 4][4 * (j % 4) + 1], o[j / 4][4 * (j % 4) + 2],
-                                 o[j / 4][4 * (j % 4) + 3]);
-      reinterpret_cast<float2 *>(slot + kPartOFloats)[wave * 64 + lane] = make_float2(ref, l);
-      return;
     }
   }
 
@@ -1972,7 +1990,6 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
   }
 }
 
-template <bool SPLIT>
 __global__ void __launch_bounds__(kP3Threads, 1) attn_p3_kernel(AttnParams p) {
   // the eight tile slots (K 0-3, V 4-7) in one 64 KB array at the start of
   // LDS, so that every fragment read addresses its slot by an immediate
@@ -1980,102 +1997,100 @@ __global__ void __launch_bounds__(kP3Threads, 1) attn_p3_kernel(AttnParams p) {
   // issued before the work list is read)
   // (a tail item uses sixteen slots: its own K and V pairs per key quarter)
   __shared__ __attribute__((aligned(16))) uint16_t kv[16 * kPTileElems];
-  static_assert(8 * kPTileElems * 2 >= 6 * kSchedMax * 4, "work-list scratch fits in the tile slots");
+  static_assert(8 * kPTileElems * 2 >= 4 * kSchedMax * 4, "work-list scratch fits in the tile slots");
   int *sched = reinterpret_cast<int *>(kv);
-  if constexpr (SPLIT) {
-    SplitItem it{};
-    const int c = xcd_remap(blockIdx.x, p.n_wg);
-    const bool ok = split_item(p, p.n_wg, c, sched, it);
-    if (threadIdx.x == 0) p.rec[c] = ok ? make_int4(it.seq, it.qt, it.j | (it.k << 16), it.nq) : make_int4(0, 0, 0, 0);
-    if (!ok) return;
-    p3_item<true>(p, kv, it.seq, it.qt, it);
-  } else {
-    const int n_seq = p.n_wg / p.q_tiles;
-    __shared__ QueueTable tab;
-    if (p.queue) queue_table(p.cu_q, p.cu_k, p.Hq, n_seq, p.kv_per_head, kP3Rows, sched, tab);
-    unsigned spent = 0;  // queue mode: the bins this workgroup found empty (thread 0)
-    for (bool first = true;; first = false) {
-      int seq, qt;
-      if (p.queue) {
-        if (!queue_next(p.queue, tab, spent, seq, qt)) break;
+  const int n_seq = p.n_wg / p.q_tiles;
+  __shared__ QueueTable tab;
+  if (p.queue) queue_table(p.cu_q, p.cu_k, p.Hq, n_seq, p.kv_per_head, kP3Rows, sched, tab);
+  unsigned spent = 0;  // queue mode: the bins this workgroup found empty (thread 0)
+  for (bool first = true;; first = false) {
+    int seq, qt;
+    if (p.queue) {
+      if (!queue_next(p.queue, tab, spent, seq, qt)) break;
+    } else {
+      // one item per workgroup, in the XCD-balanced order
+      if (!first) break;
+      if (n_seq <= kSchedMax) {
+        if (!balanced_item(p.cu_q, p.cu_k, p.Hq, n_seq, p.kv_per_head, kP3Rows, xcd_remap(blockIdx.x, p.n_wg),
+                           sched, seq, qt))
+          break;
       } else {
-        // one item per workgroup, in the XCD-balanced order
-        if (!first) break;
-        if (n_seq <= kSchedMax) {
-          if (!balanced_item(p.cu_q, p.cu_k, p.Hq, n_seq, p.kv_per_head, kP3Rows, xcd_remap(blockIdx.x, p.n_wg),
-                             sched, seq, qt))
-            break;
-        } else {
-          const int wg = xcd_remap(blockIdx.x, p.n_wg);
-          seq = wg / p.q_tiles;
-          qt = wg % p.q_tiles;
-        }
+        const int wg = xcd_remap(blockIdx.x, p.n_wg);
+        seq = wg / p.q_tiles;
+        qt = wg % p.q_tiles;
       }
-      p3_item<false>(p, kv, seq, qt, SplitItem{});
     }
-    if (p.queue) queue_done(p.queue);
+    p3_item(p, kv, seq, qt);
   }
+  if (p.queue) queue_done(p.queue);
 }
 
-// Second launch of a key-split attention: item c with chunk j = 0 of a
-// split query tile (k > 1 chunks) merges the partial results of items
-// c + j' * nq, j' = 0 .. k-1, in that order: with M the largest reference,
-// O = sum_j' 2^(r_j' - M) O_j' / sum_j' 2^(r_j' - M) l_j' (fp32), written
-// as attn_p3_kernel's epilogue writes it.  Other items exit at once.
-__global__ void __launch_bounds__(kP3Threads) attn_combine_kernel(AttnParams p) {
-  const int c = blockIdx.x;
-  const int4 r = p.rec[c];
-  const int k = r.z >> 16, j = r.z & 0xffff;
-  if (k <= 1 || j != 0) return;
-  const int seq = r.x, qt = r.y, nq = r.w;
+// Second launch of a key-split attention: one workgroup per query tile and
+// wave of it (32 rows), each of its own waves one 32-dim block of O.  With M the
+// largest reference of the tile's chunks, O = sum_j 2^(r_j - M) O_j /
+// sum_j 2^(r_j - M) l_j in chunk order (fp32).  Tiles of one chunk, which
+// attn_pp_kernel wrote itself, exit at once.
+constexpr int kCombineWaves = 4;  // waves per workgroup: each takes one 32-dim block of the rows
+__global__ void __launch_bounds__(64 * kCombineWaves) attn_combine_kernel(AttnParams p) {
+  const int tile = blockIdx.x / kWaves, wave = blockIdx.x % kWaves;
+  const int seq = tile / p.q_tiles, qt = tile % p.q_tiles;
   const int b = seq / p.Hq, h = seq % p.Hq;
   const int q_begin = p.cu_q[b];
   const int Lq = p.cu_q[b + 1] - q_begin;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int lq = lane & 31, hf = lane >> 5;
-  const int q0 = qt * kP3Rows;
+  const int q0 = qt * 32 * kWaves;
   if (q0 + wave * 32 >= Lq) return;
-  auto slot = [&](int jj) { return p.part + static_cast<int64_t>(c + jj * nq) * kPartFloats; };
+  const SplitPlan s = split_plan(p);
+  int k = 1, nq = 0, first = 0;
+#pragma unroll
+  for (int i = 0; i < kSplitSeqLanes; ++i)
+    if (seq >> 6 == i) {
+      k = __builtin_amdgcn_readlane(s.k[i], seq & 63);
+      nq = __builtin_amdgcn_readlane(s.nq[i], seq & 63);
+      first = __builtin_amdgcn_readlane(s.base[i], seq & 63) + qt;
+    }
+  if (k <= 1) return;
+  const int lane = threadIdx.x & 63, db = threadIdx.x >> 6;
+  const int lq = lane & 31, hf = lane >> 5;
+  const float *part = p.part + static_cast<int64_t>(first) * kPartFloats;
+  const int64_t step = static_cast<int64_t>(nq) * kPartFloats;
+  const float2 *rl = reinterpret_cast<const float2 *>(part + kPartOFloats) + wave * 64 + lane;
+  const float4 *po = reinterpret_cast<const float4 *>(part) + (wave * 16 + 4 * db) * 64 + lane;
   float M = -INFINITY;
-  for (int jj = 0; jj < k; ++jj) M = fmaxf(M, reinterpret_cast<const float2 *>(slot(jj) + kPartOFloats)[wave * 64 + lane].x);
+#pragma unroll 4
+  for (int j = 0; j < k; ++j) M = fmaxf(M, reinterpret_cast<const float2 *>(reinterpret_cast<const float *>(rl) + j * step)->x);
   float l = 0.0f;
-  float4 acc[16];
+  float4 acc[4];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int jj = 0; jj < k; ++jj) {
-    const float *sp = slot(jj);
-    const float2 rl = reinterpret_cast<const float2 *>(sp + kPartOFloats)[wave * 64 + lane];
-    const float w = __builtin_amdgcn_exp2f(rl.x - M);
-    l = fmaf(w, rl.y, l);
-    const float4 *po = reinterpret_cast<const float4 *>(sp) + wave * 16 * 64 + lane;
+  for (int g = 0; g < 4; ++g) acc[g] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+  for (int j = 0; j < k; ++j) {
+    const float2 v2 = *reinterpret_cast<const float2 *>(reinterpret_cast<const float *>(rl) + j * step);
+    const float4 *pj = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(po) + j * step);
+    const float w = __builtin_amdgcn_exp2f(v2.x - M);
+    l = fmaf(w, v2.y, l);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float4 v = po[i * 64];
-      acc[i].x = fmaf(w, v.x, acc[i].x);
-      acc[i].y = fmaf(w, v.y, acc[i].y);
-      acc[i].z = fmaf(w, v.z, acc[i].z);
-      acc[i].w = fmaf(w, v.w, acc[i].w);
+    for (int g = 0; g < 4; ++g) {
+      const float4 v = pj[g * 64];
+      acc[g].x = fmaf(w, v.x, acc[g].x);
+      acc[g].y = fmaf(w, v.y, acc[g].y);
+      acc[g].z = fmaf(w, v.z, acc[g].z);
+      acc[g].w = fmaf(w, v.w, acc[g].w);
     }
   }
   const float lt = half_sum(l);
   const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
   const int row_q = q0 + wave * 32 + lq;
-  if (row_q < Lq) {
-    uint16_t *orow = p.o + static_cast<int64_t>(q_begin + row_q) * p.o_tok + h * p.o_head;
+  if (row_q >= Lq) return;
+  uint16_t *orow = p.o + static_cast<int64_t>(q_begin + row_q) * p.o_tok + h * p.o_head;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = db * 32 + 8 * g + 4 * hf;
-        const float4 v = acc[4 * db + g];
-        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-        bf16x4 o4;
-        o4[0] = static_cast<__bf16>(v.x * inv);
-        o4[1] = static_cast<__bf16>(v.y * inv);
-        o4[2] = static_cast<__bf16>(v.z * inv);
-        o4[3] = static_cast<__bf16>(v.w * inv);
-        *reinterpret_cast<bf16x4 *>(orow + d) = o4;
-      }
+  for (int g = 0; g < 4; ++g) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    bf16x4 o4;
+    o4[0] = static_cast<__bf16>(acc[g].x * inv);
+    o4[1] = static_cast<__bf16>(acc[g].y * inv);
+    o4[2] = static_cast<__bf16>(acc[g].z * inv);
+    o4[3] = static_cast<__bf16>(acc[g].w * inv);
+    *reinterpret_cast<bf16x4 *>(orow + db * 32 + 8 * g + 4 * hf) = o4;
   }
 }
 
@@ -2135,44 +2150,49 @@ static int *queue_for(hipStream_t st) {
   return q;
 }
 
-// Items a key-split launch may have: three per compute unit.
-static int64_t split_items() { return 3 * static_cast<int64_t>(device_cus()); }
-static int64_t split_ws_bytes(int64_t items) {
-  return items * (static_cast<int64_t>(kPartFloats) * 4 + static_cast<int64_t>(sizeof(int4)));
+// Items a key-split launch of `tiles` query tiles may have: one per compute
+// unit, or two where one round would leave units idle at its end (above 3/8
+// of the units in tiles).
+static int64_t split_items(int64_t tiles) { return device_cus() * static_cast<int64_t>(8 * tiles > 3 * device_cus() ? 2 : 1); }
+static int64_t split_ws_bytes() { return 2 * static_cast<int64_t>(device_cus()) * kPartFloats * 4; }
+
+// Query tiles of a launch that may split its keys, 0 for one that may not:
+// head_dim 128, at most kSplitMaxSeqs sequences and tiles on at most 9/10 of
+// the units (252 tiles of 256 units gain nothing: 416 us unsplit, 424-444
+// split), and keys for at least two chunks of the shortest length in the
+// longest sequence, whose estimate then beats the unsplit one (max_seqlen_k
+// bounds the keys of a sequence; 0 = unknown).
+static int64_t split_tiles(const pkv_attn_args *a, int64_t max_seqlen_k) {
+  const int64_t seqs = static_cast<int64_t>(a->num_batches) * a->num_heads_q;
+  const int64_t tiles = seqs * ((static_cast<int64_t>(a->max_seqlen_q) + 32 * kWaves - 1) / (32 * kWaves));
+  const bool keys = max_seqlen_k <= 0 || max_seqlen_k > 32 * kSplitUnit * (kSplitMinUnits + kSplitFixedUnits);
+  return a->head_dim == 128 && seqs <= kSplitMaxSeqs && 10 * tiles <= 9 * device_cus() && keys ? tiles : 0;
 }
 
-// Key-split launch (head_dim 128): attn_p3_kernel<true> over n items, then
-// attn_combine_kernel.  Returns -1 when the launch does not qualify (the
-// caller then runs the plain kernels).
+// Key-split launch: attn_pp_kernel<true> over as many workgroups as it may
+// have items, then attn_combine_kernel.  Returns -1 when the launch does not
+// qualify (the caller then runs the plain kernels).
 static int launch_split(const pkv_attn_args *a, void *ws, int64_t ws_bytes, hipStream_t st) {
-  const int64_t seqs = static_cast<int64_t>(a->num_batches) * a->num_heads_q;
-  const int64_t q_tiles = (a->max_seqlen_q + kP3Rows - 1) / kP3Rows;
-  const int64_t n = split_items();
-  // small launches only: those the 12-wave kernel would not fill the chip with
-  // per-head keys only (the cache's attention; a shared key sequence, as in
-  // cross-attention to a short text context, gains nothing from splitting)
-  if (!ws || a->head_dim != 128 || !a->kv_per_head || n <= 0 || seqs > kSchedMax ||
-      seqs * q_tiles >= kP3MinGrid || seqs * q_tiles > n || ws_bytes < split_ws_bytes(n))
-    return -1;
+  const int64_t tiles = split_tiles(a, 0), n = split_items(tiles);
+  if (!ws || tiles == 0 || ws_bytes < split_ws_bytes()) return -1;
   AttnParams p{};
   p.q = a->q; p.k = a->k; p.v = a->v; p.o = a->o;
   p.cu_q = a->cu_seqlens_q; p.cu_k = a->cu_seqlens_k;
   p.Hq = a->num_heads_q;
   p.kv_per_head = a->kv_per_head;
-  p.q_tiles = static_cast<int>(q_tiles);
+  p.n_seq = a->num_batches * a->num_heads_q;
+  p.q_tiles = static_cast<int>(tiles / p.n_seq);
   p.n_wg = static_cast<int>(n);
-  p.n_seq = static_cast<int>(seqs);
   p.n_cu = device_cus();
   p.q_tok = a->q_tok_stride; p.q_head = a->q_head_stride;
   p.kv_tok = a->kv_tok_stride; p.kv_head = a->kv_head_stride;
   p.o_tok = a->o_tok_stride; p.o_head = a->o_head_stride;
   p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
   p.part = static_cast<float *>(ws);
-  p.rec = reinterpret_cast<int4 *>(static_cast<char *>(ws) + n * static_cast<int64_t>(kPartFloats) * 4);
-  hipLaunchKernelGGL(attn_p3_kernel<true>, dim3(p.n_wg), dim3(kP3Threads), 0, st, p);
-  int rc = check_launch("attn_p3_kernel");
+  hipLaunchKernelGGL(attn_pp_kernel<true>, dim3(p.n_wg), dim3(kThreads), 0, st, p);
+  int rc = check_launch("attn_pp_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(p.n_wg), dim3(kP3Threads), 0, st, p);
+  hipLaunchKernelGGL(attn_combine_kernel, dim3(static_cast<unsigned>(tiles * kWaves)), dim3(64 * kCombineWaves), 0, st, p);
   return check_launch("attn_combine_kernel");
 }
 
@@ -2198,20 +2218,22 @@ static int launch_attn(const pkv_attn_args *a, hipStream_t st) {
   p.o_tok = a->o_tok_stride; p.o_head = a->o_head_stride;
   p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
   if (p.n_wg == 0) return PKV_OK;
+  p.n_cu = device_cus();
   if (p3) {
     // a queue launch (one workgroup per compute unit) when the XCD-balanced
     // work list covers the sequences and this stream has a counter block
     const int cus = device_cus();
     p.queue = seqs <= kSchedMax && cus > 0 && p.n_wg > cus ? queue_for(st) : nullptr;
-    hipLaunchKernelGGL(attn_p3_kernel<false>, dim3(p.queue ? cus : p.n_wg), dim3(kP3Threads), 0, st, p);
+    hipLaunchKernelGGL(attn_p3_kernel, dim3(p.queue ? cus : p.n_wg), dim3(kP3Threads), 0, st, p);
     return check_launch("attn_p3_kernel");
   }
-  if (D == 128) {
-    hipLaunchKernelGGL(attn_pp_kernel, dim3(p.n_wg), dim3(kThreads), 0, st, p);
+  if constexpr (D == 128) {
+    hipLaunchKernelGGL(attn_pp_kernel<false>, dim3(p.n_wg), dim3(kThreads), 0, st, p);
     return check_launch("attn_pp_kernel");
+  } else {
+    hipLaunchKernelGGL((attn_fwd_kernel<D>), dim3(p.n_wg), dim3(kThreads), 0, st, p);
+    return check_launch("attn_fwd_kernel");
   }
-  hipLaunchKernelGGL((attn_fwd_kernel<D>), dim3(p.n_wg), dim3(kThreads), 0, st, p);
-  return check_launch("attn_fwd_kernel");
 }
 
 }  // namespace pkv
@@ -2236,9 +2258,11 @@ static int attn_check(const pkv_attn_args *a) {
   return 0;
 }
 
-extern "C" int64_t pkv_ragged_attn_workspace_size(void) {
-  const int64_t n = split_items();
-  return n > 0 ? split_ws_bytes(n) : 0;
+extern "C" int64_t pkv_ragged_attn_workspace_size(void) { return split_ws_bytes(); }
+
+extern "C" int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *a, int64_t max_seqlen_k) {
+  if (!a || a->num_batches <= 0 || a->num_heads_q <= 0 || a->max_seqlen_q <= 0) return 0;
+  return split_tiles(a, max_seqlen_k) ? split_ws_bytes() : 0;
 }
 
 extern "C" int pkv_ragged_attn_fwd_ws(const pkv_attn_args *a, void *workspace, int64_t workspace_bytes,

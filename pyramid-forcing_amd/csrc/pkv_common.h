@@ -122,6 +122,20 @@ __device__ inline void stage_words(uint2 *lds, const uint2 *g, int n) {
   }
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave by DPP: row shifts 1, 2,
+// 4, 8 scan each 16-lane row, then lane 15 of rows 0 and 2 is added to rows
+// 1 and 3 (row_bcast:15) and lane 31 to rows 2 and 3 (row_bcast:31).  Lanes
+// whose source lies outside the row (or rows the mask leaves out) add 0.
+__device__ inline int32_t wave_incl_sum(int32_t x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return x;
+}
+
 // ---- error plumbing (host) --------------------------------------------------
 
 void set_error(const char *fmt, ...);

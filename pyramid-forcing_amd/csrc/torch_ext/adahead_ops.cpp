@@ -646,10 +646,12 @@ static int64_t mega_evict_merge_workspace_size(int64_t num_heads) {
 // _mega_cache.py:540-559).  q [total_q, Hq, D]; with kv_per_head k/v are
 // [total_k, D] (or [total_k, 1, D]) and cu_seqlens_k has num_batches*Hq+1
 // entries (sequence b*Hq+h); otherwise k/v are [total_k, Hq, D] with
-// cu_seqlens_k [num_batches+1].  Returns the output shaped like q.
+// cu_seqlens_k [num_batches+1].  max_seqlen_k bounds a sequence's keys (0 =
+// unknown): it only helps to tell which launches may gain from splitting
+// their keys.  Returns the output shaped like q.
 static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q, Tensor cu_seqlens_k,
                                int64_t max_seqlen_q, double softmax_scale, bool kv_per_head, bool causal,
-                               c10::optional<Tensor> workspace) {
+                               c10::optional<Tensor> workspace, int64_t max_seqlen_k) {
   TORCH_CHECK(q.is_cuda() && k.is_cuda() && v.is_cuda(), "ragged_attention: tensors must be on the GPU");
   TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 &&
                   v.scalar_type() == at::kBFloat16,
@@ -702,6 +704,15 @@ static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q
                 "ragged_attention: workspace must be a contiguous tensor on q's device");
     pkv_check(pkv_ragged_attn_fwd_ws(&a, w.data_ptr(), w.numel() * w.element_size(), stream_for(q)),
               "ragged_attention");
+    return out;
+  }
+  // a workspace of the stream's allocator for the launches that gain from one
+  // (no sequence has more keys than k has rows)
+  const int64_t rows = k.size(0);
+  const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 && max_seqlen_k < rows ? max_seqlen_k : rows);
+  if (need > 0) {
+    const Tensor w = at::empty({need}, q.options().dtype(at::kByte));
+    pkv_check(pkv_ragged_attn_fwd_ws(&a, w.data_ptr(), need, stream_for(q)), "ragged_attention");
   } else {
     pkv_check(pkv_ragged_attn_fwd(&a, stream_for(q)), "ragged_attention");
   }
@@ -1114,7 +1125,8 @@ static adahead::Plan7 plan_multi(Mgr mgr, Tensor, int64_t, Tensor t_list, int64_
                                  int64_t, int64_t, int64_t, double) {
   return plan_shapes(mgr, t_list.numel());
 }
-static Tensor attn(Tensor q, Tensor, Tensor, Tensor, Tensor, int64_t, double, bool, bool, c10::optional<Tensor>) {
+static Tensor attn(Tensor q, Tensor, Tensor, Tensor, Tensor, int64_t, double, bool, bool, c10::optional<Tensor>,
+                   int64_t) {
   return at::empty_like(q);
 }
 static Tensor rope(Tensor k, Tensor, Tensor, Tensor, Tensor) { return at::empty_like(k); }
@@ -1232,7 +1244,7 @@ TORCH_LIBRARY(adahead, m) {
         "Tensor(j!) merge_pos_pool, Tensor(k!) merge_token_count) -> ()");
   m.def("ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q, Tensor cu_seqlens_k, "
         "int max_seqlen_q, float softmax_scale, bool kv_per_head=True, bool causal=False, "
-        "Tensor? workspace=None) -> Tensor");
+        "Tensor? workspace=None, int max_seqlen_k=0) -> Tensor");
   m.def("ragged_attention_workspace_size() -> int");
   m.def("rope_apply(Tensor k, Tensor pos, Tensor freqs_ft_flat, Tensor freqs_fy_flat, Tensor freqs_fx_flat) "
         "-> Tensor");

@@ -22,7 +22,8 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
         raise NotImplementedError("grouped-query attention (different q / kv head counts) is not supported")
     qb = q if q.dtype == torch.bfloat16 else q.to(torch.bfloat16)
     out = _ops.ragged_attention(qb, k, v, cu_seqlens_q.to(torch.int32), cu_seqlens_k.to(torch.int32),
-                                int(max_seqlen_q), softmax_scale, kv_per_head=False, causal=causal)
+                                int(max_seqlen_q), softmax_scale, kv_per_head=False, causal=causal,
+                                max_seqlen_k=max_seqlen_k)
     return out if out.dtype == q.dtype else out.to(q.dtype)
 
 

@@ -37,6 +37,8 @@ from .lag import LagStrategy
 from .merge import MergeStrategy
 from .stride import StrideStrategy
 
+MAX_MERGE_TOKENS = 420  # tokens per Veil anchor
+
 _STRATEGY_TYPES = {c.__name__: c for c in (CyclicStrategy, StrideStrategy, LagStrategy, MergeStrategy)}
 
 _STRATEGY_NAME_TO_KIND = {"RecentStrategy": ref.SK_RECENT, "CyclicStrategy": ref.SK_CYCLIC,
@@ -64,6 +66,7 @@ class MegaCacheCtx:
     # per layer: any Veil (merge) head; layers without one skip the merge launches
     layer_has_merge: list = field(default_factory=list)
     layer_merge_heads: list = field(default_factory=list)  # per layer: bit h set for each Veil head h
+    layer_max_keys: list = field(default_factory=list)  # per layer: the most tokens a head's segments can hold
     sink_caps_per_head: torch.Tensor = None
     committed_vc: torch.Tensor = None
     freqs: torch.Tensor = None
@@ -75,9 +78,8 @@ class MegaCacheCtx:
     # (allocated on first use); restored when a pass for another block comes before the commit
     recent_backup: dict = field(default_factory=dict)
     cu_q: dict = field(default_factory=dict)
-    # key-split attention for attend (off by default: on a rollout's per-layer
-    # launches it measured no faster than the unsplit kernels) and the
-    # device's workspace for it (_ops.attention_workspace)
+    # attend's attention splits keys by its own rule in a workspace of the
+    # allocator's; with this switch in the device's (_ops.attention_workspace)
     split_attention: bool = False
     attn_workspace: torch.Tensor = None
 
@@ -230,7 +232,7 @@ class MegaCache:
         qb = q[0] if q.dtype == torch.bfloat16 else q[0].to(torch.bfloat16)
         out = _ops.ragged_attention(qb, ctx.mgr.k_flat_out().view(-1, D), ctx.mgr.v_flat_out().view(-1, D), cu_q,
                                     cu_k, FSEQ, softmax_scale, kv_per_head=True, causal=causal,
-                                    workspace=self._split_workspace(q.device))
+                                    workspace=self._split_workspace(q.device), max_seqlen_k=ctx.layer_max_keys[self.layer_idx])
         return out.view(1, L_q, H, D).to(q.dtype)
 
 
@@ -260,6 +262,13 @@ def _composition_to_perhead_state(composition: HeadComposition) -> ref.PerHeadSt
             s = cls.state_record(mid)
     s.sink_capacity = sink_cap
     return s
+
+
+def max_head_tokens(s: ref.PerHeadState, frame_seqlen: int, max_sink: int, max_recent: int) -> int:
+    """The most tokens that the segments of a head with record s can hold."""
+    middle = {ref.SK_CYCLIC: s.bucket_cap, ref.SK_STRIDE: s.capacity, ref.SK_LAG: s.capacity}.get(s.kind, 0)
+    merged = s.capacity * min(frame_seqlen, MAX_MERGE_TOKENS) if s.kind == ref.SK_MERGE else 0
+    return (max_sink + max_recent + middle) * frame_seqlen + merged
 
 
 def merge_head_mask(is_merge) -> int:
@@ -293,6 +302,7 @@ def build_mega_caches(num_layers: int, num_heads: int, head_dim: int, frame_seql
     any_merge = False
     layer_merge = []
     layer_heads = []
+    layer_keys = []
     for l in range(num_layers):
         if len(compositions[l]) != num_heads:
             raise ValueError(f"compositions[{l}] has {len(compositions[l])} heads, expected {num_heads}")
@@ -300,6 +310,7 @@ def build_mega_caches(num_layers: int, num_heads: int, head_dim: int, frame_seql
         layer_merge.append(any(s.kind == ref.SK_MERGE for s in per_head))
         any_merge = any_merge or layer_merge[-1]
         layer_heads.append(merge_head_mask([s.kind == ref.SK_MERGE for s in per_head]))
+        layer_keys.append(max(max_head_tokens(s, frame_seqlen, max_sink_frames, max_recent_frames) for s in per_head))
         for h, s in enumerate(per_head):
             sink_caps[l, h] = int(s.sink_capacity)
         states_np[l] = _mega_state_ops.pack_states(per_head)
@@ -319,7 +330,7 @@ def build_mega_caches(num_layers: int, num_heads: int, head_dim: int, frame_seql
                        history_relative_t_max=history_relative_t_max,
                        history_time_soft_factor=history_time_soft_factor, spatial_width=spatial_width,
                        spatial_height=spatial_height, has_merge_head=any_merge, layer_has_merge=layer_merge,
-                       layer_merge_heads=layer_heads,
+                       layer_merge_heads=layer_heads, layer_max_keys=layer_keys,
                        sink_caps_per_head=torch.from_numpy(sink_caps).to(device=device).contiguous(), freqs=freqs,
                        freq_parts=freq_parts, freq_parts_flat=freq_parts_flat,
                        pending_block=[None] * num_layers)

@@ -79,14 +79,16 @@ def attention_workspace(device) -> torch.Tensor:
 
 
 def ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_scale=None, kv_per_head=True,
-                     causal=False, workspace=None):
-    """flash_attn_varlen_func's arithmetic (non-causal) on the ragged layout;
-    with a workspace (attention_workspace), launches of a few sequences with
-    per-head keys split their keys over every compute unit."""
+                     causal=False, workspace=None, max_seqlen_k=0):
+    """flash_attn_varlen_func's arithmetic (non-causal) on the ragged layout.
+    Launches of a few query tiles split their keys over the compute units,
+    in a workspace of the allocator's or the one given (attention_workspace);
+    max_seqlen_k, an upper bound of a sequence's keys, spares launches of
+    short sequences the attempt."""
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
     return ops().ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), float(softmax_scale),
-                                  bool(kv_per_head), bool(causal), workspace)
+                                  bool(kv_per_head), bool(causal), workspace, int(max_seqlen_k or 0))
 
 
 def scatter_copy(src_ptrs, lengths, offsets, dst, col_dim: int) -> None:

@@ -136,3 +136,35 @@ def test_split_through_the_torch_op_on_strided_views():
                                 workspace=_ws())
     torch.cuda.synchronize()
     _check(to_np(out), q, k, v, cu_q, cu_k, H)
+
+
+@pytest.mark.parametrize("Lq,Lk,H,kv_per_head", [
+    # two rounds of items: 108 tiles, above 3/8 of the compute units
+    ([1300, 1300], [[3000 + 251 * h for h in range(9)]] * 2, 9, True),
+    # more than 64 sequences, several per lane of the plan, some without rows or keys
+    ([10, 0, 33] * 24, [[(s * 613 + h * 97) % 2600 for h in range(3)] for s in range(72)], 3, True),
+    # the edges of a chunk: one key more and fewer than the shortest two, and a
+    # single row over a long sequence
+    ([1], [[1023, 1024, 1025, 1151, 20000]], 5, True),
+    # key sequences shared by the heads
+    ([257, 5], [[5000], [1300]], 4, False),
+])
+def test_split_by_the_op_vs_float64(Lq, Lk, H, kv_per_head):
+    """The op without a workspace, which splits by its own rule: against
+    float64, and twice with the same bits."""
+    rng = np.random.default_rng(61)
+    B = len(Lq)
+    cu_q = np.concatenate([[0], np.cumsum(Lq)]).astype(np.int32)
+    cu_k = np.concatenate([[0], np.cumsum(np.asarray(Lk).reshape(-1))]).astype(np.int32)
+    shape = (int(cu_k[-1]), D) if kv_per_head else (int(cu_k[-1]), H, D)
+    q, k, v = (O.f32_to_bf16((rng.standard_normal(s) * 0.5).astype(np.float32))
+               for s in ((int(cu_q[-1]), H, D), shape, shape))
+    print(f"attention split by the op: {B} x {H} sequences, up to {np.max(Lq)} x {np.max(Lk)}", flush=True)
+    run = lambda: to_np(_ops.ragged_attention(to_dev(q), to_dev(k), to_dev(v), to_dev(cu_q), to_dev(cu_k),
+                                              int(np.max(Lq)), kv_per_head=kv_per_head))
+    got = run()
+    assert np.array_equal(got, run())
+    got = O.bf16_to_f32(got).astype(np.float64)
+    want = O.ragged_attention_ref(O.bf16_to_f32(q), O.bf16_to_f32(k), O.bf16_to_f32(v), cu_q, cu_k, H, kv_per_head)
+    err = np.abs(got - want)
+    assert err.max() < 2e-2 and err.mean() < 2e-3, (err.max(), err.mean())
