@@ -253,6 +253,20 @@ int pkv_plan_pack(const pkv_geometry *geo, const pkv_pools *pools,
                   const pkv_remap *remap, const pkv_rope_tables *rope,
                   const pkv_plan_out *plan_ws, pkv_stream_t stream);
 
+/* pkv_plan_pack with a device buffer of pkv_plan_list_size(geo, num_chunks)
+ * bytes (16-byte aligned, no initialisation), in which the plan lists the
+ * distinct segments of its query chunks: a segment that several chunks hold
+ * is then read once and written to each of their places.  Same outputs.  A
+ * NULL or smaller buffer, or a size of 0 (more chunks or heads than the plan
+ * can list), packs every chunk's segments by themselves. */
+int64_t pkv_plan_list_size(const pkv_geometry *geo, int32_t num_chunks);
+int pkv_plan_pack_list(const pkv_geometry *geo, const pkv_pools *pools,
+                       const uint8_t *states_layer, int32_t layer,
+                       const int64_t *current_t_list, int32_t num_chunks,
+                       const pkv_remap *remap, const pkv_rope_tables *rope,
+                       const pkv_plan_out *plan_ws, void *list, int64_t list_bytes,
+                       pkv_stream_t stream);
+
 /* scatter_copy: segment i copies lengths[i] rows of row_bytes bytes from
  * the device address src_ptrs[i] to dst rows offsets[i].. (all int64 device
  * arrays).  Segments whose rows fall outside [0, dst_rows) are skipped. */

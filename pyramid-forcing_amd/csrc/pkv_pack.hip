@@ -6,10 +6,10 @@
 // never leaves the GPU (the reference builds it on the host after three
 // blocking device-to-host copies, mega_plan.cc:557-568).
 //
-// The pack kernel is a persistent gather: each work item is (segment,
-// 64-token tile); 16 lanes move one 256-byte K row with 16-byte loads, the
-// same lanes rotate their 4 complex pairs in registers, V and positions are
-// copied alongside.
+// The pack kernel is a gather: each work item is (segment, 32-token tile); 16
+// lanes move one 256-byte K row with 16-byte loads, the same lanes rotate
+// their 4 complex pairs in registers, V and positions are copied alongside.
+// A segment that several query chunks of a call hold is read once.
 
 #include "pkv_common.h"
 
@@ -193,15 +193,37 @@ __device__ int32_t emit_pair(const PlanParams &p, const HeadState &s, const int6
 //    re-evaluates each pair's segments and writes them.
 constexpr int kPlanStageHeads = 48;  // heads whose records are staged in LDS
 constexpr int kPlanRegRounds = 4;    // pairs per wave held in registers by the one-pass form
+constexpr int kPlanListSegs = 2048;  // segments (all pairs) the one-pass form can list for the pack
+
+// One unit of the pack's work: a pool segment and the query chunks (up to
+// kPackShare) that hold it at the same place of their lists, each with its
+// first flat token and the remapped time (-1: the tokens' own).
+constexpr int kPackShare = 4;
+struct PackEntry {
+  int32_t kind, sg, len, n_to;
+  int32_t dst[kPackShare], tr[kPackShare];
+};
+static_assert(sizeof(PackEntry) == 48, "12 words, read by scalar loads");
+// a list: the entry count in the first 64 bytes, then the entries
+constexpr int64_t kPackListHead = 64;
+
+// int64 remapped time -> 32 bits as the pack's table lookup reads it (a cast,
+// then clamped to the table), negative = none
+__device__ inline int32_t remap32(int64_t tr) { return tr < 0 ? -1 : max(0, static_cast<int32_t>(tr)); }
 
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const HeadState *states,
                                                             const int64_t *vc, const int32_t *mtc,
-                                                            pkv_plan_out o, int32_t *total_out) {
+                                                            pkv_plan_out o, int32_t *total_out, char *list) {
   __shared__ int32_t len[kMaxPlanPairs];
   __shared__ int32_t part[1];
   __shared__ __attribute__((aligned(16))) HeadState s_states[kPlanStageHeads];
   __shared__ int64_t s_vc[kPlanStageHeads * 3];
   __shared__ int32_t s_mtc[kPlanStageHeads * kMaxMergeBlocks];
+  // the segments as (kind, slot, length, first flat token) and remapped time,
+  // for the pack's list
+  __shared__ int4 s_seg[kPlanListSegs];
+  __shared__ int32_t s_tr[kPlanListSegs];
+  __shared__ int32_t s_waves[kPlanThreads / 64];
   const int tid = threadIdx.x;
   const int pairs = p.C * p.H;
   const bool staged = p.H <= kPlanStageHeads && p.MMB <= kMaxMergeBlocks;
@@ -280,6 +302,68 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
       if (emit[r]) put_seg(o, i0 + pos[r], cd[r], base + excl[r]);
       if (lane >= nv[r] && lane < p.S) put_inactive(o, i0 + lane);
       if (lane == 0) o.cu_seqlens_k[q + 1] = end;
+      if (list) {
+        if (emit[r]) {
+          s_seg[i0 + pos[r]] = make_int4(cd[r].kind, cd[r].sg, cd[r].len, base + excl[r]);
+          s_tr[i0 + pos[r]] = remap32(cd[r].tremap);
+        }
+        if (lane >= nv[r] && lane < p.S) s_seg[i0 + lane] = make_int4(PKV_SEG_INACTIVE, 0, 0, 0);
+      }
+    }
+    if (!list) return;
+    // the pack's list: a thread per place of kPackShare chunks' lists finds
+    // the distinct segments there (at most kPackShare); a block-wide scan of
+    // the counts numbers them
+    __syncthreads();
+    const int per_chunk = p.H * p.S, groups = (p.C + kPackShare - 1) / kPackShare;
+    const int c0 = tid / per_chunk * kPackShare, place = tid % per_chunk;
+    const bool mine = tid < groups * per_chunk;
+    int4 sv[kPackShare];
+    int first_of[kPackShare], n_ent = 0;  // chunk whose entry chunk u joins (-1: inactive)
+#pragma unroll
+    for (int u = 0; u < kPackShare; ++u) {
+      sv[u] = make_int4(PKV_SEG_INACTIVE, 0, 0, 0);
+      if (mine && c0 + u < p.C) sv[u] = s_seg[(c0 + u) * per_chunk + place];
+      first_of[u] = sv[u].x >= 0 ? u : -1;
+#pragma unroll
+      for (int w = u - 1; w >= 0; --w)
+        if (sv[u].x >= 0 && sv[w].x == sv[u].x && sv[w].y == sv[u].y && sv[w].z == sv[u].z) first_of[u] = w;
+      n_ent += first_of[u] == u;
+    }
+    const int incl_n = wave_incl_sum(n_ent);
+    if (lane == 63) s_waves[wave] = incl_n;
+    __syncthreads();
+    int at = incl_n - n_ent, all = 0;
+    for (int w = 0; w < n_waves; ++w) {
+      if (w < wave) at += s_waves[w];
+      all += s_waves[w];
+    }
+    if (tid == 0) *reinterpret_cast<int32_t *>(list) = all;
+    PackEntry *ent = reinterpret_cast<PackEntry *>(list + kPackListHead) + at;
+#pragma unroll
+    for (int u = 0; u < kPackShare; ++u) {
+      if (first_of[u] != u) continue;
+      PackEntry e;
+      e.kind = sv[u].x;
+      e.sg = sv[u].y;
+      e.len = sv[u].z;
+      e.n_to = 0;
+      int4 dst = make_int4(0, 0, 0, 0), tr = make_int4(-1, -1, -1, -1);
+#pragma unroll
+      for (int w = u; w < kPackShare; ++w) {
+        if (first_of[w] != u) continue;
+        const int t = s_tr[(c0 + w) * per_chunk + place];
+        if (e.n_to == 0) { dst.x = sv[w].w; tr.x = t; }
+        else if (e.n_to == 1) { dst.y = sv[w].w; tr.y = t; }
+        else if (e.n_to == 2) { dst.z = sv[w].w; tr.z = t; }
+        else { dst.w = sv[w].w; tr.w = t; }
+        ++e.n_to;
+      }
+      int4 *out = reinterpret_cast<int4 *>(ent);
+      out[0] = make_int4(e.kind, e.sg, e.len, e.n_to);
+      out[1] = dst;
+      out[2] = tr;
+      ++ent;
     }
     return;
   }
@@ -396,16 +480,20 @@ __device__ inline uint32_t cvt_bf16x2(float lo, float hi) {
   return u;
 }
 
-// rope_chunk with the table entries of the chunk's 4 pairs resolved
-// (tabs) and the clamped rows of the token's (t, y, x) given
-__device__ inline uint4 rope_chunk_rows(uint4 raw, const PairTab (&tabs)[4], const int (&rows)[3]) {
-  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-  float2 f[4];
+// Table entries (cos, sin) of the 4 complex pairs of a chunk for a token's
+// clamped rows.
+__device__ inline void rope_entries(float2 (&f)[4], int chunk, const Rope &r, int row_t, int row_y, int row_x) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int row = tabs[e].sel == 0 ? rows[0] : (tabs[e].sel == 1 ? rows[1] : rows[2]);
-    f[e] = *reinterpret_cast<const float2 *>(tabs[e].p + row * tabs[e].stride);
+    const PairTab tab = pair_tab(chunk, e, r);
+    const int row = tab.sel == 0 ? row_t : (tab.sel == 1 ? row_y : row_x);
+    f[e] = *reinterpret_cast<const float2 *>(tab.p + row * tab.stride);
   }
+}
+
+// rope_chunk with the chunk's table entries given
+__device__ inline uint4 rope_rotate(uint4 raw, const float2 (&f)[4]) {
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
   uint32_t o[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -432,9 +520,10 @@ __device__ inline void st16_nt(uint16_t *p, uint4 v) {
 // ---------------------------------------------------------------------------
 // pack
 // ---------------------------------------------------------------------------
-constexpr int kPackTok = 64;
+constexpr int kPackTok = 32;
 constexpr int kPackThreads = 256;
-constexpr int kPackPer = 4;  // 16-byte chunks per thread per round
+constexpr int kPackListGrid = 8192;
+constexpr int kPackPer = 2;  // 16-byte chunks per thread per round
 
 struct PackArgs {
   const uint16_t *k[4], *v[4];
@@ -444,96 +533,139 @@ struct PackArgs {
   int64_t *pos_out;
   const int32_t *kind, *sg, *len, *dst;
   const int64_t *tremap;
+  const char *list;  // the plan's PackEntry list (null: one entry per segment of the arrays above)
   Rope rope;
   int fuse;  // rope tables + tremap present
   int n_seg, tiles_per_seg, FSEQ, MTPA, D;
   int64_t capacity;
 };
 
+// One workgroup per (entry, 32-token tile).  Bound by memory, by the stores
+// above all: each query chunk's flat copy is written, but most segments of a
+// call's chunks are the same frames (a head's sink and recent frames and its
+// Anchor and Veil segments in every chunk; a Wave head's middle frames differ
+// by phase), so the plan lists each once with the places it goes to (K rotated
+// anew where the remapped time differs).  One layer of 12 heads and 3 chunks
+// (117 MB read, 274 MB written): 74 us = 5.3 TB/s, against 99 us with every
+// chunk's segments read by themselves; a copy of one source to three places
+// runs at 6.6 TB/s.  Without the rotation it takes as long.  Tiles of 64
+// tokens hold 187 registers (88 us), of 16 tokens 71 (81 us).
+// kD: the head_dim, 0 for one known only at run time.
+template <int kD>
 __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
   // clamped RoPE table rows (t, y, x) of the tile's tokens
-  __shared__ int s_rows[kPackTok][3];
-  const int items = a.n_seg * a.tiles_per_seg;
-  const int cpt = a.D / 8;
-  for (int it = blockIdx.x; it < items; it += gridDim.x) {
-    const int seg = it / a.tiles_per_seg, tile = it % a.tiles_per_seg;
-    // every descriptor field is read before the first test, by scalar loads
-    // in one round trip (seg < n_seg, so all of them are in bounds; the
-    // descriptors do not change while the kernel runs)
-    const int kind = ld_uniform(a.kind + seg);
-    const int len = ld_uniform(a.len + seg);
-    const int64_t sg = ld_uniform(a.sg + seg);
-    const int64_t dst = ld_uniform(a.dst + seg);
-    const int64_t tr_seg = a.fuse ? ld_uniform(a.tremap + seg) : -1;
+  __shared__ int s_rows[kPackTok * 3];
+  const int D = kD ? kD : a.D, cpt = D / 8;
+  const int n_ent = a.list ? ld_uniform(reinterpret_cast<const int32_t *>(a.list)) : a.n_seg;
+  const PackEntry *entries = reinterpret_cast<const PackEntry *>(a.list + kPackListHead);
+  for (int64_t it = blockIdx.x;; it += gridDim.x) {
+    const int ei = static_cast<int>(it / a.tiles_per_seg), tile = static_cast<int>(it % a.tiles_per_seg);
+    if (ei >= a.n_seg) return;
+    // every field is read before the first test, by scalar loads in one round
+    // trip (ei < n_seg, so all of them are in bounds, with whatever value past
+    // the list's end; they do not change while the kernel runs)
+    PackEntry en;
+    if (a.list) {
+      const int32_t *w = reinterpret_cast<const int32_t *>(entries + ei);
+#pragma unroll
+      for (int i = 0; i < 12; ++i) reinterpret_cast<int32_t *>(&en)[i] = ld_uniform(w + i);
+    } else {
+      en.kind = ld_uniform(a.kind + ei);
+      en.sg = ld_uniform(a.sg + ei);
+      en.len = ld_uniform(a.len + ei);
+      en.dst[0] = ld_uniform(a.dst + ei);
+      en.tr[0] = a.fuse ? remap32(ld_uniform(a.tremap + ei)) : -1;
+      en.n_to = 1;
+    }
+    if (ei >= n_ent) return;
+    const int kind = en.kind, len = en.len;
     if (kind < 0 || kind > 3) continue;
     if (len <= 0 || tile * kPackTok >= len) continue;
     const int stride = (kind == PKV_SEG_MERGE) ? a.MTPA : a.FSEQ;
+    const int64_t sg = en.sg;
     // a segment starts at its slot and may run on through the following
     // slots of the pool (the legacy plan's whole-pool segments), never past
     // the pool's end
-    if (sg < 0 || sg * stride + len > a.slots[kind] * stride || dst < 0 || dst + len > a.capacity || !a.k[kind])
-      continue;
-    const uint16_t *sk = a.k[kind] + sg * stride * a.D;
-    const uint16_t *sv = a.v[kind] + sg * stride * a.D;
+    if (sg < 0 || sg * stride + len > a.slots[kind] * stride || !a.k[kind]) continue;
+    bool to[kPackShare];
+#pragma unroll
+    for (int w = 0; w < kPackShare; ++w)
+      to[w] = w < en.n_to && en.dst[w] >= 0 && static_cast<int64_t>(en.dst[w]) + len <= a.capacity;
+    const uint16_t *sk = a.k[kind] + sg * stride * D;
+    const uint16_t *sv = a.v[kind] + sg * stride * D;
     const int64_t *sp = a.pos[kind] ? a.pos[kind] + sg * stride * 3 : nullptr;
-    uint16_t *ok = a.k_out + dst * a.D;
-    uint16_t *ov = a.v_out + dst * a.D;
     const bool rope = a.fuse && sp;  // uniform over the workgroup
-    const int64_t tr = rope ? tr_seg : -1;
     // segments up to tiles_per_seg tiles long (every frame or merge anchor)
     // take one pass; longer ones are walked tiles_per_seg tiles at a time
-    for (int tok0 = tile * kPackTok; tok0 < len; tok0 += a.tiles_per_seg * kPackTok) {
-      const int ntok = min(kPackTok, len - tok0);
+    for (int64_t tok0 = tile * kPackTok; tok0 < len; tok0 += static_cast<int64_t>(a.tiles_per_seg) * kPackTok) {
+      const int ntok = static_cast<int>(min<int64_t>(kPackTok, len - tok0));
       const int n_items = ntok * cpt;
-      if (rope) {
-        // the tile's table rows, one thread per token (the positions are
-        // read once per token instead of once per chunk)
-        __syncthreads();  // the previous tile's readers are done
-        for (int i = threadIdx.x; i < ntok; i += blockDim.x) {
-          const int64_t *pp = sp + static_cast<int64_t>(tok0 + i) * 3;
-          s_rows[i][0] = clamp_row(tr >= 0 ? tr : pp[0], a.rope.ft_rows);
-          s_rows[i][1] = clamp_row(pp[1], a.rope.fy_rows);
-          s_rows[i][2] = clamp_row(pp[2], a.rope.fx_rows);
-        }
-        __syncthreads();
-      }
-      // all of this thread's chunks of a round are loaded before any store
-      // (up to kPackPer 16-byte K and V reads in flight per thread; one round
-      // covers the tile for head_dim <= 128)
+      // the tile's positions: one word per thread, written on to every copy
+      // and, clamped to the tables, kept for the rotation
+      static_assert(kPackTok * 3 <= kPackThreads, "one position word per thread");
+      int64_t pw = 0;
+      const bool has_pos = sp && static_cast<int>(threadIdx.x) < ntok * 3;
+      if (has_pos) pw = sp[tok0 * 3 + threadIdx.x];
       for (int base = 0; base < n_items; base += kPackPer * kPackThreads) {
+        // all of this thread's chunks of a round are loaded before any store
+        // (up to kPackPer 16-byte K and V reads in flight per thread; one round
+        // covers the tile for head_dim <= 128)
         uint4 kk[kPackPer], vv[kPackPer];
 #pragma unroll
         for (int u = 0; u < kPackPer; ++u) {
           const int i = base + threadIdx.x + u * kPackThreads;
           if (i < n_items) {
-            const int64_t e = static_cast<int64_t>(tok0 + i / cpt) * a.D + (i % cpt) * 8;
-            kk[u] = ld16(sk + e);
-            vv[u] = ld16(sv + e);
+            const int e = i / cpt * D + i % cpt * 8;
+            kk[u] = ld16(sk + tok0 * D + e);
+            vv[u] = ld16(sv + tok0 * D + e);
+          }
+        }
+        if (base == 0) {
+          __syncthreads();  // the previous tile's readers are done
+          if (has_pos) {
+            const int axis = threadIdx.x % 3;
+            s_rows[threadIdx.x] = clamp_row(pw, axis == 0 ? a.rope.ft_rows : (axis == 1 ? a.rope.fy_rows : a.rope.fx_rows));
+          }
+          __syncthreads();
+          if (has_pos && a.pos_out) {
+#pragma unroll
+            for (int w = 0; w < kPackShare; ++w)
+              if (to[w]) a.pos_out[(en.dst[w] + tok0) * 3 + threadIdx.x] = pw;
           }
         }
 #pragma unroll
-        for (int u = 0; u < kPackPer; ++u) {
-          const int i = base + threadIdx.x + u * kPackThreads;
-          if (i >= n_items) continue;
-          const int tl = i / cpt, ch = i % cpt;
-          const int64_t e = static_cast<int64_t>(tok0 + tl) * a.D + ch * 8;
-          uint4 k4 = kk[u];
-          if (rope) {
-            const int rows[3] = {s_rows[tl][0], s_rows[tl][1], s_rows[tl][2]};
-            PairTab t4[4];
+        for (int w = 0; w < kPackShare; ++w) {
+          if (!to[w]) continue;
+          uint16_t *ov = a.v_out + (en.dst[w] + tok0) * D;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) t4[q] = pair_tab(ch, q, a.rope);
-            k4 = rope_chunk_rows(k4, t4, rows);
+          for (int u = 0; u < kPackPer; ++u) {
+            const int i = base + threadIdx.x + u * kPackThreads;
+            if (i < n_items) st16_nt(ov + (i / cpt * D + i % cpt * 8), vv[u]);
           }
-          st16_nt(ok + e, k4);
-          st16_nt(ov + e, vv[u]);
         }
-      }
-      if (a.pos_out && sp) {
-        int64_t *op = a.pos_out + dst * 3;
-        for (int i = threadIdx.x; i < ntok * 3; i += blockDim.x) {
-          const int64_t e = static_cast<int64_t>(tok0) * 3 + i;
-          op[e] = sp[e];
+        // K: the table entries of all of the thread's chunks are fetched
+        // together, once for copies at the same time
+        float2 f[kPackPer][4];
+        int at = -2;
+#pragma unroll
+        for (int w = 0; w < kPackShare; ++w) {
+          if (!to[w]) continue;
+          uint16_t *ok = a.k_out + (en.dst[w] + tok0) * D;
+          if (rope && en.tr[w] != at) {
+            at = en.tr[w];
+#pragma unroll
+            for (int u = 0; u < kPackPer; ++u) {
+              const int i = min(base + static_cast<int>(threadIdx.x) + u * kPackThreads, n_items - 1);
+              const int tl = i / cpt, ch = i % cpt;
+              const int row_t = at >= 0 ? min(at, a.rope.ft_rows - 1) : s_rows[tl * 3];
+              rope_entries(f[u], ch, a.rope, row_t, s_rows[tl * 3 + 1], s_rows[tl * 3 + 2]);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < kPackPer; ++u) {
+            const int i = base + threadIdx.x + u * kPackThreads;
+            if (i < n_items) st16_nt(ok + (i / cpt * D + i % cpt * 8), rope ? rope_rotate(kk[u], f[u]) : kk[u]);
+          }
         }
       }
     }  // tiles of a long segment
@@ -577,7 +709,7 @@ using namespace pkv;
 // layer slot_layer of the [L, H, slots] pools).
 static int plan_launch(const pkv_geometry *geo, const uint8_t *states_layer, const int64_t *valid_count_layer,
                        const int32_t *merge_token_count_layer, const int64_t *current_t_list, int32_t num_chunks,
-                       const pkv_remap *remap, const pkv_plan_out *out, int32_t *total_tokens_out, int slot_layer,
+                       const pkv_remap *remap, const pkv_plan_out *out, int32_t *total_tokens_out, int slot_layer, char *list,
                        hipStream_t st) {
   if (!geo || !states_layer || !valid_count_layer || !merge_token_count_layer || !current_t_list || !remap ||
       !out)
@@ -610,7 +742,7 @@ static int plan_launch(const pkv_geometry *geo, const uint8_t *states_layer, con
   }
   hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, p,
                      reinterpret_cast<const HeadState *>(states_layer), valid_count_layer,
-                     merge_token_count_layer, *out, total_tokens_out);
+                     merge_token_count_layer, *out, total_tokens_out, list);
   int rc = check_launch("plan_kernel");
   if (rc) return rc;
   // Static bound on the packed tokens: every (chunk, head) emits at most S
@@ -645,27 +777,31 @@ static int plan_launch(const pkv_geometry *geo, const uint8_t *states_layer, con
   return PKV_OK;
 }
 
-extern "C" {
-
-int pkv_plan_multi(const pkv_geometry *geo, const uint8_t *states_layer, const int64_t *valid_count_layer,
-                   const int32_t *merge_token_count_layer, const int64_t *current_t_list, int32_t num_chunks,
-                   const pkv_remap *remap, const pkv_plan_out *out, int32_t *total_tokens_out,
-                   pkv_stream_t stream) {
-  return plan_launch(geo, states_layer, valid_count_layer, merge_token_count_layer, current_t_list, num_chunks,
-                     remap, out, total_tokens_out, -1, as_stream(stream));
+// Whether the plan of num_chunks chunks can list the pack's work: its
+// one-pass form (plan_kernel), with every segment in LDS and a thread per
+// place of kPackShare chunks' lists.  At 12 heads and 37 segments that is up
+// to 4 chunks.
+static bool plan_lists(const pkv_geometry *g, int64_t num_chunks) {
+  const int64_t S = g->max_sink + g->max_middle + g->max_recent + g->max_merge_blocks, pairs = num_chunks * g->num_heads;
+  const int64_t cand = g->max_sink + g->max_recent + kMaxTKeyed + kMaxMergeBlocks;
+  return g->num_heads <= kPlanStageHeads && g->max_merge_blocks <= kMaxMergeBlocks && cand <= 64 && S <= 64 &&
+         pairs <= 64 && pairs <= kPlanThreads / 64 * kPlanRegRounds && pairs * S <= kPlanListSegs &&
+         (num_chunks + kPackShare - 1) / kPackShare * g->num_heads * S <= kPlanThreads;
 }
 
-int pkv_pack(const pkv_geometry *geo, const pkv_pools *pools, const int32_t *src_kind,
-             const int32_t *src_slot_global, const int32_t *seg_lengths, const int32_t *dst_token_offsets,
-             int32_t n_segments, const int64_t *anchor_t_remap, const pkv_rope_tables *rope,
-             pkv_stream_t stream) {
+// Pack of a segment list, or of the plan's entry list of those segments
+// (list non-null).
+static int pack_launch(const pkv_geometry *geo, const pkv_pools *pools, const int32_t *src_kind,
+                       const int32_t *src_slot_global, const int32_t *seg_lengths, const int32_t *dst_token_offsets,
+                       int32_t n_segments, const char *list, const int64_t *anchor_t_remap,
+                       const pkv_rope_tables *rope, hipStream_t stream) {
   if (!geo || !pools) return fail(PKV_ERR_INVALID, "pyramidkv_pack: NULL geometry/pools");
   if (n_segments == 0) return PKV_OK;
   if (n_segments < 0 || !src_kind || !src_slot_global || !seg_lengths || !dst_token_offsets)
     return fail(PKV_ERR_INVALID, "pyramidkv_pack: bad descriptors");
   if (geo->head_dim % 8) return fail(PKV_ERR_INVALID, "pyramidkv_pack: head_dim must be a multiple of 8");
   if (!pools->k_flat_out || !pools->v_flat_out) return fail(PKV_ERR_INVALID, "pyramidkv_pack: no flat outputs");
-  PackArgs a;
+  PackArgs a{};
   const int64_t lh = static_cast<int64_t>(geo->num_layers) * geo->num_heads;
   a.k[0] = pools->sink_k; a.v[0] = pools->sink_v; a.pos[0] = pools->sink_pos; a.slots[0] = lh * geo->max_sink;
   a.k[1] = pools->middle_k; a.v[1] = pools->middle_v; a.pos[1] = pools->middle_pos; a.slots[1] = lh * geo->max_middle;
@@ -686,6 +822,7 @@ int pkv_pack(const pkv_geometry *geo, const pkv_pools *pools, const int32_t *src
     a.fuse = 1;
   }
   a.n_seg = n_segments;
+  a.list = list;
   a.FSEQ = geo->frame_seqlen;
   a.MTPA = geo->max_merge_tokens;
   a.D = geo->head_dim;
@@ -694,27 +831,65 @@ int pkv_pack(const pkv_geometry *geo, const pkv_pools *pools, const int32_t *src
   a.tiles_per_seg = (seg_max + kPackTok - 1) / kPackTok;
   const int64_t items = static_cast<int64_t>(n_segments) * a.tiles_per_seg;
   if (items > 0x7fffffff) return fail(PKV_ERR_UNSUPPORTED, "pyramidkv_pack: too many segments");
-  const int grid = static_cast<int>(items);  // one workgroup per (segment, tile); inactive ones exit at once
-  hipLaunchKernelGGL(pack_kernel, dim3(grid), dim3(kPackThreads), 0, as_stream(stream), a);
+  // one workgroup per (segment, tile), inactive ones exit at once; of a list
+  // most segments are inactive or another's copy, so at most kPackListGrid
+  // workgroups walk it (one layer of the production shape has about 4,500 items)
+  const int grid = static_cast<int>(list && items > kPackListGrid ? kPackListGrid : items);
+  if (a.D == 128) hipLaunchKernelGGL(pack_kernel<128>, dim3(grid), dim3(kPackThreads), 0, stream, a);
+  else hipLaunchKernelGGL(pack_kernel<0>, dim3(grid), dim3(kPackThreads), 0, stream, a);
   return check_launch("pack_kernel");
+}
+
+extern "C" {
+
+int pkv_plan_multi(const pkv_geometry *geo, const uint8_t *states_layer, const int64_t *valid_count_layer,
+                   const int32_t *merge_token_count_layer, const int64_t *current_t_list, int32_t num_chunks,
+                   const pkv_remap *remap, const pkv_plan_out *out, int32_t *total_tokens_out,
+                   pkv_stream_t stream) {
+  return plan_launch(geo, states_layer, valid_count_layer, merge_token_count_layer, current_t_list, num_chunks,
+                     remap, out, total_tokens_out, -1, nullptr, as_stream(stream));
+}
+
+int pkv_pack(const pkv_geometry *geo, const pkv_pools *pools, const int32_t *src_kind,
+             const int32_t *src_slot_global, const int32_t *seg_lengths, const int32_t *dst_token_offsets,
+             int32_t n_segments, const int64_t *anchor_t_remap, const pkv_rope_tables *rope,
+             pkv_stream_t stream) {
+  return pack_launch(geo, pools, src_kind, src_slot_global, seg_lengths, dst_token_offsets, n_segments, nullptr,
+                     anchor_t_remap, rope, as_stream(stream));
 }
 
 int pkv_plan_pack(const pkv_geometry *geo, const pkv_pools *pools, const uint8_t *states_layer, int32_t layer,
                   const int64_t *current_t_list, int32_t num_chunks, const pkv_remap *remap,
                   const pkv_rope_tables *rope, const pkv_plan_out *plan_ws, pkv_stream_t stream) {
+  return pkv_plan_pack_list(geo, pools, states_layer, layer, current_t_list, num_chunks, remap, rope, plan_ws, nullptr,
+                            0, stream);
+}
+
+int64_t pkv_plan_list_size(const pkv_geometry *geo, int32_t num_chunks) {
+  if (!geo || num_chunks <= 0 || !plan_lists(geo, num_chunks)) return 0;
+  const int64_t S = geo->max_sink + geo->max_middle + geo->max_recent + geo->max_merge_blocks;
+  return kPackListHead + num_chunks * geo->num_heads * S * static_cast<int64_t>(sizeof(PackEntry));
+}
+
+int pkv_plan_pack_list(const pkv_geometry *geo, const pkv_pools *pools, const uint8_t *states_layer, int32_t layer,
+                       const int64_t *current_t_list, int32_t num_chunks, const pkv_remap *remap,
+                       const pkv_rope_tables *rope, const pkv_plan_out *plan_ws, void *list, int64_t list_bytes,
+                       pkv_stream_t stream) {
   if (!geo || !pools || !plan_ws || !pools->valid_count || !pools->merge_token_count)
     return fail(PKV_ERR_INVALID, "plan_pack: NULL argument");
   if (layer < 0 || layer >= geo->num_layers) return fail(PKV_ERR_INVALID, "plan_pack: layer out of range");
   const int H = geo->num_heads;
   const int S = geo->max_sink + geo->max_middle + geo->max_recent + geo->max_merge_blocks;
   hipStream_t st = as_stream(stream);
+  const int64_t need = pkv_plan_list_size(geo, num_chunks);
+  char *lst = list && need > 0 && list_bytes >= need && reinterpret_cast<uintptr_t>(list) % 16 == 0 ? static_cast<char *>(list) : nullptr;
   int rc = plan_launch(geo, states_layer, pools->valid_count + static_cast<int64_t>(layer) * H * 3,
                        pools->merge_token_count + static_cast<int64_t>(layer) * H * geo->max_merge_blocks,
-                       current_t_list, num_chunks, remap, plan_ws, nullptr, layer, st);
+                       current_t_list, num_chunks, remap, plan_ws, nullptr, layer, lst, st);
   if (rc) return rc;
-  return pkv_pack(geo, pools, plan_ws->src_kind, plan_ws->src_slot_global, plan_ws->seg_lengths,
-                  plan_ws->dst_token_offsets, num_chunks * H * S, rope ? plan_ws->anchor_t_remap : nullptr, rope,
-                  stream);
+  return pack_launch(geo, pools, plan_ws->src_kind, plan_ws->src_slot_global, plan_ws->seg_lengths,
+                     plan_ws->dst_token_offsets, num_chunks * H * S, lst,
+                     rope ? plan_ws->anchor_t_remap : nullptr, rope, st);
 }
 
 int pkv_rope_apply(const uint16_t *k, const int64_t *pos, int64_t n_tokens, int32_t head_dim,

@@ -14,6 +14,7 @@
 #include <torch/custom_class.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <tuple>
@@ -304,6 +305,18 @@ class PyramidKVCacheManager : public torch::CustomClassHolder {
                         pw_tremap_.data_ptr<int64_t>()};
   }
 
+  // The plan's list for the pack of up to max_attend_chunks chunks (empty when
+  // the plan lists none).
+  Tensor plan_list() {
+    if (!pw_list_.defined()) {
+      const pkv_geometry g = geometry();
+      int64_t n = 0;
+      for (int64_t c = 1; c <= mac_; ++c) n = std::max(n, pkv_plan_list_size(&g, static_cast<int32_t>(c)));
+      pw_list_ = at::empty({n}, at::TensorOptions().dtype(at::kByte).device(valid_count_.device()));
+    }
+    return pw_list_;
+  }
+
   std::vector<Tensor> update_descriptors(int64_t frames) {
     Tensor ws = update_workspace(frames);
     const int64_t n = H_ * frames;
@@ -323,7 +336,7 @@ class PyramidKVCacheManager : public torch::CustomClassHolder {
   Tensor acc_k_, acc_v_, acc_pos_, acc_gid_, acc_tpg_, acc_ng_, acc_wsum_;
   Tensor ws_;
   int64_t ws_frames_ = -1;
-  Tensor pw_kind_, pw_sg_, pw_len_, pw_dst_, pw_traw_, pw_tremap_;
+  Tensor pw_kind_, pw_sg_, pw_len_, pw_dst_, pw_traw_, pw_tremap_, pw_list_;
 };
 
 using Mgr = c10::intrusive_ptr<PyramidKVCacheManager>;
@@ -1086,9 +1099,10 @@ static Tensor mega_attend_kv(Mgr mgr, Tensor states_layer, int64_t layer_idx, Te
   const pkv_geometry g = mgr->geometry();
   const pkv_pools p = mgr->pools();
   const pkv_plan_out ws = mgr->plan_workspace();
-  pkv_check(pkv_plan_pack(&g, &p, states_layer.data_ptr<uint8_t>(), static_cast<int32_t>(layer_idx),
-                          tl.data_ptr<int64_t>(), static_cast<int32_t>(C), &rm, rope, &ws,
-                          stream_for(states_layer)),
+  const Tensor list = mgr->plan_list();
+  pkv_check(pkv_plan_pack_list(&g, &p, states_layer.data_ptr<uint8_t>(), static_cast<int32_t>(layer_idx),
+                               tl.data_ptr<int64_t>(), static_cast<int32_t>(C), &rm, rope, &ws,
+                               ptr_or_null<void>(list), list.numel(), stream_for(states_layer)),
             "mega_attend_kv");
   return mgr->cu_seqlens_k().narrow(0, 0, C * mgr->num_heads() + 1);
 }
