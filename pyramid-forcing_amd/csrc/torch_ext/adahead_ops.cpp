@@ -10,6 +10,7 @@
 // the same namespace.
 
 #include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/custom_class.h>
 #include <torch/library.h>
@@ -1107,6 +1108,47 @@ static Tensor mega_attend_kv(Mgr mgr, Tensor states_layer, int64_t layer_idx, Te
   return mgr->cu_seqlens_k().narrow(0, 0, C * mgr->num_heads() + 1);
 }
 
+// ---------------------------------------------------------------------------
+// MegaCache's calls as methods of the manager.  Python's call of an op that
+// takes a script object walks all of its arguments first (13-20 us for these
+// ops, twice what the op itself takes); a method's does not.  They go through
+// the dispatcher like the ops' own calls, so that modes and subclasses see the
+// same ops.
+// ---------------------------------------------------------------------------
+static void update_layer(const Mgr &mgr, const Tensor &states, const Tensor &sink_caps, const Tensor &committed_vc,
+                         const Tensor &new_k, const Tensor &new_v, int64_t layer, int64_t t0, int64_t pass_kind,
+                         int64_t shift_pending, int64_t spatial_width, int64_t merge_heads) {
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("adahead::cache_update", "").typed<decltype(cache_update)>();
+  op.call(mgr, states.select(0, layer), sink_caps.select(0, layer), committed_vc.select(0, layer), new_k, new_v, layer,
+          t0, pass_kind, shift_pending, spatial_width, merge_heads);
+}
+
+static Tensor attend_kv_layer(const Mgr &mgr, const Tensor &states, int64_t layer, int64_t t0, int64_t num_chunks,
+                              int64_t sink_mode_code, int64_t sink_clamp_min, int64_t sink_clamp_max,
+                              int64_t decoupled_sink_lag, const Tensor &ft, const Tensor &fy, const Tensor &fx) {
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("adahead::mega_attend_kv", "").typed<decltype(mega_attend_kv)>();
+  const Tensor times = at::arange(t0, t0 + num_chunks, at::TensorOptions().dtype(at::kLong));
+  return op.call(mgr, states.select(0, layer), layer, times, sink_mode_code, sink_clamp_min, sink_clamp_max,
+                 decoupled_sink_lag, ft, fy, fx);
+}
+
+// attend_kv_layer, then the attention of q [num_chunks * frame_seqlen, H, D]
+// over the packed keys.
+static Tensor attend_layer(const Mgr &mgr, const Tensor &states, int64_t layer, int64_t t0, int64_t num_chunks,
+                           int64_t sink_mode_code, int64_t sink_clamp_min, int64_t sink_clamp_max,
+                           int64_t decoupled_sink_lag, const Tensor &ft, const Tensor &fy, const Tensor &fx,
+                           const Tensor &q, const Tensor &cu_seqlens_q, double softmax_scale, bool causal,
+                           const c10::optional<Tensor> &workspace, int64_t max_seqlen_k) {
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("adahead::ragged_attention", "").typed<decltype(ragged_attention)>();
+  const Tensor cu_k = attend_kv_layer(mgr, states, layer, t0, num_chunks, sink_mode_code, sink_clamp_min,
+                                      sink_clamp_max, decoupled_sink_lag, ft, fy, fx);
+  return op.call(q, mgr->k_flat_out(), mgr->v_flat_out(), cu_seqlens_q, cu_k, mgr->frame_seqlen(), softmax_scale, true,
+                 causal, workspace, max_seqlen_k);
+}
+
 }  // namespace adahead
 
 // ---------------------------------------------------------------------------
@@ -1215,7 +1257,15 @@ TORCH_LIBRARY(adahead, m) {
       .def("max_total", &M::max_total)
       .def("max_total_tokens", &M::max_total_tokens)
       .def("max_attend_chunks", &M::max_attend_chunks)
-      .def("max_pack_tokens", &M::max_pack_tokens);
+      .def("max_pack_tokens", &M::max_pack_tokens)
+      .def("update_layer",
+           [](const adahead::Mgr &m, const at::Tensor &st, const at::Tensor &caps, const at::Tensor &vc,
+              const at::Tensor &k, const at::Tensor &v, int64_t layer, int64_t t0, int64_t pass_kind, int64_t pending,
+              int64_t width, int64_t heads) {
+             adahead::update_layer(m, st, caps, vc, k, v, layer, t0, pass_kind, pending, width, heads);
+           })
+      .def("attend_kv_layer", &adahead::attend_kv_layer)
+      .def("attend_layer", &adahead::attend_layer);
 
   m.def("pyramidkv_pack(__torch__.torch.classes.adahead.PyramidKVCacheManager mgr, Tensor src_kind, "
         "Tensor src_slot_global, Tensor seg_lengths, Tensor dst_token_offsets, Tensor anchor_t_remap, "

@@ -113,7 +113,7 @@ class MegaCache:
         assert B == 1, "MegaCache.update: B>1 not yet supported"
         assert Hk == H and Dk == D
         assert L_in % FSEQ == 0, f"L_in ({L_in}) not multiple of FSEQ ({FSEQ})"
-        t0 = current_start // FSEQ
+        t0 = int(current_start // FSEQ)
         l = self.layer_idx
         if ctx.committed_vc is None:
             ctx.committed_vc = ctx.mgr.valid_count().clone()
@@ -135,9 +135,9 @@ class MegaCache:
         if nv.stride() != nk.stride():
             nv = nv.contiguous()
             nk = nk.contiguous()
-        _ops.ops().cache_update(ctx.mgr, ctx.states_bytes[l], ctx.sink_caps_per_head[l], ctx.committed_vc[l], nk, nv,
-                                l, t0, 1 if clean else 0, 1 if pending == block else 0, ctx.spatial_width,
-                                ctx.layer_merge_heads[l])
+        ctx.mgr.update_layer(ctx.states_bytes, ctx.sink_caps_per_head, ctx.committed_vc, nk, nv, l, t0,
+                             1 if clean else 0, 1 if pending == block else 0, ctx.spatial_width,
+                             ctx.layer_merge_heads[l])
         ctx.pending_block[l] = None if clean else block
 
     def _recent_fifo(self, restore: bool) -> None:
@@ -197,9 +197,10 @@ class MegaCache:
     def attend_kv(self, current_start: int, num_chunks: int, freqs=None) -> torch.Tensor:
         """Plan + layer offset + pack (+RoPE) in one op; returns cu_seqlens_k
         [C*H+1] (a view of the manager's buffer, valid until the next call)."""
+        return self.ctx.mgr.attend_kv_layer(*self._attend_args(current_start, num_chunks, freqs))
+
+    def _attend_args(self, current_start: int, num_chunks: int, freqs):
         ctx = self.ctx
-        FSEQ = ctx.frame_seqlen
-        t_list = torch.arange(current_start // FSEQ, current_start // FSEQ + num_chunks, dtype=torch.int64)
         eff = ctx.freqs if ctx.freqs is not None else freqs
         if eff is not None:
             parts = ctx.freq_parts_flat
@@ -208,10 +209,9 @@ class MegaCache:
                 parts = ctx.freq_parts_flat = flat_freq_parts(eff, ctx.states_bytes.device)
         else:
             parts = (_ops._empty(torch.float32, ctx.states_bytes.device),) * 3
-        return _ops.ops().mega_attend_kv(ctx.mgr, self.states_bytes_for_layer, self.layer_idx, t_list,
-                                         _mega_state_ops._SINK_MODE.get(ctx.sink_time_mapping_mode, 0),
-                                         int(ctx.sink_time_clamp_min), int(ctx.sink_time_clamp_max),
-                                         int(ctx.decoupled_sink_time_lag), *parts)
+        return (ctx.states_bytes, self.layer_idx, int(current_start // ctx.frame_seqlen), int(num_chunks),
+                _mega_state_ops._SINK_MODE.get(ctx.sink_time_mapping_mode, 0), int(ctx.sink_time_clamp_min),
+                int(ctx.sink_time_clamp_max), int(ctx.decoupled_sink_time_lag), *parts)
 
     def attend(self, q: torch.Tensor, current_start: int, *, freqs=None, softmax_scale=None, causal=False,
                max_seqlen_k=None) -> torch.Tensor:
@@ -222,17 +222,20 @@ class MegaCache:
         assert B == 1, "MegaCache.attend: B>1 not yet supported"
         assert L_q % FSEQ == 0, f"L_q ({L_q}) must be a multiple of FSEQ ({FSEQ})"
         C = L_q // FSEQ
-        if C <= int(ctx.mgr.max_attend_chunks()):
-            cu_k = self.attend_kv(current_start, C, freqs)
-        else:  # more chunks than the fused plan buffers hold: the reference op sequence (raises on overflow)
-            cu_k = self.pack(self.plan(current_start, C), freqs)
         cu_q = ctx.cu_q.get(L_q)
         if cu_q is None or cu_q.device != q.device:
             cu_q = ctx.cu_q[L_q] = torch.arange(0, L_q + 1, FSEQ, dtype=torch.int32, device=q.device)
         qb = q[0] if q.dtype == torch.bfloat16 else q[0].to(torch.bfloat16)
-        out = _ops.ragged_attention(qb, ctx.mgr.k_flat_out().view(-1, D), ctx.mgr.v_flat_out().view(-1, D), cu_q,
-                                    cu_k, FSEQ, softmax_scale, kv_per_head=True, causal=causal,
-                                    workspace=self._split_workspace(q.device), max_seqlen_k=ctx.layer_max_keys[self.layer_idx])
+        max_keys = ctx.layer_max_keys[self.layer_idx] if ctx.layer_max_keys else 0
+        if C <= int(ctx.mgr.max_attend_chunks()):
+            scale = float(softmax_scale) if softmax_scale is not None else D ** -0.5
+            out = ctx.mgr.attend_layer(*self._attend_args(current_start, C, freqs), qb, cu_q, scale, bool(causal),
+                                       self._split_workspace(q.device), max_keys)
+        else:  # more chunks than the fused plan buffers hold: the reference op sequence (raises on overflow)
+            cu_k = self.pack(self.plan(current_start, C), freqs)
+            out = _ops.ragged_attention(qb, ctx.mgr.k_flat_out().view(-1, D), ctx.mgr.v_flat_out().view(-1, D), cu_q,
+                                        cu_k, FSEQ, softmax_scale, kv_per_head=True, causal=causal,
+                                        workspace=self._split_workspace(q.device), max_seqlen_k=max_keys)
         return out.view(1, L_q, H, D).to(q.dtype)
 
 
