@@ -913,6 +913,22 @@ struct UpdShared {
   int32_t grid_ng, grid_cols, grid_w;
 };
 
+// The patch grid of a frame of FSEQ tokens in rows of W (the last row may be
+// short) in patches of p: its columns and groups, and the members of a group
+// in ascending token order.  Patches at the right and lower edge may hold
+// fewer than p * p tokens; member m of group g is the token in row m / p,
+// column m % p of the patch, when the frame has it.
+__host__ __device__ inline int grid_columns(int FSEQ, int W, int p) { return ((W < FSEQ ? W : FSEQ) - 1) / p + 1; }
+__host__ __device__ inline int grid_groups(int FSEQ, int W, int p) {
+  return ((FSEQ - 1) / W / p + 1) * grid_columns(FSEQ, W, p);
+}
+// first member of group g of the grid with `cols` columns
+__device__ inline int grid_first(int g, int W, int p, int cols) { return (g / cols) * p * W + (g % cols) * p; }
+__device__ inline bool grid_has(int g, int m, int FSEQ, int W, int p, int cols) {
+  const int x = (g % cols) * p + m % p;
+  return x < W && ((g / cols) * p + m / p) * W + x < FSEQ;
+}
+
 // group of token t on the arithmetic grid (y = t / W, x = t % W) in patches
 // of p (mega_merge_accum.cu:100-184, ids past the group count fold into 0)
 __device__ inline int32_t grid_gid(int t, int W, int p, int cols, int ng) {
@@ -939,7 +955,7 @@ __device__ void upd_merge_plan(const UpdArgs &a, int h, UpdShared &sh) {
   const int we = maxx + 1;
   sh.grid_cols = cols;
   sh.grid_ng = min(rows * cols, MTPA);
-  sh.grid_w = (p > 0 && FSEQ % we == 0 && we % p == 0 && (FSEQ / we) % p == 0 && rows * cols <= MTPA) ? we : 0;
+  sh.grid_w = (p > 0 && rows * cols <= MTPA) ? we : 0;
   for (int s = 0; s < a.MMA; ++s) {
     sh.s_src[s] = kSrcNone;
     sh.s_grid[s] = -1;
@@ -968,14 +984,14 @@ __device__ void upd_merge_plan(const UpdArgs &a, int h, UpdShared &sh) {
   }
 }
 
-// Width W of the regular patch grid when the group ids stored for a block
-// are exactly its ids (group of token t = ((t / W) / p) * (W / p) +
-// (t % W) / p), else 0; the same in every thread (a block-wide vote).
+// Width W of the patch grid when the group ids stored for a block are exactly
+// its ids (group of token t = ((t / W) / p) * columns + (t % W) / p), else 0;
+// the same in every thread (a block-wide vote).
 __device__ int stored_grid_width(const int32_t *gids, int FSEQ, int W, int p, int ng) {
-  const bool ok = W > 0 && p > 0 && FSEQ % W == 0 && W % p == 0 && (FSEQ / W) % p == 0 && ng == FSEQ / (p * p);
+  const bool ok = W > 0 && p > 0 && ng == grid_groups(FSEQ, W, p);
   bool bad = false;
   if (ok) {
-    const int cols = W / p;
+    const int cols = grid_columns(FSEQ, W, p);
     for (int t = threadIdx.x; t < FSEQ; t += blockDim.x) bad |= gids[t] != ((t / W) / p) * cols + (t % W) / p;
   }
   const int any_bad = __syncthreads_or(bad);
@@ -1003,8 +1019,9 @@ __host__ __device__ inline int64_t merge_lds_words(int FSEQ, int MMA) {
 
 // Patch chunks of a merge tile's groups in every frame of a call, loaded
 // before the record is staged and the state machine run: the members of a
-// group on the regular grid of width W = min(spatial width, FSEQ) depend on
-// nothing else.  merge_prefetch returns W, or 0 when the call does not
+// group on the grid of width W = min(spatial width, FSEQ) depend on nothing
+// else (members that an edge patch lacks load the group's first token, and
+// are not added).  merge_prefetch returns W, or 0 when the call does not
 // qualify (then nothing is loaded); frames whose lists turn out otherwise
 // load their members themselves.
 constexpr int kPreFrames = 3;
@@ -1034,17 +1051,21 @@ __device__ __forceinline__ int merge_prefetch(const UpdArgs &a, int h, int mt, M
   constexpr int p = kPrePatch;
   const int FSEQ = a.FSEQ, W = min(a.width, FSEQ);
   const MergeLane ln(a, mt);
-  if (a.F > kPreFrames || FSEQ % W != 0 || W % p != 0 || (FSEQ / W) % p != 0) return 0;
-  if (ln.own && ln.g < FSEQ / (p * p)) {
+  if (a.F > kPreFrames) return 0;
+  if (ln.own && ln.g < grid_groups(FSEQ, W, p)) {
     const uint16_t *src = ln.is_v ? a.src.v : a.src.k;
-    const int gcols = W / p;
-    const int gbase = (ln.g / gcols) * p * W + (ln.g % gcols) * p;
+    const int gcols = grid_columns(FSEQ, W, p);
+    const int gbase = grid_first(ln.g, W, p, gcols);
+    uint32_t off[kPreTok];
+#pragma unroll
+    for (int m = 0; m < kPreTok; ++m)
+      off[m] = (gbase + (grid_has(ln.g, m, FSEQ, W, p, gcols) ? (m / p) * W + m % p : 0)) * a.src_tb;
 #pragma unroll
     for (int f = 0; f < kPreFrames; ++f)
 #pragma unroll
       for (int m = 0; m < kPreTok; ++m)
         if (f < a.F && m < p * p)
-          pre.x[f][m] = ld16o(src, f * a.src_fb + h * a.src_hb + ln.c * 2 + (gbase + (m / p) * W + m % p) * a.src_tb);
+          pre.x[f][m] = ld16o(src, f * a.src_fb + h * a.src_hb + ln.c * 2 + off[m]);
   }
   return W;
 }
@@ -1119,11 +1140,11 @@ __device__ void upd_merge_tile(const UpdArgs &a, int h, int mt, UpdShared &sh, i
     return sh.s_grid[src_kind];
   };
   // Merge frame f.  kClosed: the lists are the closed form of width spec
-  // and pf holds the patch's chunks, loaded up front.  Otherwise, on a
-  // regular grid of width W the members are loaded here, and without one
-  // each thread scans the block's group ids (staged in LDS) for its group's
-  // tokens in ascending order -- the path of grids that do not tile into
-  // patches and of blocks begun with other positions.
+  // and pf holds the patch's chunks, loaded up front.  Otherwise, on the
+  // grid of width W the members are loaded here, and without one each thread
+  // scans the block's group ids (staged in LDS) for its group's tokens in
+  // ascending order -- the path of grids of more groups than an anchor holds
+  // and of blocks begun with other positions.
   auto frame = [&](int f, const uint4 *pf, auto closed_tag) {
     constexpr bool kClosed = decltype(closed_tag)::value;
     const int src_kind = sh.f_src[f];
@@ -1159,23 +1180,34 @@ __device__ void upd_merge_tile(const UpdArgs &a, int h, int mt, UpdShared &sh, i
       int cnt = p * p;  // members of group g
       if (g < ng) {
         if constexpr (kClosed) {
+          const int gcols = grid_columns(FSEQ, W, kPrePatch);
+          cnt = 0;
 #pragma unroll
           for (int m = 0; m < kPreTok; ++m)
-            if (m < p * p) add16(pf[m]);
+            if (grid_has(g, m, FSEQ, W, kPrePatch, gcols)) {
+              add16(pf[m]);
+              ++cnt;
+            }
         } else {
           const uint32_t fo = f * a.src_fb + h * a.src_hb + c * 2;
           if (W) {
-            const int gcols = W / p;
-            const int gbase = (g / gcols) * p * W + (g % gcols) * p;
+            const int gcols = grid_columns(FSEQ, W, p), gbase = grid_first(g, W, p, gcols);
+            cnt = 0;
             for (int mb = 0; mb < p * p; mb += kUpdAccBatch) {
               const int n = min(kUpdAccBatch, p * p - mb);
               uint4 xx[kUpdAccBatch];
+              bool has[kUpdAccBatch];
+#pragma unroll
+              for (int b = 0; b < kUpdAccBatch; ++b) {
+                has[b] = b < n && grid_has(g, mb + b, FSEQ, W, p, gcols);
+                if (has[b]) xx[b] = ld16o(src, fo + (gbase + ((mb + b) / p) * W + (mb + b) % p) * a.src_tb);
+              }
 #pragma unroll
               for (int b = 0; b < kUpdAccBatch; ++b)
-                if (b < n) xx[b] = ld16o(src, fo + (gbase + ((mb + b) / p) * W + (mb + b) % p) * a.src_tb);
-#pragma unroll
-              for (int b = 0; b < kUpdAccBatch; ++b)
-                if (b < n) add16(xx[b]);
+                if (has[b]) {
+                  add16(xx[b]);
+                  ++cnt;
+                }
             }
           } else {
             const int32_t *ids = src_kind == kSrcGrid ? dyn : dyn + merge_fseq_words(FSEQ) * (1 + src_kind);
@@ -1728,24 +1760,69 @@ __device__ inline void veil_apply_wave(const VeilStep &s, uint32_t &w) {
 constexpr int kEvTiles = 3;
 constexpr int kEvIdLoads = 2;  // 16-byte loads of stored group ids per thread
 constexpr int kEvMaxFseq = 4 * kEvIdLoads * kUpdThreads;
+
+// The group ids stored for a block, as the threads of a workgroup hold them
+// for the vote on whether they are the grid's: 16 bytes at a time where every
+// slot's ids start on a 16-byte boundary (kRagged: not known), else one.
+template <bool kRagged>
+struct GridIds {
+  static constexpr int kVec = kRagged ? 1 : 4, kLoads = 4 * kEvIdLoads / kVec;
+  int32_t v[kLoads][kVec];
+  __device__ void load(const int32_t *ids, int FSEQ) {
+    const int n = FSEQ / kVec;
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int i = min(static_cast<int>(threadIdx.x) + k * kUpdThreads, n - 1);
+      if constexpr (kRagged) {
+        v[k][0] = ids[i];
+      } else {
+        const int4 q = reinterpret_cast<const int4 *>(ids)[i];
+        v[k][0] = q.x; v[k][1] = q.y; v[k][2] = q.z; v[k][3] = q.w;
+      }
+    }
+  }
+  __device__ bool off_grid(int FSEQ, int W, int p, int cols) const {
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int i = static_cast<int>(threadIdx.x) + k * kUpdThreads;
+      if (i < FSEQ / kVec) {
+        int y = (kVec * i) / W, xx = (kVec * i) % W;
+#pragma unroll
+        for (int e = 0; e < kVec; ++e) {
+          bad |= v[k][e] != (y / p) * cols + xx / p;
+          if (++xx == W) {
+            xx = 0;
+            ++y;
+          }
+        }
+      }
+    }
+    return bad;
+  }
+};
+
 __host__ __device__ inline int evict_tile_groups(int D) { return kEvTiles * merge_tile_groups(D); }
 
 // One frame per call.  One wave-wide gather brings the record's decision
 // words, the frame time and weight and the slots' counts while the frame's
-// patch chunks (regular grid of patch 2) stream in; the step is decided in
+// patch chunks (patch 2) stream in; the step is decided in
 // scalar registers, and only a continued block then reads its slot's sums,
 // stored group ids (verified against the grid by a block-wide vote) and
 // anchor positions.  A head this path does not cover (another strategy kind
 // or patch size, a continued block whose stored ids are not the grid's)
 // runs update_kernel's merge tiles instead; the choice is the same in every
 // workgroup of the head.  Launched only where the frame's grid of width
-// W = spatial width tiles into 2 x 2 patches with at most MTPA of them, with
-// at most 2 accumulator slots, FSEQ <= kEvMaxFseq, head_dim >= 32 and
-// 16-byte aligned frames, sums and group ids (pkv_evict_merge checks).
+// W = min(spatial width, FSEQ) has at most MTPA 2 x 2 patches, with at most 2
+// accumulator slots, FSEQ <= kEvMaxFseq, head_dim >= 32 and 16-byte aligned
+// frames and sums (pkv_evict_merge checks).
 // The values the first reads need come as leading scalar arguments, which
 // the build preloads into scalar registers (-amdgpu-kernarg-preload-count),
 // so that the gather does not wait for a kernel-argument load; they repeat
 // fields of a.
+// kRagged: some patches lack members (their copies read zeros past the
+// resource's end and are added with weight 0, which changes no sum).
+template <bool kRagged>
 __global__ void __launch_bounds__(kUpdThreads)
     evict_kernel(const HeadState *states, const int64_t *t_vals, const float *weights, const int32_t *num_groups,
                  const float *weight_sum, int32_t n_merge, int32_t mma, UpdArgs a) {
@@ -1783,7 +1860,8 @@ __global__ void __launch_bounds__(kUpdThreads)
   __builtin_amdgcn_sched_barrier(0);
 
   const int FSEQ = a.FSEQ, D = a.D, MTPA = a.MTPA, MMA = mma, W = a.width;
-  const int cols = W / p, grid_ng = FSEQ / (p * p);
+  const int cols = kRagged ? grid_columns(FSEQ, W, p) : W / p;
+  const int grid_ng = kRagged ? grid_groups(FSEQ, W, p) : FSEQ / (p * p);
   const pkv_merge_layer &ml = a.ml;
   const MergeLane ln0(a, tile * kEvTiles);
   const int c = ln0.c, is_v = ln0.is_v;
@@ -1804,9 +1882,12 @@ __global__ void __launch_bounds__(kUpdThreads)
 #pragma unroll
   for (int j = 0; j < kEvTiles; ++j) {
     const int gc = min(g[j], grid_ng - 1);
-    const int gbase = (gc / cols) * p * W + (gc % cols) * p;
+    const int gbase = grid_first(gc, W, p, cols);
 #pragma unroll
-    for (int m = 0; m < kTok; ++m) x[j][m] = bld16_nt(srsrc, c * 2 + (gbase + (m / p) * W + m % p) * a.src_tb);
+    for (int m = 0; m < kTok; ++m) {
+      const bool has = !kRagged || grid_has(gc, m, FSEQ, W, p, cols);
+      x[j][m] = bld16_nt(srsrc, has ? c * 2 + (gbase + (m / p) * W + m % p) * a.src_tb : 0x80000000u);
+    }
   }
   // the chunk loads stay issued ahead of the first use of the gather
   __builtin_amdgcn_sched_barrier(0);
@@ -1853,11 +1934,8 @@ __global__ void __launch_bounds__(kUpdThreads)
   float wsum = 0.0f + fw;
   bool fast = veil;
   if (merging && !is_new) {
-    int4 ids[kEvIdLoads];
-    const int n4 = FSEQ / 4;
-#pragma unroll
-    for (int k = 0; k < kEvIdLoads; ++k)
-      ids[k] = reinterpret_cast<const int4 *>(ml.accum_group_ids + hs * FSEQ)[min(tid + k * kUpdThreads, n4 - 1)];
+    GridIds<kRagged> ids;
+    ids.load(ml.accum_group_ids + hs * FSEQ, FSEQ);
     float *acc_sum = is_v ? ml.accum_sum_v : ml.accum_sum_k;
 #pragma unroll
     for (int j = 0; j < kEvTiles; ++j) {
@@ -1873,23 +1951,7 @@ __global__ void __launch_bounds__(kUpdThreads)
     }
     ng = min(slot ? ng1 : ng0, MTPA);
     wsum = (slot ? ws1 : ws0) + fw;
-    bool bad = false;
-#pragma unroll
-    for (int k = 0; k < kEvIdLoads; ++k) {
-      const int i = tid + k * kUpdThreads;
-      if (i < n4) {
-        int y = (4 * i) / W, xx = (4 * i) % W;
-        const int32_t v[4] = {ids[k].x, ids[k].y, ids[k].z, ids[k].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          bad |= v[e] != (y / p) * cols + xx / p;
-          if (++xx == W) {
-            xx = 0;
-            ++y;
-          }
-        }
-      }
-    }
+    const bool bad = ids.off_grid(FSEQ, W, p, cols);
     if (tid == 0) sh.last = early;
     fast = ng == grid_ng && !__syncthreads_or(bad);
   } else {
@@ -1936,14 +1998,21 @@ __global__ void __launch_bounds__(kUpdThreads)
         ax[0] = acc[j][0].x; ax[1] = acc[j][0].y; ax[2] = acc[j][0].z; ax[3] = acc[j][0].w;
         ax[4] = acc[j][1].x; ax[5] = acc[j][1].y; ax[6] = acc[j][1].z; ax[7] = acc[j][1].w;
       }
+      int cnt = kTok;  // members of the group
+      if (kRagged) {
+        cnt = 0;
+#pragma unroll
+        for (int m = 0; m < kTok; ++m) cnt += grid_has(gj, m, FSEQ, W, p, cols);
+      }
       if (gj < ng) {
 #pragma unroll
         for (int m = 0; m < kTok; ++m) {
           const uint32_t xw[4] = {x[j][m].x, x[j][m].y, x[j][m].z, x[j][m].w};
+          const float mw = !kRagged || grid_has(gj, m, FSEQ, W, p, cols) ? fw : 0.0f;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            ax[2 * e] += fw * bf16_to_f32(static_cast<uint16_t>(xw[e] & 0xffff));
-            ax[2 * e + 1] += fw * bf16_to_f32(static_cast<uint16_t>(xw[e] >> 16));
+            ax[2 * e] += mw * bf16_to_f32(static_cast<uint16_t>(xw[e] & 0xffff));
+            ax[2 * e + 1] += mw * bf16_to_f32(static_cast<uint16_t>(xw[e] >> 16));
           }
         }
       }
@@ -1954,11 +2023,11 @@ __global__ void __launch_bounds__(kUpdThreads)
       // a block begun here: the group ids of the group's members, one
       // member per K-side thread (no workgroup of the head reads them in
       // this call)
-      if (is_new && !is_v && c < 8 * kTok && gj < ng)
+      if (is_new && !is_v && c < 8 * kTok && gj < ng && (!kRagged || grid_has(gj, c / 8, FSEQ, W, p, cols)))
         ml.accum_group_ids[hs * FSEQ + (gj / cols) * p * W + (gj % cols) * p + (c / 8 / p) * W + (c / 8) % p] = gj;
       if (is_new && meta_lane) {
         ml.accum_tokens_per_group[hs * MTPA + gj] =
-            gj < ng ? static_cast<float>(kTok) * static_cast<float>(bf) : 0.0f;
+            gj < ng ? static_cast<float>(cnt) * static_cast<float>(bf) : 0.0f;
         if (gj < ng) {
           int64_t *pp = ml.accum_pos + (hs * MTPA + gj) * 3;
           pp[0] = t;
@@ -1968,7 +2037,7 @@ __global__ void __launch_bounds__(kUpdThreads)
       }
       if (fin >= 0 && fin < a.MMB && gj < ng) {
         // count * sum(w) for weighted merges, else the reference's count * block_frames
-        const float div = static_cast<float>(kTok) * (a.weights ? wsum : static_cast<float>(bf));
+        const float div = static_cast<float>(cnt) * (a.weights ? wsum : static_cast<float>(bf));
         const float inv = div > 0.0f ? 1.0f / div : 0.0f;
         const int64_t hp = static_cast<int64_t>(h) * a.MMB + fin;
         uint4 ox;
@@ -2055,6 +2124,7 @@ static int frames_tile_groups(int H, int MTPA, int D) {
   return best;
 }
 
+template <bool kRagged>
 __global__ void __launch_bounds__(kUpdThreads)
     evict_frames_kernel(const HeadState *states, const int64_t *t_vals, const float *weights,
                         const int32_t *num_groups, const float *weight_sum, int32_t n_merge, int32_t mma, UpdArgs a) {
@@ -2092,7 +2162,8 @@ __global__ void __launch_bounds__(kUpdThreads)
   __builtin_amdgcn_sched_barrier(0);
 
   const int FSEQ = a.FSEQ, D = a.D, MTPA = a.MTPA, W = a.width;
-  const int cols = W / p, grid_ng = FSEQ / (p * p);
+  const int cols = kRagged ? grid_columns(FSEQ, W, p) : W / p;
+  const int grid_ng = kRagged ? grid_groups(FSEQ, W, p) : FSEQ / (p * p);
   const pkv_merge_layer &ml = a.ml;
   // a tile is gpt groups (the host's choice, at most merge_tile_groups(D)):
   // lanes of the wave pairs' groups past gpt idle (no copies, no writes)
@@ -2122,12 +2193,23 @@ __global__ void __launch_bounds__(kUpdThreads)
   uint32_t toff[kTok];
   {
     const int gc = min(g, grid_ng - 1);
-    const int gbase = (gc / cols) * p * W + (gc % cols) * p;
-    // an idle lane's offset lies past the resource's end (the frames' bytes
-    // are below 2^31): its copies read zeros and fetch nothing
+    const int gbase = grid_first(gc, W, p, cols);
+    // the offset of an idle lane, or of a member the group lacks, lies past
+    // the resource's end (the frames' bytes are below 2^31): its copies read
+    // zeros and fetch nothing
 #pragma unroll
     for (int m = 0; m < kTok; ++m)
-      toff[m] = local < gpt ? c * 2 + (gbase + (m / p) * W + m % p) * a.src_tb : 0x80000000u;
+      toff[m] = local < gpt && (!kRagged || grid_has(gc, m, FSEQ, W, p, cols))
+                    ? c * 2 + (gbase + (m / p) * W + m % p) * a.src_tb
+                    : 0x80000000u;
+  }
+  int cnt = kTok;      // members of the group
+  uint32_t has = 0xf;  // bit m: it has member m
+  if (kRagged) {
+    has = 0;
+#pragma unroll
+    for (int m = 0; m < kTok; ++m) has |= grid_has(g, m, FSEQ, W, p, cols) ? 1u << m : 0u;
+    cnt = __popc(has);
   }
   const int wave_s = uni(wave);
   typedef __attribute__((address_space(3))) char lds_char_t;
@@ -2211,11 +2293,8 @@ __global__ void __launch_bounds__(kUpdThreads)
     for (int e = 0; e < 8; ++e) ax[sl][e] = 0.0f;
     if (!(cont & (1u << sl))) continue;
     const int64_t hs = hs0 + sl;
-    int4 ids[kEvIdLoads];
-    const int n4 = FSEQ / 4;
-#pragma unroll
-    for (int k = 0; k < kEvIdLoads; ++k)
-      ids[k] = reinterpret_cast<const int4 *>(ml.accum_group_ids + hs * FSEQ)[min(tid + k * kUpdThreads, n4 - 1)];
+    GridIds<kRagged> ids;
+    ids.load(ml.accum_group_ids + hs * FSEQ, FSEQ);
     const float *acc_sum = is_v ? ml.accum_sum_v : ml.accum_sum_k;
     const float4 *ap = reinterpret_cast<const float4 *>(acc_sum + (hs * MTPA + min(g, MTPA - 1)) * D + c);
     const float4 a0 = ap[0], a1 = ap[1];
@@ -2225,23 +2304,7 @@ __global__ void __launch_bounds__(kUpdThreads)
 #pragma unroll
       for (int e = 0; e < 3; ++e) apos[sl][e] = ml.accum_pos[(hs * MTPA + min(g, MTPA - 1)) * 3 + e];
     }
-    bool bad = min(sl ? ng1 : ng0, MTPA) != grid_ng;
-#pragma unroll
-    for (int k = 0; k < kEvIdLoads; ++k) {
-      const int i = tid + k * kUpdThreads;
-      if (i < n4) {
-        int y = (4 * i) / W, xx = (4 * i) % W;
-        const int32_t v[4] = {ids[k].x, ids[k].y, ids[k].z, ids[k].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          bad |= v[e] != (y / p) * cols + xx / p;
-          if (++xx == W) {
-            xx = 0;
-            ++y;
-          }
-        }
-      }
-    }
+    const bool bad = min(sl ? ng1 : ng0, MTPA) != grid_ng || ids.off_grid(FSEQ, W, p, cols);
     fast = fast && !__syncthreads_or(bad);
   }
   if (tid == 0) sh.last = early;
@@ -2314,20 +2377,21 @@ __global__ void __launch_bounds__(kUpdThreads)
 #pragma unroll
           for (int m = 0; m < kTok; ++m) {
             const uint32_t xw[4] = {xr[m].x, xr[m].y, xr[m].z, xr[m].w};
+            const float mw = !kRagged || (has >> m & 1u) ? fw : 0.0f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              ax[sl][2 * e] += fw * bf16_to_f32(static_cast<uint16_t>(xw[e] & 0xffff));
-              ax[sl][2 * e + 1] += fw * bf16_to_f32(static_cast<uint16_t>(xw[e] >> 16));
+              ax[sl][2 * e] += mw * bf16_to_f32(static_cast<uint16_t>(xw[e] & 0xffff));
+              ax[sl][2 * e + 1] += mw * bf16_to_f32(static_cast<uint16_t>(xw[e] >> 16));
             }
           }
         }
         // a block begun here: the group ids of the group's members (one
         // member per K-side thread), its count and anchor positions
-        if (is_new && !is_v && c < 8 * kTok && g < grid_ng)
+        if (is_new && !is_v && c < 8 * kTok && g < grid_ng && (has >> (c / 8) & 1u))
           ml.accum_group_ids[hs * FSEQ + (g / cols) * p * W + (g % cols) * p + (c / 8 / p) * W + (c / 8) % p] = g;
         if (is_new && meta_lane) {
           ml.accum_tokens_per_group[hs * MTPA + g] =
-              g < grid_ng ? static_cast<float>(kTok) * static_cast<float>(bf) : 0.0f;
+              g < grid_ng ? static_cast<float>(cnt) * static_cast<float>(bf) : 0.0f;
           if (g < grid_ng) {
             int64_t *pp = ml.accum_pos + (hs * MTPA + g) * 3;
             pp[0] = t;
@@ -2337,7 +2401,7 @@ __global__ void __launch_bounds__(kUpdThreads)
         }
         if (fin >= 0 && fin < a.MMB && g < grid_ng) {
           // count * sum(w) for weighted merges, else the reference's count * block_frames
-          const float div = static_cast<float>(kTok) * (a.weights ? wsum[sl] : static_cast<float>(bf));
+          const float div = static_cast<float>(cnt) * (a.weights ? wsum[sl] : static_cast<float>(bf));
           const float inv = div > 0.0f ? 1.0f / div : 0.0f;
           const int64_t hp = static_cast<int64_t>(h) * a.MMB + fin;
           uint4 ox;
@@ -2725,36 +2789,37 @@ int pkv_evict_merge(uint8_t *states, int32_t H, int32_t F, int32_t FSEQ, int32_t
   u.n_scat = 0;
   u.n_mh = H;
   u.merge_heads = H >= 64 ? ~uint64_t{0} : (uint64_t{1} << H) - 1;
-  // frames on a grid of 2 x 2 patches: evict_kernel (one frame) or
+  // patch grids of at most MTPA groups: evict_kernel (one frame) or
   // evict_frames_kernel (several), which still run update_kernel's merge
-  // tile for heads their path does not cover
+  // tile for heads their path does not cover.  Grids that tile into 2 x 2
+  // patches, with slots' ids 16-byte aligned, take the instances without
+  // members to leave out (40 frames of 12 heads: 107 us on 30 x 52 tokens; on
+  // 29 x 51 108 us, against 3,708 in update_kernel, whose threads scanned the
+  // frame's ids for their group's members; one frame 12 against 108 us).
   auto al16 = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  const int W = spatial_width;
-  const bool grid = MMA <= 2 && W <= FSEQ && FSEQ % W == 0 && W % 2 == 0 && (FSEQ / W) % 2 == 0 &&
-                    FSEQ / 4 <= MTPA && FSEQ <= kEvMaxFseq && D >= 8 * kPreTok && al16(new_k) && al16(new_v) &&
-                    al16(ml->accum_sum_k) && al16(ml->accum_sum_v) && al16(ml->accum_group_ids);
+  const int W = std::min(spatial_width, FSEQ);
+  const bool grid = MMA <= 2 && grid_groups(FSEQ, W, kPrePatch) <= MTPA && FSEQ <= kEvMaxFseq && D >= 8 * kPreTok &&
+                    al16(new_k) && al16(new_v) && al16(ml->accum_sum_k) && al16(ml->accum_sum_v);
+  const bool ragged = FSEQ % W != 0 || W % 2 != 0 || (FSEQ / W) % 2 != 0 || !al16(ml->accum_group_ids);
   const bool one = grid && F == 1, many = grid && F > 1;
+  if (grid) u.width = W;
   int gpt = one ? evict_tile_groups(D) : merge_tile_groups(D);
   if (many) gpt = frames_tile_groups(H, MTPA, D);
   u.n_merge = (MTPA + gpt - 1) / gpt;
-  const void *kern = one ? reinterpret_cast<const void *>(evict_kernel)
-                         : many ? reinterpret_cast<const void *>(evict_frames_kernel)
+  auto *one_k = ragged ? evict_kernel<true> : evict_kernel<false>;
+  auto *many_k = ragged ? evict_frames_kernel<true> : evict_frames_kernel<false>;
+  const void *kern = one ? reinterpret_cast<const void *>(one_k)
+                         : many ? reinterpret_cast<const void *>(many_k)
                                 : reinterpret_cast<const void *>(update_kernel);
   size_t smem = static_cast<size_t>(merge_lds_words(FSEQ, MMA)) * sizeof(int32_t);
   if (many) smem = std::max(smem, static_cast<size_t>(kEfRing) * (kUpdThreads / 64) * kPreTok * 1024);
   if (smem > 65536 &&
       hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem)) != hipSuccess)
     return fail(PKV_ERR_HIP, "evict_merge: cannot reserve %zu bytes of LDS", smem);
-  if (one) {
-    hipLaunchKernelGGL(evict_kernel, dim3(H * u.n_merge), dim3(kUpdThreads), smem, as_stream(stream), u.states,
+  if (grid) {
+    hipLaunchKernelGGL(one ? one_k : many_k, dim3(H * u.n_merge), dim3(kUpdThreads), smem, as_stream(stream), u.states,
                        u.t_vals, u.weights, u.ml.accum_num_groups, u.ml.accum_weight_sum, u.n_merge, u.MMA, u);
-    return check_launch("evict_kernel");
-  }
-  if (many) {
-    hipLaunchKernelGGL(evict_frames_kernel, dim3(H * u.n_merge), dim3(kUpdThreads), smem, as_stream(stream),
-                       u.states, u.t_vals, u.weights, u.ml.accum_num_groups, u.ml.accum_weight_sum, u.n_merge, u.MMA,
-                       u);
-    return check_launch("evict_frames_kernel");
+    return check_launch(one ? "evict_kernel" : "evict_frames_kernel");
   }
   hipLaunchKernelGGL(update_kernel, dim3(H * u.n_merge), dim3(kUpdThreads), smem, as_stream(stream), u);
   return check_launch("update_kernel");

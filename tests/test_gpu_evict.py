@@ -195,3 +195,34 @@ def test_evict_frames_long_calls(F):
     calls = [list(range(1, F + 1)), list(range(F + 1, F + 7))]
     recs = [O.make_merge(2, 6), O.make_merge(2, 2)]
     _evict_run(H=2, FSEQ=1560, W=52, calls=calls, seed=20 + F, weighted=True, recs=recs)
+
+
+@pytest.mark.parametrize("FSEQ,W,D_", [
+    (29 * 51, 51, 128),   # short patches at the right and lower edge
+    (30 * 51, 51, 128),   # at the right edge alone
+    (29 * 52, 52, 64),    # at the lower edge alone; slots' ids 16-byte aligned
+    (1000, 37, 128),      # a last row of 1 token
+    (41, 60, 128),        # one row, narrower than the grid
+    (7 * 2, 2, 128),      # one column of patches
+    (419, 1, 32),         # one token wide
+    (1900, 45, 128),      # more groups than an anchor holds: ids past the last fold into group 0
+])
+@pytest.mark.parametrize("F", [1, 3])
+def test_evict_grids_with_short_patches(FSEQ, W, D_, F):
+    calls = [[2 + F * b + f for f in range(F)] for b in range(12 // F)]
+    _evict_run(H=2, FSEQ=FSEQ, W=W, calls=calls, seed=FSEQ + F, weighted=F == 1, D=D_)
+
+
+def test_evict_short_patches_blocks_out_of_order_and_other_heads():
+    # both slots busy, repeated frames, a Wave head beside the Veil heads, and a
+    # block whose stored ids are another grid's when it continues
+    rng = np.random.default_rng(77)
+    calls = [[int(t) for t in rng.integers(0, 24, n)] for n in (5, 1, 8, 3, 1, 6, 40)]
+
+    def tamper(ci, acc, dacc):
+        if ci == 4:
+            acc["gid"][1] = acc["gid"][1][:, ::-1]
+            dacc["gid"].copy_(to_dev(acc["gid"]))
+
+    _evict_run(H=3, FSEQ=21 * 33, W=33, calls=calls, seed=9, weighted=True, kinds=["merge", "merge", "cyclic"],
+               tamper=tamper)
