@@ -311,6 +311,12 @@ int pkv_anchor_store_write_frames(const void *k_seq, const void *v_seq,
                                   int64_t capacity, int64_t frame_seqlen,
                                   int64_t row_bytes, pkv_stream_t stream);
 
+/* A layer's recent FIFO (K, V [H, max_recent, FSEQ, D] and positions) copied
+ * to the caller's buffers of the same shapes, or back from them (restore = 1),
+ * in one launch (the snapshot and restore of _mega_cache.py:226-245, 406-414). */
+int pkv_recent_fifo_copy(const pkv_geometry *geo, const pkv_pools *pools, int32_t layer, uint16_t *k,
+                         uint16_t *v, int64_t *pos, int32_t restore, pkv_stream_t stream);
+
 /* pyramidkv_plan (legacy): over all L*H heads, three segments each in the
  * order sink, recent, middle covering slots 0..valid_count-1; outputs cu
  * [L*H+1] and [3*L*H] descriptor arrays (int32, device). */

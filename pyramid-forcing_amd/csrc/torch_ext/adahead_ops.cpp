@@ -1134,6 +1134,30 @@ static Tensor attend_kv_layer(const Mgr &mgr, const Tensor &states, int64_t laye
                  decoupled_sink_lag, ft, fy, fx);
 }
 
+// The layer's recent FIFO into (or, restore, from) tensors of its pools' shapes.
+static void recent_fifo_copy(const Mgr &mgr, int64_t layer, const Tensor &k, const Tensor &v, const Tensor &pos,
+                             bool restore) {
+  TORCH_CHECK(layer >= 0 && layer < mgr->num_layers(), "recent_fifo_copy: layer out of range");
+  const c10::Device dev = mgr->valid_count().device();
+  if (!dev.is_cuda() || mgr->recent_k_pool().scalar_type() != at::kBFloat16) {  // pools that no kernel updates
+    const Tensor pool[3] = {mgr->recent_k_pool().select(0, layer), mgr->recent_v_pool().select(0, layer),
+                            mgr->recent_pos_pool().select(0, layer)};
+    const Tensor mine[3] = {k, v, pos};
+    for (int i = 0; i < 3; ++i) (restore ? pool[i] : mine[i]).copy_(restore ? mine[i] : pool[i]);
+    return;
+  }
+  const std::vector<int64_t> kv = {mgr->num_heads(), mgr->max_recent(), mgr->frame_seqlen(), mgr->head_dim()};
+  expect_tensor(k, at::kBFloat16, kv, dev, "recent_fifo_copy", "k");
+  expect_tensor(v, at::kBFloat16, kv, dev, "recent_fifo_copy", "v");
+  expect_tensor(pos, at::kLong, {kv[0], kv[1], kv[2], 3}, dev, "recent_fifo_copy", "pos");
+  const pkv_geometry g = mgr->geometry();
+  const pkv_pools p = mgr->pools();
+  pkv_check(pkv_recent_fifo_copy(&g, &p, static_cast<int32_t>(layer), reinterpret_cast<uint16_t *>(k.data_ptr()),
+                                 reinterpret_cast<uint16_t *>(v.data_ptr()), pos.data_ptr<int64_t>(), restore ? 1 : 0,
+                                 stream_for(k)),
+            "recent_fifo_copy");
+}
+
 // attend_kv_layer, then the attention of q [num_chunks * frame_seqlen, H, D]
 // over the packed keys.
 static Tensor attend_layer(const Mgr &mgr, const Tensor &states, int64_t layer, int64_t t0, int64_t num_chunks,
@@ -1264,6 +1288,9 @@ TORCH_LIBRARY(adahead, m) {
               int64_t width, int64_t heads) {
              adahead::update_layer(m, st, caps, vc, k, v, layer, t0, pass_kind, pending, width, heads);
            })
+      .def("recent_fifo_copy",
+           [](const adahead::Mgr &m, int64_t layer, const at::Tensor &k, const at::Tensor &v, const at::Tensor &pos,
+              bool restore) { adahead::recent_fifo_copy(m, layer, k, v, pos, restore); })
       .def("attend_kv_layer", &adahead::attend_kv_layer)
       .def("attend_layer", &adahead::attend_layer);
 

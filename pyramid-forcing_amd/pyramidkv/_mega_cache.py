@@ -145,17 +145,12 @@ class MegaCache:
         (restore=False), or back from it (restore=True)."""
         ctx, l = self.ctx, self.layer_idx
         mgr = ctx.mgr
-        pools = (mgr.recent_k_pool()[l], mgr.recent_v_pool()[l], mgr.recent_pos_pool()[l])
         backup = ctx.recent_backup.get(l)
-        if restore:
-            for dst, src in zip(pools, backup):
-                dst.copy_(src)
-            return
         if backup is None:
-            backup = tuple(torch.empty_like(t) for t in pools)
+            backup = tuple(torch.empty_like(t[l]) for t in (mgr.recent_k_pool(), mgr.recent_v_pool(),
+                                                            mgr.recent_pos_pool()))
             ctx.recent_backup[l] = backup
-        for dst, src in zip(backup, pools):
-            dst.copy_(src)
+        mgr.recent_fifo_copy(l, *backup, restore)
 
     def last_update_descriptors(self, frames: int):
         """The 8 state-machine descriptor arrays of the last update call."""

@@ -45,3 +45,24 @@ def test_methods_equal_ops(layers, layer):
         for name in ("recent_k_pool", "middle_v_pool", "merge_k_pool", "valid_count", "merge_token_count"):
             assert torch.equal(getattr(a.ctx.mgr, name)(), getattr(ctx.mgr, name)()), (blk, name)
         assert torch.equal(a.ctx.states_bytes, ctx.states_bytes)
+
+
+# one token of positions more than a 16-byte multiple; a layer whose FIFO starts off one; several workgroups
+@pytest.mark.parametrize("layers,heads,D,FS,recent", [(3, 1, 8, 5, 1), (2, 3, 128, 63, 3), (2, 4, 64, 700, 4),
+                                                      (3, 1, 24, 341, 1)])
+def test_recent_fifo_copy_and_restore(layers, heads, D, FS, recent):
+    mgr = torch.classes.adahead.PyramidKVCacheManager(layers, heads, D, FS, 1, 1, recent, DEV, "bfloat16", 1)
+    pools = (mgr.recent_k_pool(), mgr.recent_v_pool(), mgr.recent_pos_pool())
+    g = torch.Generator(device=DEV)
+    g.manual_seed(FS)
+    for t in pools:
+        t.copy_(torch.randint(-1000, 1000, t.shape, generator=g, device=DEV))
+    want = [t.clone() for t in pools]
+    for layer in range(layers):
+        mine = [torch.zeros_like(t[layer]) for t in pools]
+        mgr.recent_fifo_copy(layer, *mine, False)
+        assert all(torch.equal(a, t[layer]) for a, t in zip(mine, want))
+        for t in pools:
+            t[layer].zero_()
+        mgr.recent_fifo_copy(layer, *mine, True)
+        assert all(torch.equal(a, b) for a, b in zip(pools, want))
