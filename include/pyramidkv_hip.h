@@ -360,16 +360,16 @@ int pkv_ragged_attn_fwd(const pkv_attn_args *args, pkv_stream_t stream);
 
 /* The same attention with a device workspace (replaces the same call,
  * _mega_cache.py:540-559).  Launches of head_dim 128 whose query tiles of 256
- * rows occupy at most 9/10 of the compute units (and of at most 256
- * sequences) may split sequences' keys into chunks, so that the (query tile,
+ * rows occupy at most 9/10 of the compute units, or take one to one and a half
+ * rounds of them (and of at most 256 sequences), may split sequences' keys into chunks, so that the (query tile,
  * chunk) items fill the units, and merge a query tile's chunks in a second
  * launch, in chunk order (deterministic).  Other launches, or a workspace
  * smaller than pkv_ragged_attn_workspace_size(), run as pkv_ragged_attn_fwd.
  * The workspace needs no initialisation; calls sharing one must be ordered
  * (one stream).  pkv_ragged_attn_workspace_for: the bytes that would serve
- * these arguments, 0 where no workspace would be used; max_seqlen_k is an
- * upper bound of a sequence's keys (0 = unknown). */
-int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *args, int64_t max_seqlen_k);
+ * these arguments, 0 where none would be used or gain anything; keys is the
+ * number of keys a sequence is expected to have (0 = unknown). */
+int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *args, int64_t keys);
 int64_t pkv_ragged_attn_workspace_size(void);
 int pkv_ragged_attn_fwd_ws(const pkv_attn_args *args, void *workspace, int64_t workspace_bytes,
                            pkv_stream_t stream);

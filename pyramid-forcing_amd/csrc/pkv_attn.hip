@@ -86,8 +86,9 @@ struct AttnParams {
   int64_t q_tok, q_head, kv_tok, kv_head, o_tok, o_head;
   float scale_log2;
   // key-split launches (attn_pp_kernel<true> + attn_combine_kernel): the
-  // items' partial results in the caller's workspace
+  // items' partial results in the caller's workspace, and its head
   float *part;
+  int *head;
   int n_seq, n_cu;
   // queue launches of attn_p3_kernel (one workgroup per compute
   // unit, items claimed from per-XCD counters): this stream's counter
@@ -331,20 +332,25 @@ __device__ void queue_done(int *queue) {
 // Every wave of both launches computes the same plan from cu_q / cu_k in
 // registers (no LDS, no barrier; lane i holds sequences i, i + 64, ...).
 // Keys are counted in units of kSplitUnit tiles, the key loop's unroll.  With
-// at most R * n_cu items (R = 1, and 2 when the launch has room for it) the
-// chunk length C is the smallest that fits, at least kSplitMinUnits; sequence
-// s has k_s = ceil(units_s / C) chunks of equal length (+-1 unit).  Chosen is
-// the least estimated time in units (an item costs its units and
-// kSplitItemUnits more; a unit is 2.6-3.1 us):
-//   unsplit  longest
+// at most R * n_cu items the chunk length C is the smallest that fits, at
+// least kSplitMinUnits; sequence s has k_s = ceil(units_s / C) chunks of equal
+// length (+-1 unit).  Chosen is the least estimated time in units (an item
+// costs its units and kSplitItemUnits more; a unit is 2.6-3.1 us), of the R
+// that the launch has workgroups for:
+//   unsplit  longest, for at most one tile per compute unit;
+//            2 * mean + (longest - mean) / 2 for more (two rounds)
 //   R = 1    C + kSplitFixedUnits
 //   R = 2    sum of the items' units / n_cu + C / 3 + 2 * kSplitFixedUnits
-// (the fixed part is the second launch and the partial results' traffic, C / 3
-// the unevenness of a second round).  Measured against all the alternatives
-// on 28 shapes of 6-252 tiles it took the fastest one or one within 5%: for
-// instance 168 tiles of 12,480-17,160 keys 353 us unsplit, 337 in one round
-// and 290 in two; 209 tiles of 3,000-5,000 keys 118, 130 and 130; 81 tiles of
-// 3,200-5,000 keys 112, 64 and 75.
+//   R = 3    sum of the items' units / n_cu + C / 2 + 3 * kSplitFixedUnits,
+//            only with more tiles than units and 5% less than unsplit
+// (the fixed part is the second launch and the partial results' traffic, the
+// part of C the unevenness of the last round).  Measured against all the
+// alternatives on 40 shapes of 6-684 tiles it took the fastest one or one
+// within 6%: for instance 168 tiles of 12,480-17,160 keys 353 us unsplit, 337
+// in one round and 290 in two; 209 tiles of 3,000-5,000 keys 118, 130 and 130;
+// 81 tiles of 3,200-5,000 keys 112, 64 and 75; 336 tiles of 8,000-14,000 keys
+// 533, 522 in two rounds and 464 in three; 320 tiles of 3,000-6,000 keys 207,
+// 218 and 221.
 // Items are numbered base_s + j * nq_s + qt, so a chunk's query tiles are
 // consecutive and, numbered by xcd_remap, share their keys in one XCD's L2.
 constexpr int kSplitSeqLanes = 4;                    // sequences per lane
@@ -356,7 +362,7 @@ constexpr int kSplitFixedUnits = 4;
 
 struct SplitPlan {
   int nq[kSplitSeqLanes], nu[kSplitSeqLanes], k[kSplitSeqLanes], base[kSplitSeqLanes];
-  int n_items;
+  int n_items, tiles, chunk;
 };
 
 // One item: query tile qt of sequence seq (of nq tiles) against units
@@ -369,7 +375,9 @@ __device__ inline int div_up(int a, int b) {
   return static_cast<int>(static_cast<unsigned>(a + b - 1) / static_cast<unsigned>(b));
 }
 
-__device__ inline SplitPlan split_plan(const AttnParams &p) {
+// chunk: the plan's C where it is known (attn_combine_kernel reads it from the
+// workspace's head), -1 to choose it.
+__device__ inline SplitPlan split_plan(const AttnParams &p, int chunk) {
   SplitPlan s;
   const int lane = threadIdx.x & 63;
   auto wave_total = [](int x) { return __builtin_amdgcn_readlane(wave_incl_sum(x), 63); };
@@ -389,39 +397,49 @@ __device__ inline SplitPlan split_plan(const AttnParams &p) {
     work += s.nq[i] * s.nu[i];
     longest = max(longest, s.nu[i]);
   }
-  tiles = wave_total(tiles);
-  work = wave_total(work);
+  int C = chunk;
+  if (chunk < 0) {
+    tiles = wave_total(tiles);
+    work = wave_total(work);
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
-  longest = __builtin_amdgcn_readfirstlane(longest);
-  auto items = [&](int C) {
-    int n = 0;
+    for (int off = 32; off >= 1; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+    longest = __builtin_amdgcn_readfirstlane(longest);
+    auto items = [&](int C) {
+      int n = 0;
 #pragma unroll
-    for (int i = 0; i < kSplitSeqLanes; ++i) n += s.nq[i] * (s.nu[i] <= C ? 1 : div_up(s.nu[i], C));
-    return wave_total(n);
-  };
-  // chunk lengths are tried in [work / G, work / (G - tiles)]: no shorter one
-  // can fit G items, and that one does (items <= work / C + tiles)
-  auto shortest = [&](int G) {
-    int lo = max(kSplitMinUnits, work / G), hi = max(lo, min(longest, div_up(work, max(1, G - tiles))));
-    while (lo < hi) {
-      const int C = (lo + hi) >> 1;
-      if (items(C) <= G) hi = C;
-      else lo = C + 1;
+      for (int i = 0; i < kSplitSeqLanes; ++i) n += s.nq[i] * (s.nu[i] <= C ? 1 : div_up(s.nu[i], C));
+      return wave_total(n);
+    };
+    // chunk lengths are tried in [work / G, work / (G - tiles)]: no shorter one
+    // can fit G items, and that one does (items <= work / C + tiles)
+    auto shortest = [&](int G) {
+      int lo = max(kSplitMinUnits, work / G), hi = max(lo, min(longest, div_up(work, max(1, G - tiles))));
+      while (lo < hi) {
+        const int C = (lo + hi) >> 1;
+        if (items(C) <= G) hi = C;
+        else lo = C + 1;
+      }
+      return lo;
+    };
+    const int mean = work / max(1, tiles);
+    C = max(1, longest);
+    int best = tiles <= p.n_cu ? longest : 2 * mean + (longest - mean) / 2;
+    if (tiles > p.n_cu) {
+      const int c3 = shortest(p.n_wg);
+      const int t = (work + kSplitItemUnits * (items(c3) - tiles)) / p.n_cu + c3 / 2 + 3 * kSplitFixedUnits;
+      if (t + t / 20 < best) C = c3;
     }
-    return lo;
-  };
-  int C = max(1, longest), best = longest;
-  if (tiles < p.n_cu) {
-    const int c1 = shortest(p.n_cu);
-    if (c1 + kSplitFixedUnits < best) {
-      C = c1;
-      best = c1 + kSplitFixedUnits;
+    if (tiles < p.n_cu) {
+      const int c1 = shortest(p.n_cu);
+      if (c1 + kSplitFixedUnits < best) {
+        C = c1;
+        best = c1 + kSplitFixedUnits;
+      }
     }
-  }
-  if (p.n_wg >= 2 * p.n_cu) {
-    const int c2 = shortest(2 * p.n_cu);
-    if ((work + kSplitItemUnits * (items(c2) - tiles)) / p.n_cu + c2 / 3 + 2 * kSplitFixedUnits < best) C = c2;
+    if (tiles <= p.n_cu && p.n_wg >= 2 * p.n_cu) {
+      const int c2 = shortest(2 * p.n_cu);
+      if ((work + kSplitItemUnits * (items(c2) - tiles)) / p.n_cu + c2 / 3 + 2 * kSplitFixedUnits < best) C = c2;
+    }
   }
   int run = 0;
 #pragma unroll
@@ -432,6 +450,8 @@ __device__ inline SplitPlan split_plan(const AttnParams &p) {
     run += __builtin_amdgcn_readlane(incl, 63);
   }
   s.n_items = run;
+  s.chunk = C;
+  s.tiles = tiles;
   return s;
 }
 
@@ -906,7 +926,10 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
   int slot_idx = 0;
   const int n_seq = p.n_wg / p.q_tiles;
   if constexpr (SPLIT) {
-    const SplitPlan plan = split_plan(p);
+    const SplitPlan plan = split_plan(p, -1);
+    // the workspace's head: the chunk length, 0 when no tile has two chunks
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      *p.head = __builtin_amdgcn_readfirstlane(plan.tiles) == plan.n_items ? 0 : plan.chunk;
     if (static_cast<int>(blockIdx.x) >= plan.n_items) return;
     slot_idx = xcd_remap(blockIdx.x, plan.n_items);
     it = split_item(plan, slot_idx);
@@ -2039,7 +2062,9 @@ __global__ void __launch_bounds__(64 * kCombineWaves) attn_combine_kernel(AttnPa
   const int Lq = p.cu_q[b + 1] - q_begin;
   const int q0 = qt * 32 * kWaves;
   if (q0 + wave * 32 >= Lq) return;
-  const SplitPlan s = split_plan(p);
+  const int chunk = *(const __attribute__((address_space(4))) int *)p.head;
+  if (chunk == 0) return;
+  const SplitPlan s = split_plan(p, chunk);
   int k = 1, nq = 0, first = 0;
 #pragma unroll
   for (int i = 0; i < kSplitSeqLanes; ++i)
@@ -2151,22 +2176,37 @@ static int *queue_for(hipStream_t st) {
 }
 
 // Items a key-split launch of `tiles` query tiles may have: one per compute
-// unit, or two where one round would leave units idle at its end (above 3/8
-// of the units in tiles).
-static int64_t split_items(int64_t tiles) { return device_cus() * static_cast<int64_t>(8 * tiles > 3 * device_cus() ? 2 : 1); }
-static int64_t split_ws_bytes() { return 2 * static_cast<int64_t>(device_cus()) * kPartFloats * 4; }
+// unit, two where one round would leave units idle at its end (above 3/8 of
+// the units in tiles), or three where the tiles themselves take two rounds.
+static int64_t split_items(int64_t tiles) {
+  const int64_t cus = device_cus();
+  return cus * (tiles > cus ? 3 : (8 * tiles > 3 * cus ? 2 : 1));
+}
+constexpr int64_t kSplitHead = 256;  // the workspace's head
+static int64_t split_ws_bytes() { return kSplitHead + 3 * static_cast<int64_t>(device_cus()) * kPartFloats * 4; }
 
 // Query tiles of a launch that may split its keys, 0 for one that may not:
-// head_dim 128, at most kSplitMaxSeqs sequences and tiles on at most 9/10 of
+// head_dim 128, at most kSplitMaxSeqs sequences, and tiles on at most 9/10 of
 // the units (252 tiles of 256 units gain nothing: 416 us unsplit, 424-444
-// split), and keys for at least two chunks of the shortest length in the
-// longest sequence, whose estimate then beats the unsplit one (max_seqlen_k
-// bounds the keys of a sequence; 0 = unknown).
-static int64_t split_tiles(const pkv_attn_args *a, int64_t max_seqlen_k) {
-  const int64_t seqs = static_cast<int64_t>(a->num_batches) * a->num_heads_q;
+// split) or on up to three halves of them (504 tiles 824 us unsplit, 832-910
+// split).  `keys` is what a sequence is expected to have (0 = unknown): where
+// the estimates of split_plan would not split sequences of that length the
+// launch and its second kernel are saved.  With t tiles per unit and u units
+// of keys each these are, in turn, a chunk of the shortest length and the
+// fixed part (u > 6, as sequences differ), up to half of the units; the gain
+// of a second round (u >= 32, measured: 168 tiles of 36 units 113.5 us
+// unsplit, 112.5 split; of 116 units 353 and 290); and 2 u > 1.05 (t u + 3 t +
+// u / 4 + 12).
+static int64_t split_tiles(const pkv_attn_args *a, int64_t keys) {
+  const int64_t seqs = static_cast<int64_t>(a->num_batches) * a->num_heads_q, cus = device_cus();
   const int64_t tiles = seqs * ((static_cast<int64_t>(a->max_seqlen_q) + 32 * kWaves - 1) / (32 * kWaves));
-  const bool keys = max_seqlen_k <= 0 || max_seqlen_k > 32 * kSplitUnit * (kSplitMinUnits + kSplitFixedUnits);
-  return a->head_dim == 128 && seqs <= kSplitMaxSeqs && 10 * tiles <= 9 * device_cus() && keys ? tiles : 0;
+  if (a->head_dim != 128 || seqs > kSplitMaxSeqs || cus <= 0) return 0;
+  if (tiles > cus ? 2 * tiles > 3 * cus : 10 * tiles > 9 * cus) return 0;
+  if (keys > 0) {
+    const double u = static_cast<double>(keys) / (32 * kSplitUnit), t = static_cast<double>(tiles) / cus;
+    if (tiles > cus ? 2 * u <= 1.05 * (t * u + 3 * t + u / 4 + 12) : u <= (2 * tiles > cus ? 32 : 6)) return 0;
+  }
+  return tiles;
 }
 
 // Key-split launch: attn_pp_kernel<true> over as many workgroups as it may
@@ -2188,7 +2228,8 @@ static int launch_split(const pkv_attn_args *a, void *ws, int64_t ws_bytes, hipS
   p.kv_tok = a->kv_tok_stride; p.kv_head = a->kv_head_stride;
   p.o_tok = a->o_tok_stride; p.o_head = a->o_head_stride;
   p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
-  p.part = static_cast<float *>(ws);
+  p.head = static_cast<int *>(ws);
+  p.part = reinterpret_cast<float *>(static_cast<char *>(ws) + kSplitHead);
   hipLaunchKernelGGL(attn_pp_kernel<true>, dim3(p.n_wg), dim3(kThreads), 0, st, p);
   int rc = check_launch("attn_pp_kernel");
   if (rc) return rc;
@@ -2260,9 +2301,9 @@ static int attn_check(const pkv_attn_args *a) {
 
 extern "C" int64_t pkv_ragged_attn_workspace_size(void) { return split_ws_bytes(); }
 
-extern "C" int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *a, int64_t max_seqlen_k) {
+extern "C" int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *a, int64_t keys) {
   if (!a || a->num_batches <= 0 || a->num_heads_q <= 0 || a->max_seqlen_q <= 0) return 0;
-  return split_tiles(a, max_seqlen_k) ? split_ws_bytes() : 0;
+  return split_tiles(a, keys) ? split_ws_bytes() : 0;
 }
 
 extern "C" int pkv_ragged_attn_fwd_ws(const pkv_attn_args *a, void *workspace, int64_t workspace_bytes,

@@ -661,8 +661,8 @@ static int64_t mega_evict_merge_workspace_size(int64_t num_heads) {
 // [total_k, D] (or [total_k, 1, D]) and cu_seqlens_k has num_batches*Hq+1
 // entries (sequence b*Hq+h); otherwise k/v are [total_k, Hq, D] with
 // cu_seqlens_k [num_batches+1].  max_seqlen_k bounds a sequence's keys (0 =
-// unknown): it only helps to tell which launches may gain from splitting
-// their keys.  Returns the output shaped like q.
+// unknown): with k's rows it tells which launches may gain from splitting
+// their keys, nothing else.  Returns the output shaped like q.
 static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q, Tensor cu_seqlens_k,
                                int64_t max_seqlen_q, double softmax_scale, bool kv_per_head, bool causal,
                                c10::optional<Tensor> workspace, int64_t max_seqlen_k) {
@@ -721,9 +721,9 @@ static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q
     return out;
   }
   // a workspace of the stream's allocator for the launches that gain from one
-  // (no sequence has more keys than k has rows)
-  const int64_t rows = k.size(0);
-  const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 && max_seqlen_k < rows ? max_seqlen_k : rows);
+  // (k's rows are those of the sequences, or a buffer's that holds them)
+  const int64_t mean = k.size(0) / std::max<int64_t>(1, kv_per_head ? B * Hq : B);
+  const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 && max_seqlen_k < mean ? max_seqlen_k : mean);
   if (need > 0) {
     const Tensor w = at::empty({need}, q.options().dtype(at::kByte));
     pkv_check(pkv_ragged_attn_fwd_ws(&a, w.data_ptr(), need, stream_for(q)), "ragged_attention");

@@ -141,8 +141,10 @@ def test_split_through_the_torch_op_on_strided_views():
 @pytest.mark.parametrize("Lq,Lk,H,kv_per_head", [
     # two rounds of items: 108 tiles, above 3/8 of the compute units
     ([1300, 1300], [[3000 + 251 * h for h in range(9)]] * 2, 9, True),
+    # three rounds: 290 tiles, more than there are compute units
+    ([290] * 29, [[4200 + (s * 37 + h * 211) % 1500 for h in range(5)] for s in range(29)], 5, True),
     # more than 64 sequences, several per lane of the plan, some without rows or keys
-    ([10, 0, 33] * 24, [[(s * 613 + h * 97) % 2600 for h in range(3)] for s in range(72)], 3, True),
+    ([10, 0, 33] * 13, [[(s * 613 + h * 97) % 2600 for h in range(3)] for s in range(39)], 3, True),
     # the edges of a chunk: one key more and fewer than the shortest two, and a
     # single row over a long sequence
     ([1], [[1023, 1024, 1025, 1151, 20000]], 5, True),
