@@ -25,7 +25,25 @@ __device__ inline float wave_sum(float x) {
   return x;
 }
 
+// f32 pair -> bf16x2 by the hardware round-to-nearest-even conversion (NaN
+// halves to 0x7fc0, as pack_bf16x2)
+__device__ inline uint32_t cvt_bf16x2(float lo, float hi) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  if ((u & 0x7fffu) > 0x7f80u) u = (u & 0xffff0000u) | 0x7fc0u;
+  if ((u & 0x7fff0000u) > 0x7f800000u) u = (u & 0xffffu) | 0x7fc00000u;
+  return u;
+}
+
 __device__ inline float4 ld_f4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+
+// 16 bytes at any 4-byte boundary (gfx950 loads need no more)
+__device__ inline float4 ld_f4u(const float *p) {
+  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  const f4u v = *reinterpret_cast<const f4u *>(p);
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
 
 // a + float(b) * gate[4j..4j+3] with one rounding per element (fma), or
 // a + float(b) without a gate: the residual update of 4 columns, shared by
@@ -44,8 +62,15 @@ __device__ inline float4 residual4(float4 a, uint2 b, const float *gate, int j) 
 // out[r, :] = bf16(LN(x[r, :]) * m + a), LN without affine weights; m =
 // (one_plus ? 1 + mul : mul) and a = add, each optional (1 and 0).  kRes
 // first applies the residual update x[r, :] += float(y[r, :]) * gate in
-// registers and writes the updated row back, so the row is read once.
-template <int K, bool kRes>
+// registers and writes the updated row back, so the row is read once.  K
+// vectors of 4 values per lane, guarded unless kFull (the row is exactly K * 64
+// vectors long).  Bound by memory, and, since a launch of a few thousand rows
+// has all of its waves resident at once, by the chain of reads and sums of one
+// row: K fits the row (6 vectors at 1,536 columns), the row's y is read with
+// it, and the weights are read between the two sums.  4,680 rows of 1,536:
+// 14.9 us with the residual update (86 MB, 5.8 TB/s) and 9.3 us without,
+// against 17.2 and 11.4 with 8 guarded vectors and the weights read last.
+template <int K, bool kRes, bool kFull>
 __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x, int64_t rows, int C,
                                                                        const float *mul, const float *add,
                                                                        int one_plus, float eps, uint16_t *out,
@@ -57,23 +82,42 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
   float *xr = x + r * C;
   const int nv = C / 4;
   float4 v[K];
+  uint2 yv[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int j = lane + 64 * k;
+    const bool in = kFull || j < nv;
+    v[k] = in ? ld_f4(xr + 4 * j) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (kRes && in) yv[k] = *reinterpret_cast<const uint2 *>(y + r * y_stride + 4 * j);
+  }
   float s = 0.0f;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    v[k] = j < nv ? ld_f4(xr + 4 * j) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (kRes && j < nv) {
-      v[k] = residual4(v[k], *reinterpret_cast<const uint2 *>(y + r * y_stride + 4 * j), gate, j);
+    if (kRes && (kFull || j < nv)) {
+      v[k] = residual4(v[k], yv[k], gate, j);
       *reinterpret_cast<float4 *>(xr + 4 * j) = v[k];
     }
     s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
   }
   const float mean = wave_sum(s) / static_cast<float>(C);
+  // the weights are on their way while the second sum is taken (rows of more
+  // vectors have no registers left for them)
+  constexpr bool kEarly = K <= 6;
+  float4 mv[kEarly ? K : 1], av[kEarly ? K : 1];
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int j = kFull ? lane + 64 * k : min(lane + 64 * k, nv - 1);
+      if (mul) mv[k] = ld_f4(mul + 4 * j);
+      if (add) av[k] = ld_f4(add + 4 * j);
+    }
+  }
   float q = 0.0f;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    if (j < nv) {
+    if (kFull || j < nv) {
       const float a = v[k].x - mean, b = v[k].y - mean, c = v[k].z - mean, d = v[k].w - mean;
       q += (a * a + b * b) + (c * c + d * d);
     }
@@ -83,27 +127,34 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    if (j >= nv) continue;
+    if (!kFull && j >= nv) continue;
     float y[4] = {(v[k].x - mean) * rstd, (v[k].y - mean) * rstd, (v[k].z - mean) * rstd, (v[k].w - mean) * rstd};
     if (mul) {
-      const float4 m = ld_f4(mul + 4 * j);
+      const float4 m = kEarly ? mv[kEarly ? k : 0] : ld_f4(mul + 4 * j);
       const float mm[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] *= one_plus ? 1.0f + mm[e] : mm[e];
     }
     if (add) {
-      const float4 a = ld_f4(add + 4 * j);
+      const float4 a = kEarly ? av[kEarly ? k : 0] : ld_f4(add + 4 * j);
       y[0] += a.x;
       y[1] += a.y;
       y[2] += a.z;
       y[3] += a.w;
     }
-    *reinterpret_cast<uint2 *>(orow + 4 * j) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+    *reinterpret_cast<uint2 *>(orow + 4 * j) = make_uint2(cvt_bf16x2(y[0], y[1]), cvt_bf16x2(y[2], y[3]));
   }
 }
 
-// out[r, :] = bf16(x * rsqrt(mean(x^2) + eps) * w) in fp32, x bf16
-template <int K>
+// out[r, :] = bf16(x * rsqrt(mean(x^2) + eps) * w) in fp32, x bf16.  K
+// vectors of 8 values per lane, the last one guarded unless kFull (the row is
+// exactly K * 64 vectors long).  Bound by latency more than by memory: at
+// 4,680 rows of 1,536 every wave of the launch is resident at once, so its time
+// is one chain of read, wave sum, store.  The weights are therefore read with
+// the row, not after its sum, and K fits the row: 6.9 us (4.2 TB/s) for 4,680
+// rows of 1,536 out of rows of 4,608, 8.4 us with 4 guarded vectors and the
+// weights read last.
+template <int K, bool kFull>
 __global__ void __launch_bounds__(64 * kDitRowsPerBlock) rms_kernel(const uint16_t *x, int64_t x_stride, int64_t rows,
                                                                     int C, const float *w, float eps,
                                                                     uint16_t *out, int64_t out_stride) {
@@ -113,11 +164,27 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) rms_kernel(const uint16
   const uint16_t *xr = x + r * x_stride;
   const int nv = C / 8;
   uint4 v[K];
-  float s = 0.0f;
+  constexpr bool kEarly = K <= 4;  // (longer rows have no registers left for the weights)
+  float4 g[kEarly ? K : 1][2];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    v[k] = j < nv ? *reinterpret_cast<const uint4 *>(xr + 8 * j) : make_uint4(0, 0, 0, 0);
+    v[k] = kFull || j < nv ? *reinterpret_cast<const uint4 *>(xr + 8 * j) : make_uint4(0, 0, 0, 0);
+  }
+  auto weights = [&](int j, float4 (&to)[2]) {
+    to[0] = to[1] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    if (w && (kFull || j < nv)) {
+      to[0] = ld_f4u(w + 8 * j);
+      to[1] = ld_f4u(w + 8 * j + 4);
+    }
+  };
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) weights(lane + 64 * k, g[k]);
+  }
+  float s = 0.0f;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
     const uint32_t wd[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -131,18 +198,21 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) rms_kernel(const uint16
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    if (j >= nv) continue;
+    if (!kFull && j >= nv) continue;
     const uint32_t wd[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+    float4 (&gk)[2] = g[kEarly ? k : 0];
+    if constexpr (!kEarly) weights(j, gk);
+    const float gg[8] = {gk[0].x, gk[0].y, gk[0].z, gk[0].w, gk[1].x, gk[1].y, gk[1].z, gk[1].w};
     uint32_t o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float a = bf16_to_f32(static_cast<uint16_t>(wd[e] & 0xffff)) * rn;
       float b = bf16_to_f32(static_cast<uint16_t>(wd[e] >> 16)) * rn;
       if (w) {
-        a *= w[8 * j + 2 * e];
-        b *= w[8 * j + 2 * e + 1];
+        a *= gg[2 * e];
+        b *= gg[2 * e + 1];
       }
-      o[e] = pack_bf16x2(a, b);
+      o[e] = cvt_bf16x2(a, b);
     }
     *reinterpret_cast<uint4 *>(orow + 8 * j) = make_uint4(o[0], o[1], o[2], o[3]);
   }
@@ -175,17 +245,6 @@ __device__ inline float gelu_tanh_f32(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
 }
 
-// f32 pair -> bf16x2 by the hardware round-to-nearest-even conversion (NaN
-// halves to 0x7fc0, as pack_bf16x2)
-__device__ inline uint32_t cvt_bf16x2(float lo, float hi) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  const bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-  uint32_t u = __builtin_bit_cast(uint32_t, v);
-  if ((u & 0x7fffu) > 0x7f80u) u = (u & 0xffff0000u) | 0x7fc0u;
-  if ((u & 0x7fff0000u) > 0x7f800000u) u = (u & 0xffffu) | 0x7fc00000u;
-  return u;
-}
-
 __global__ void __launch_bounds__(256) gelu_tanh_kernel(const uint16_t *x, int64_t n8, uint16_t *out) {
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n8;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
@@ -209,18 +268,17 @@ static int launch_ln_k(float *x, int64_t rows, int cols, const float *mul, const
                        float eps, uint16_t *out, const uint16_t *y, int64_t y_stride, const float *gate, hipStream_t st,
                        const char *who) {
   const int vec = (cols / 4 + 63) / 64;
-  const dim3 grid(row_grid(rows)), block(64 * kDitRowsPerBlock);
-  if (vec <= 4)
-    hipLaunchKernelGGL((ln_mod_kernel<4, kRes>), grid, block, 0, st, x, rows, cols, mul, add, mul_plus_one, eps, out, y,
-                       y_stride, gate);
-  else if (vec <= 8)
-    hipLaunchKernelGGL((ln_mod_kernel<8, kRes>), grid, block, 0, st, x, rows, cols, mul, add, mul_plus_one, eps, out, y,
-                       y_stride, gate);
-  else if (vec <= kMaxVec)
-    hipLaunchKernelGGL((ln_mod_kernel<kMaxVec, kRes>), grid, block, 0, st, x, rows, cols, mul, add, mul_plus_one, eps,
-                       out, y, y_stride, gate);
-  else
-    return fail(PKV_ERR_UNSUPPORTED, "%s: cols (%d) above %d", who, cols, 64 * 4 * kMaxVec);
+  if (vec > kMaxVec) return fail(PKV_ERR_UNSUPPORTED, "%s: cols (%d) above %d", who, cols, 64 * 4 * kMaxVec);
+  const bool full = cols % 256 == 0;
+  auto *k = vec <= 2              ? ln_mod_kernel<2, kRes, false>
+            : vec <= 4            ? ln_mod_kernel<4, kRes, false>
+            : vec == 6 && full    ? ln_mod_kernel<6, kRes, true>
+            : vec <= 6            ? ln_mod_kernel<6, kRes, false>
+            : vec <= 8            ? ln_mod_kernel<8, kRes, false>
+            : vec <= 12           ? ln_mod_kernel<12, kRes, false>
+                                  : ln_mod_kernel<kMaxVec, kRes, false>;
+  hipLaunchKernelGGL(k, dim3(row_grid(rows)), dim3(64 * kDitRowsPerBlock), 0, st, x, rows, cols, mul, add, mul_plus_one,
+                     eps, out, y, y_stride, gate);
   return check_launch("ln_mod_kernel");
 }
 
@@ -279,15 +337,16 @@ extern "C" int pkv_dit_rms_norm(const uint16_t *x, int64_t x_row_stride, int64_t
     return fail(PKV_ERR_INVALID, "dit_rms_norm: cols and row strides must be multiples of 8 (cols %d)", cols);
   if (rows > 0x7fffffffLL * kDitRowsPerBlock) return fail(PKV_ERR_UNSUPPORTED, "dit_rms_norm: too many rows");
   const int vec = (cols / 8 + 63) / 64;
-  hipStream_t st = as_stream(stream);
-  const dim3 grid(row_grid(rows)), block(64 * kDitRowsPerBlock);
-  if (vec <= 4)
-    hipLaunchKernelGGL(rms_kernel<4>, grid, block, 0, st, x, x_row_stride, rows, cols, weight, eps, out, out_row_stride);
-  else if (vec <= kMaxVec)
-    hipLaunchKernelGGL(rms_kernel<kMaxVec>, grid, block, 0, st, x, x_row_stride, rows, cols, weight, eps, out,
-                       out_row_stride);
-  else
-    return fail(PKV_ERR_UNSUPPORTED, "dit_rms_norm: cols (%d) above %d", cols, 64 * 8 * kMaxVec);
+  if (vec > kMaxVec) return fail(PKV_ERR_UNSUPPORTED, "dit_rms_norm: cols (%d) above %d", cols, 64 * 8 * kMaxVec);
+  const bool full = cols % 512 == 0;
+  auto *k = vec == 1   ? (full ? rms_kernel<1, true> : rms_kernel<1, false>)
+            : vec == 2 ? (full ? rms_kernel<2, true> : rms_kernel<2, false>)
+            : vec == 3 ? (full ? rms_kernel<3, true> : rms_kernel<3, false>)
+            : vec == 4 ? (full ? rms_kernel<4, true> : rms_kernel<4, false>)
+            : vec <= 8 ? rms_kernel<8, false>
+                       : rms_kernel<kMaxVec, false>;
+  hipLaunchKernelGGL(k, dim3(row_grid(rows)), dim3(64 * kDitRowsPerBlock), 0, as_stream(stream), x, x_row_stride, rows,
+                     cols, weight, eps, out, out_row_stride);
   return check_launch("rms_kernel");
 }
 

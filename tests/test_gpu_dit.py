@@ -138,3 +138,33 @@ def test_dit_residual_layer_norm_equals_the_two_ops(rows, C, gated, one_plus):
     got = ops.dit_residual_layer_norm_(xb, y, gate, mul, add, one_plus, eps)
     assert torch.equal(xb, xa)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("C", [8, 256, 264, 512, 520, 768, 1024, 1032, 1280, 1536, 1544, 2048, 2056, 3072, 3080, 4096])
+def test_dit_norms_at_the_edges_of_their_widths(C):
+    """The norms hold a row in as many vectors per lane as it needs: widths at,
+    below and above the edges of each count, a weight that starts off a
+    16-byte line, one row and a partly filled workgroup, against float64."""
+    import torch.nn.functional as F
+    from pyramidkv import _ops
+    ops = _ops.ops()
+    g = torch.Generator(device=DEV)
+    g.manual_seed(C)
+    for rows in (1, 7):
+        x = torch.randn(rows, C, generator=g, device=DEV) * 2.0 + 1.0
+        mul, add, gate = (torch.randn(C, generator=g, device=DEV) * 0.1 for _ in range(3))
+        y = torch.randn(rows, C, generator=g, device=DEV).to(torch.bfloat16)
+        ln = F.layer_norm(x.double(), (C,), eps=1e-6)
+        _bf16_close(ops.dit_layer_norm(x, mul, add, True, 1e-6), ln * (1 + mul.double()) + add.double())
+        _bf16_close(ops.dit_layer_norm(x, mul, None, False, 1e-6), ln * mul.double())
+        _bf16_close(ops.dit_layer_norm(x, None, add, False, 1e-6), ln + add.double())
+        a, b = x.clone(), x.clone()
+        ops.dit_residual_(a, y, gate)
+        out = ops.dit_residual_layer_norm_(b, y, gate, mul, add, True, 1e-6)
+        assert torch.equal(a, b)
+        assert torch.equal(out.view(torch.int16), ops.dit_layer_norm(a, mul, add, True, 1e-6).view(torch.int16))
+        for w in (None, torch.rand(C, generator=g, device=DEV) + 0.5,
+                  (torch.rand(C + 1, generator=g, device=DEV) + 0.5)[1:]):
+            d = y.double()
+            want = d * torch.rsqrt(d.pow(2).mean(-1, keepdim=True) + 1e-6)
+            _bf16_close(ops.dit_rms_norm(y, w, 1e-6), want if w is None else want * w.double())
