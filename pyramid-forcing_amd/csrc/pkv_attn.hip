@@ -85,10 +85,10 @@ struct AttnParams {
   int Hq, kv_per_head, q_tiles, n_wg;
   int64_t q_tok, q_head, kv_tok, kv_head, o_tok, o_head;
   float scale_log2;
-  // key-split launches (attn_pp_kernel<true> + attn_combine_kernel): the
-  // items' partial results in the caller's workspace, and its head
+  // key-split launches (attn_pp_kernel<true> + attn_combine_kernel): in the
+  // caller's workspace the items' partial results and one entry per query tile
   float *part;
-  int *head;
+  int4 *head;
   int n_seq, n_cu;
   // queue launches of attn_p3_kernel (one workgroup per compute
   // unit, items claimed from per-XCD counters): this stream's counter
@@ -329,8 +329,9 @@ __device__ void queue_done(int *queue) {
 // bounds such a launch is its longest workgroup, not the chip: 42 tiles of
 // 3,000-8,000 keys took 163 us on 42 of 256 units, 49 us split over 219.
 //
-// Every wave of both launches computes the same plan from cu_q / cu_k in
-// registers (no LDS, no barrier; lane i holds sequences i, i + 64, ...).
+// Every wave of the first launch computes the same plan from cu_q / cu_k in
+// registers (no LDS, no barrier; lane i holds sequences i, i + 64, ...); the
+// workgroup of a tile's chunk 0 leaves where its chunks lie for the second.
 // Keys are counted in units of kSplitUnit tiles, the key loop's unroll.  With
 // at most R * n_cu items the chunk length C is the smallest that fits, at
 // least kSplitMinUnits; sequence s has k_s = ceil(units_s / C) chunks of equal
@@ -362,7 +363,7 @@ constexpr int kSplitFixedUnits = 4;
 
 struct SplitPlan {
   int nq[kSplitSeqLanes], nu[kSplitSeqLanes], k[kSplitSeqLanes], base[kSplitSeqLanes];
-  int n_items, tiles, chunk;
+  int n_items;
 };
 
 // One item: query tile qt of sequence seq (of nq tiles) against units
@@ -375,9 +376,7 @@ __device__ inline int div_up(int a, int b) {
   return static_cast<int>(static_cast<unsigned>(a + b - 1) / static_cast<unsigned>(b));
 }
 
-// chunk: the plan's C where it is known (attn_combine_kernel reads it from the
-// workspace's head), -1 to choose it.
-__device__ inline SplitPlan split_plan(const AttnParams &p, int chunk) {
+__device__ inline SplitPlan split_plan(const AttnParams &p) {
   SplitPlan s;
   const int lane = threadIdx.x & 63;
   auto wave_total = [](int x) { return __builtin_amdgcn_readlane(wave_incl_sum(x), 63); };
@@ -397,49 +396,46 @@ __device__ inline SplitPlan split_plan(const AttnParams &p, int chunk) {
     work += s.nq[i] * s.nu[i];
     longest = max(longest, s.nu[i]);
   }
-  int C = chunk;
-  if (chunk < 0) {
-    tiles = wave_total(tiles);
-    work = wave_total(work);
+  tiles = wave_total(tiles);
+  work = wave_total(work);
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
-    longest = __builtin_amdgcn_readfirstlane(longest);
-    auto items = [&](int C) {
-      int n = 0;
+  for (int off = 32; off >= 1; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  auto items = [&](int C) {
+    int n = 0;
 #pragma unroll
-      for (int i = 0; i < kSplitSeqLanes; ++i) n += s.nq[i] * (s.nu[i] <= C ? 1 : div_up(s.nu[i], C));
-      return wave_total(n);
-    };
-    // chunk lengths are tried in [work / G, work / (G - tiles)]: no shorter one
-    // can fit G items, and that one does (items <= work / C + tiles)
-    auto shortest = [&](int G) {
-      int lo = max(kSplitMinUnits, work / G), hi = max(lo, min(longest, div_up(work, max(1, G - tiles))));
-      while (lo < hi) {
-        const int C = (lo + hi) >> 1;
-        if (items(C) <= G) hi = C;
-        else lo = C + 1;
-      }
-      return lo;
-    };
-    const int mean = work / max(1, tiles);
-    C = max(1, longest);
-    int best = tiles <= p.n_cu ? longest : 2 * mean + (longest - mean) / 2;
-    if (tiles > p.n_cu) {
-      const int c3 = shortest(p.n_wg);
-      const int t = (work + kSplitItemUnits * (items(c3) - tiles)) / p.n_cu + c3 / 2 + 3 * kSplitFixedUnits;
-      if (t + t / 20 < best) C = c3;
+    for (int i = 0; i < kSplitSeqLanes; ++i) n += s.nq[i] * (s.nu[i] <= C ? 1 : div_up(s.nu[i], C));
+    return wave_total(n);
+  };
+  // chunk lengths are tried in [work / G, work / (G - tiles)]: no shorter one
+  // can fit G items, and that one does (items <= work / C + tiles)
+  auto shortest = [&](int G) {
+    int lo = max(kSplitMinUnits, work / G), hi = max(lo, min(longest, div_up(work, max(1, G - tiles))));
+    while (lo < hi) {
+      const int C = (lo + hi) >> 1;
+      if (items(C) <= G) hi = C;
+      else lo = C + 1;
     }
-    if (tiles < p.n_cu) {
-      const int c1 = shortest(p.n_cu);
-      if (c1 + kSplitFixedUnits < best) {
-        C = c1;
-        best = c1 + kSplitFixedUnits;
-      }
+    return lo;
+  };
+  const int mean = work / max(1, tiles);
+  int C = max(1, longest);
+  int best = tiles <= p.n_cu ? longest : 2 * mean + (longest - mean) / 2;
+  if (tiles > p.n_cu) {
+    const int c3 = shortest(p.n_wg);
+    const int t = (work + kSplitItemUnits * (items(c3) - tiles)) / p.n_cu + c3 / 2 + 3 * kSplitFixedUnits;
+    if (t + t / 20 < best) C = c3;
+  }
+  if (tiles < p.n_cu) {
+    const int c1 = shortest(p.n_cu);
+    if (c1 + kSplitFixedUnits < best) {
+      C = c1;
+      best = c1 + kSplitFixedUnits;
     }
-    if (tiles <= p.n_cu && p.n_wg >= 2 * p.n_cu) {
-      const int c2 = shortest(2 * p.n_cu);
-      if ((work + kSplitItemUnits * (items(c2) - tiles)) / p.n_cu + c2 / 3 + 2 * kSplitFixedUnits < best) C = c2;
-    }
+  }
+  if (tiles <= p.n_cu && p.n_wg >= 2 * p.n_cu) {
+    const int c2 = shortest(2 * p.n_cu);
+    if ((work + kSplitItemUnits * (items(c2) - tiles)) / p.n_cu + c2 / 3 + 2 * kSplitFixedUnits < best) C = c2;
   }
   int run = 0;
 #pragma unroll
@@ -450,8 +446,6 @@ __device__ inline SplitPlan split_plan(const AttnParams &p, int chunk) {
     run += __builtin_amdgcn_readlane(incl, 63);
   }
   s.n_items = run;
-  s.chunk = C;
-  s.tiles = tiles;
   return s;
 }
 
@@ -926,15 +920,14 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
   int slot_idx = 0;
   const int n_seq = p.n_wg / p.q_tiles;
   if constexpr (SPLIT) {
-    const SplitPlan plan = split_plan(p, -1);
-    // the workspace's head: the chunk length, 0 when no tile has two chunks
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-      *p.head = __builtin_amdgcn_readfirstlane(plan.tiles) == plan.n_items ? 0 : plan.chunk;
+    const SplitPlan plan = split_plan(p);
     if (static_cast<int>(blockIdx.x) >= plan.n_items) return;
     slot_idx = xcd_remap(blockIdx.x, plan.n_items);
     it = split_item(plan, slot_idx);
     seq = it.seq;
     qt = it.qt;
+    // for attn_combine_kernel: where the tile's chunks lie
+    if (it.j == 0 && threadIdx.x == 0) p.head[seq * p.q_tiles + qt] = make_int4(it.first, it.nq, it.k, 0);
   } else if (n_seq <= kSchedMax && p.n_wg > p.n_cu) {
     if (!balanced_item(p.cu_q, p.cu_k, p.Hq, n_seq, p.kv_per_head, 32 * kWaves, xcd_remap(blockIdx.x, p.n_wg),
                        sched, seq, qt))
@@ -2053,54 +2046,70 @@ __global__ void __launch_bounds__(kP3Threads, 1) attn_p3_kernel(AttnParams p) {
 // largest reference of the tile's chunks, O = sum_j 2^(r_j - M) O_j /
 // sum_j 2^(r_j - M) l_j in chunk order (fp32).  Tiles of one chunk, which
 // attn_pp_kernel wrote itself, exit at once.
+// What bounds it is one chain of reads, not the 132 KB per item: the tile's
+// entry, then the references, sums and O blocks of the first kCombineAhead
+// chunks together (219 items of 42 tiles: 8.8 us; with the plan computed again
+// and the references read before the O blocks 9.6).
 constexpr int kCombineWaves = 4;  // waves per workgroup: each takes one 32-dim block of the rows
+constexpr int kCombineAhead = 4;  // chunks whose O blocks are read at once
 __global__ void __launch_bounds__(64 * kCombineWaves) attn_combine_kernel(AttnParams p) {
   const int tile = blockIdx.x / kWaves, wave = blockIdx.x % kWaves;
   const int seq = tile / p.q_tiles, qt = tile % p.q_tiles;
   const int b = seq / p.Hq, h = seq % p.Hq;
+  const int4 e = p.head[tile];
   const int q_begin = p.cu_q[b];
   const int Lq = p.cu_q[b + 1] - q_begin;
   const int q0 = qt * 32 * kWaves;
+  // (a tile past its sequence's rows has no entry)
   if (q0 + wave * 32 >= Lq) return;
-  const int chunk = *(const __attribute__((address_space(4))) int *)p.head;
-  if (chunk == 0) return;
-  const SplitPlan s = split_plan(p, chunk);
-  int k = 1, nq = 0, first = 0;
-#pragma unroll
-  for (int i = 0; i < kSplitSeqLanes; ++i)
-    if (seq >> 6 == i) {
-      k = __builtin_amdgcn_readlane(s.k[i], seq & 63);
-      nq = __builtin_amdgcn_readlane(s.nq[i], seq & 63);
-      first = __builtin_amdgcn_readlane(s.base[i], seq & 63) + qt;
-    }
+  const int first = __builtin_amdgcn_readfirstlane(e.x), nq = __builtin_amdgcn_readfirstlane(e.y);
+  const int k = __builtin_amdgcn_readfirstlane(e.z);
   if (k <= 1) return;
   const int lane = threadIdx.x & 63, db = threadIdx.x >> 6;
   const int lq = lane & 31, hf = lane >> 5;
   const float *part = p.part + static_cast<int64_t>(first) * kPartFloats;
   const int64_t step = static_cast<int64_t>(nq) * kPartFloats;
-  const float2 *rl = reinterpret_cast<const float2 *>(part + kPartOFloats) + wave * 64 + lane;
-  const float4 *po = reinterpret_cast<const float4 *>(part) + (wave * 16 + 4 * db) * 64 + lane;
+  const float *rl = part + kPartOFloats + (wave * 64 + lane) * 2;
+  const float *po = part + ((wave * 16 + 4 * db) * 64 + lane) * 4;
+  auto stat = [&](int j) { return *reinterpret_cast<const float2 *>(rl + j * step); };
+  float2 st[kCombineAhead];
+  float4 ob[kCombineAhead][4];
+  auto read = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < kCombineAhead; ++i)
+      if (j0 + i < k) {  // uniform
+        st[i] = stat(j0 + i);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) ob[i][g] = reinterpret_cast<const float4 *>(po + (j0 + i) * step)[g * 64];
+      }
+  };
+  read(0);
   float M = -INFINITY;
 #pragma unroll 4
-  for (int j = 0; j < k; ++j) M = fmaxf(M, reinterpret_cast<const float2 *>(reinterpret_cast<const float *>(rl) + j * step)->x);
+  for (int j = kCombineAhead; j < k; ++j) M = fmaxf(M, stat(j).x);
+#pragma unroll
+  for (int i = 0; i < kCombineAhead; ++i)
+    if (i < k) M = fmaxf(M, st[i].x);
   float l = 0.0f;
   float4 acc[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) acc[g] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll 4
-  for (int j = 0; j < k; ++j) {
-    const float2 v2 = *reinterpret_cast<const float2 *>(reinterpret_cast<const float *>(rl) + j * step);
-    const float4 *pj = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(po) + j * step);
-    const float w = __builtin_amdgcn_exp2f(v2.x - M);
-    l = fmaf(w, v2.y, l);
+  for (int j0 = 0; j0 < k; j0 += kCombineAhead) {
+    if (j0 > 0) read(j0);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float4 v = pj[g * 64];
-      acc[g].x = fmaf(w, v.x, acc[g].x);
-      acc[g].y = fmaf(w, v.y, acc[g].y);
-      acc[g].z = fmaf(w, v.z, acc[g].z);
-      acc[g].w = fmaf(w, v.w, acc[g].w);
-    }
+    for (int i = 0; i < kCombineAhead; ++i)
+      if (j0 + i < k) {
+        const float w = __builtin_amdgcn_exp2f(st[i].x - M);
+        l = fmaf(w, st[i].y, l);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 v = ob[i][g];
+          acc[g].x = fmaf(w, v.x, acc[g].x);
+          acc[g].y = fmaf(w, v.y, acc[g].y);
+          acc[g].z = fmaf(w, v.z, acc[g].z);
+          acc[g].w = fmaf(w, v.w, acc[g].w);
+        }
+      }
   }
   const float lt = half_sum(l);
   const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
@@ -2182,8 +2191,12 @@ static int64_t split_items(int64_t tiles) {
   const int64_t cus = device_cus();
   return cus * (tiles > cus ? 3 : (8 * tiles > 3 * cus ? 2 : 1));
 }
-constexpr int64_t kSplitHead = 256;  // the workspace's head
-static int64_t split_ws_bytes() { return kSplitHead + 3 * static_cast<int64_t>(device_cus()) * kPartFloats * 4; }
+// The workspace: an entry per query tile (of which there are at most 3/2 per
+// unit), then the items' partial results.
+static int64_t split_head_bytes() { return 2 * static_cast<int64_t>(device_cus()) * static_cast<int64_t>(sizeof(int4)); }
+static int64_t split_ws_bytes() {
+  return split_head_bytes() + 3 * static_cast<int64_t>(device_cus()) * kPartFloats * 4;
+}
 
 // Query tiles of a launch that may split its keys, 0 for one that may not:
 // head_dim 128, at most kSplitMaxSeqs sequences, and tiles on at most 9/10 of
@@ -2228,8 +2241,8 @@ static int launch_split(const pkv_attn_args *a, void *ws, int64_t ws_bytes, hipS
   p.kv_tok = a->kv_tok_stride; p.kv_head = a->kv_head_stride;
   p.o_tok = a->o_tok_stride; p.o_head = a->o_head_stride;
   p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
-  p.head = static_cast<int *>(ws);
-  p.part = reinterpret_cast<float *>(static_cast<char *>(ws) + kSplitHead);
+  p.head = static_cast<int4 *>(ws);
+  p.part = reinterpret_cast<float *>(static_cast<char *>(ws) + split_head_bytes());
   hipLaunchKernelGGL(attn_pp_kernel<true>, dim3(p.n_wg), dim3(kThreads), 0, st, p);
   int rc = check_launch("attn_pp_kernel");
   if (rc) return rc;
