@@ -47,10 +47,9 @@ struct PairCtx {
   int64_t sync_t;
 };
 
-__device__ inline PairCtx pair_ctx(const PlanParams &p, const HeadState &s, const int64_t *vc_h, int c) {
+__device__ inline PairCtx pair_ctx(const HeadState &s, const int64_t *vc_h, int64_t t_c, int64_t sync_t) {
   PairCtx x;
-  const int64_t t_c = p.t[c];
-  x.sync_t = p.sync_t[c];
+  x.sync_t = sync_t;
   x.thresh = s.sink_capacity;
   const int n_sink_raw = static_cast<int>(vc_h[0]);
   x.n_sink = (x.thresh > 0 && x.thresh < n_sink_raw) ? x.thresh : n_sink_raw;
@@ -162,7 +161,7 @@ __device__ int32_t emit_pair(const PlanParams &p, const HeadState &s, const int6
   const int lane = threadIdx.x & 63;
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   const int S = p.S;
-  const PairCtx x = pair_ctx(p, s, vc_h, c);
+  const PairCtx x = pair_ctx(s, vc_h, p.t[c], p.sync_t[c]);
   const int n_cand = p.max_sink + p.max_recent + kMaxTKeyed + kMaxMergeBlocks;
   int fp = 0;
   int32_t run = 0;
@@ -187,7 +186,11 @@ __device__ int32_t emit_pair(const PlanParams &p, const HeadState &s, const int6
 //  - One-pass form (at most 64 candidates and segments per pair, at most 64
 //    pairs): each wave evaluates the candidates of up to kPlanRegRounds pairs
 //    once and keeps them in registers; one barrier publishes the pair totals,
-//    every wave scans those 64 values itself and writes its segments.
+//    every wave scans those 64 values itself and writes its segments.  A
+//    chain of round trips bounds it (one workgroup, 9.2 us for 36 pairs with
+//    the list): the chunks' times are read with the records, not pair by pair,
+//    and every global store comes after the last barrier, which would wait for
+//    it (8.7 us so).
 //  - General form: a count-only pass gives every pair its token total, a
 //    block-wide exclusive scan turns those into offsets, and a second pass
 //    re-evaluates each pair's segments and writes them.
@@ -226,6 +229,15 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
   __shared__ int32_t s_waves[kPlanThreads / 64];
   const int tid = threadIdx.x;
   const int pairs = p.C * p.H;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), n_waves = blockDim.x >> 6, lane = tid & 63;
+  // the times of this wave's pairs, for the one-pass form
+  int64_t pt[kPlanRegRounds], psync[kPlanRegRounds];
+#pragma unroll
+  for (int r = 0; r < kPlanRegRounds; ++r) {
+    const int c = min(wave + r * n_waves, pairs - 1) / p.H;
+    pt[r] = p.t[c];
+    psync[r] = p.sync_t[c];
+  }
   const bool staged = p.H <= kPlanStageHeads && p.MMB <= kMaxMergeBlocks;
   if (staged) {
     // every read is issued before the LDS writes (one memory round trip for
@@ -256,7 +268,6 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
   const HeadState *st = staged ? s_states : states;
   const int64_t *vcs = staged ? s_vc : vc;
   const int32_t *mts = staged ? s_mtc : mtc;
-  const int wave = tid >> 6, n_waves = blockDim.x >> 6, lane = tid & 63;
   const int n_cand = p.max_sink + p.max_recent + kMaxTKeyed + kMaxMergeBlocks;
   // (the one-pass form reads the staged copies by their LDS arrays, so that
   // the compiler issues LDS reads rather than generic ones)
@@ -271,8 +282,8 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
       emit[r] = false;
       pos[r] = excl[r] = nv[r] = 0;
       if (q < pairs) {  // uniform over the wave
-        const int c = q / p.H, h = q % p.H;
-        const PairCtx x = pair_ctx(p, s_states[h], s_vc + h * 3, c);
+        const int h = q % p.H;
+        const PairCtx x = pair_ctx(s_states[h], s_vc + h * 3, pt[r], psync[r]);
         cd[r] = eval_cand(p, s_states[h], s_mtc + h * p.MMB, x, h, lane);
         const uint64_t mask = __ballot(cd[r].valid);
         pos[r] = __popcll(mask & below);
@@ -288,29 +299,38 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
     const int32_t v = lane < pairs ? len[lane] : 0;
     const int32_t incl = wave_incl_sum(v);  // lane q: end offset of pair q
     const int32_t total = __shfl(incl, 63);
-    if (tid == 0) {
-      o.cu_seqlens_k[0] = 0;
-      if (total_out) *total_out = total;
+    auto write_plan = [&]() {
+      if (tid == 0) {
+        o.cu_seqlens_k[0] = 0;
+        if (total_out) *total_out = total;
+      }
+#pragma unroll
+      for (int r = 0; r < kPlanRegRounds; ++r) {
+        const int q = wave + r * n_waves;
+        if (q >= pairs) continue;  // uniform over the wave
+        const int i0 = q * p.S;
+        const int32_t end = __builtin_amdgcn_readlane(incl, q), base = end - __builtin_amdgcn_readlane(v, q);
+        if (emit[r]) put_seg(o, i0 + pos[r], cd[r], base + excl[r]);
+        if (lane >= nv[r] && lane < p.S) put_inactive(o, i0 + lane);
+        if (lane == 0) o.cu_seqlens_k[q + 1] = end;
+      }
+    };
+    if (!list) {
+      write_plan();
+      return;
     }
 #pragma unroll
     for (int r = 0; r < kPlanRegRounds; ++r) {
       const int q = wave + r * n_waves;
       if (q >= pairs) continue;  // uniform over the wave
-      const int32_t end = __shfl(incl, q);
-      const int32_t base = __shfl(incl - v, q);
       const int i0 = q * p.S;
-      if (emit[r]) put_seg(o, i0 + pos[r], cd[r], base + excl[r]);
-      if (lane >= nv[r] && lane < p.S) put_inactive(o, i0 + lane);
-      if (lane == 0) o.cu_seqlens_k[q + 1] = end;
-      if (list) {
-        if (emit[r]) {
-          s_seg[i0 + pos[r]] = make_int4(cd[r].kind, cd[r].sg, cd[r].len, base + excl[r]);
-          s_tr[i0 + pos[r]] = remap32(cd[r].tremap);
-        }
-        if (lane >= nv[r] && lane < p.S) s_seg[i0 + lane] = make_int4(PKV_SEG_INACTIVE, 0, 0, 0);
+      const int32_t base = __builtin_amdgcn_readlane(incl - v, q);
+      if (emit[r]) {
+        s_seg[i0 + pos[r]] = make_int4(cd[r].kind, cd[r].sg, cd[r].len, base + excl[r]);
+        s_tr[i0 + pos[r]] = remap32(cd[r].tremap);
       }
+      if (lane >= nv[r] && lane < p.S) s_seg[i0 + lane] = make_int4(PKV_SEG_INACTIVE, 0, 0, 0);
     }
-    if (!list) return;
     // the pack's list: a thread per place of kPackShare chunks' lists finds
     // the distinct segments there (at most kPackShare); a block-wide scan of
     // the counts numbers them
@@ -333,12 +353,9 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
     const int incl_n = wave_incl_sum(n_ent);
     if (lane == 63) s_waves[wave] = incl_n;
     __syncthreads();
-    int at = incl_n - n_ent, all = 0;
-    for (int w = 0; w < n_waves; ++w) {
-      if (w < wave) at += s_waves[w];
-      all += s_waves[w];
-    }
-    if (tid == 0) *reinterpret_cast<int32_t *>(list) = all;
+    const int wn = lane < n_waves ? s_waves[lane] : 0, incl_w = wave_incl_sum(wn);
+    const int at = incl_n - n_ent + __builtin_amdgcn_readlane(incl_w - wn, wave);
+    if (tid == 0) *reinterpret_cast<int32_t *>(list) = __builtin_amdgcn_readlane(incl_w, 63);
     PackEntry *ent = reinterpret_cast<PackEntry *>(list + kPackListHead) + at;
 #pragma unroll
     for (int u = 0; u < kPackShare; ++u) {
@@ -365,6 +382,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanParams p, const 
       out[2] = tr;
       ++ent;
     }
+    write_plan();
     return;
   }
   for (int q = wave; q < pairs; q += n_waves) {
