@@ -1224,6 +1224,9 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
     wait_vm<0>();  // no copy may land in LDS after the workgroup ends
     // every tile's sums were rebased below 2^kHeadroom (or flagged)
     ovf = ovf || !(l < exp2f(kHeadroom));
+    // a chunk whose first tile scores -inf in a row has no reference for it,
+    // while the row's other chunks may hold finite scores
+    if constexpr (SPLIT) ovf = ovf || (wave_rows && m == -INFINITY);
     if (ovf) ovf_any = 1;
     __syncthreads();
     if (ovf_any) {
@@ -1255,7 +1258,8 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
           bf16x8 pq[2];
-          l = l * alpha + probs(s, m, pq);
+          // (such keys weigh nothing: 0, not 2^(inf - inf))
+          l = l * alpha + probs(s, SPLIT && m == -INFINITY ? 0.0f : m, pq);
           gemm1(pq);
         }
         __syncthreads();

@@ -170,3 +170,15 @@ def test_split_by_the_op_vs_float64(Lq, Lk, H, kv_per_head):
     want = O.ragged_attention_ref(O.bf16_to_f32(q), O.bf16_to_f32(k), O.bf16_to_f32(v), cu_q, cu_k, H, kv_per_head)
     err = np.abs(got - want)
     assert err.max() < 2e-2 and err.mean() < 2e-3, (err.max(), err.mean())
+
+
+def test_split_chunks_of_keys_whose_scores_are_minus_infinity():
+    """Keys whose score is -inf weigh nothing, also where they are the first
+    tile of a chunk, or all of it, and other chunks have finite scores."""
+    rng = np.random.default_rng(53)
+    q, k, v, cu_q, cu_k = _case(rng, [300], [[9000, 7000]], 2)
+    q[..., 0] = O.f32_to_bf16(np.ones(q.shape[:-1], np.float32))
+    k[cu_k[0] + 500:cu_k[0] + 6000, 0] = 0xFF80  # -inf
+    k[cu_k[1] + 700:cu_k[1] + 7000, 0] = 0xFF80
+    got = _run(q, k, v, cu_q, cu_k, 1, 2, _ws())
+    _check(got, q, k, v, cu_q, cu_k, 2)
