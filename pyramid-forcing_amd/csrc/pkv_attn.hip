@@ -1226,7 +1226,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
     ovf = ovf || !(l < exp2f(kHeadroom));
     // a chunk whose first tile scores -inf in a row has no reference for it,
     // while the row's other chunks may hold finite scores
-    if constexpr (SPLIT) ovf = ovf || (wave_rows && m == -INFINITY);
+    if constexpr (SPLIT) ovf = ovf || (it.k > 1 && wave_rows && m == -INFINITY);
     if (ovf) ovf_any = 1;
     __syncthreads();
     if (ovf_any) {
@@ -1258,8 +1258,9 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
           bf16x8 pq[2];
-          // (such keys weigh nothing: 0, not 2^(inf - inf))
-          l = l * alpha + probs(s, SPLIT && m == -INFINITY ? 0.0f : m, pq);
+          // (in a chunk such keys weigh nothing: 0, not 2^(inf - inf); a row
+          // that has all of its keys here is NaN, as unsplit)
+          l = l * alpha + probs(s, SPLIT && it.k > 1 && m == -INFINITY ? 0.0f : m, pq);
           gemm1(pq);
         }
         __syncthreads();

@@ -182,3 +182,16 @@ def test_split_chunks_of_keys_whose_scores_are_minus_infinity():
     k[cu_k[1] + 700:cu_k[1] + 7000, 0] = 0xFF80
     got = _run(q, k, v, cu_q, cu_k, 1, 2, _ws())
     _check(got, q, k, v, cu_q, cu_k, 2)
+
+
+def test_split_rows_whose_scores_are_all_minus_infinity():
+    """A row without a finite score is NaN, as 0 / 0 and in the unsplit
+    kernels, whether its sequence is one chunk of the launch or many; the
+    other sequences are not touched by it."""
+    rng = np.random.default_rng(59)
+    q, k, v, cu_q, cu_k = _case(rng, [300], [[9000, 400, 5000]], 3)
+    q[..., 0] = O.f32_to_bf16(np.ones(q.shape[:-1], np.float32))
+    k[:cu_k[2], 0] = 0xFF80  # -inf
+    for ws in (None, _ws()):
+        got = O.bf16_to_f32(_run(q, k, v, cu_q, cu_k, 1, 3, ws))
+        assert np.isnan(got[:, :2]).all() and np.isfinite(got[:, 2]).all()
