@@ -66,7 +66,6 @@ class MegaCacheCtx:
     # per layer: any Veil (merge) head; layers without one skip the merge launches
     layer_has_merge: list = field(default_factory=list)
     layer_merge_heads: list = field(default_factory=list)  # per layer: bit h set for each Veil head h
-    layer_max_keys: list = field(default_factory=list)  # per layer: the most tokens a head's segments can hold
     sink_caps_per_head: torch.Tensor = None
     committed_vc: torch.Tensor = None
     freqs: torch.Tensor = None
@@ -82,6 +81,7 @@ class MegaCacheCtx:
     # allocator's; with this switch in the device's (_ops.attention_workspace)
     split_attention: bool = False
     attn_workspace: torch.Tensor = None
+    layer_max_keys: list = field(default_factory=list)  # per layer: the most tokens a head's segments can hold
 
 
 class MegaCache:
