@@ -423,6 +423,13 @@ int pkv_evict_merge(uint8_t *states, int32_t num_heads, int32_t frames, int32_t 
                     const int64_t *t_vals, const uint16_t *new_k, const uint16_t *new_v, int32_t spatial_width,
                     const float *frame_weights, const pkv_state_desc *desc, const pkv_merge_layer *ml,
                     void *workspace, pkv_stream_t stream);
+/* The patch grid that the merges of a frame of frame_seqlen tokens in rows of
+ * width walk (patches of patch x patch tokens; the last row may be short), by
+ * the kernels' own arithmetic on the host.  Returns the group count (0: no
+ * grid).  read and has (NULL or patch * patch entries per group): the token
+ * that a merge reads for each member place of a group, always one of the
+ * frame's, and whether the patch has that member (others are not added). */
+int32_t pkv_patch_grid(int32_t frame_seqlen, int32_t width, int32_t patch, int32_t *read, uint8_t *has);
 /* Workspace bytes pkv_evict_merge needs for num_heads heads. */
 int64_t pkv_evict_merge_workspace_size(int32_t num_heads);
 

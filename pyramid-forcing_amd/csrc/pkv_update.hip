@@ -923,10 +923,18 @@ __host__ __device__ inline int grid_groups(int FSEQ, int W, int p) {
   return ((FSEQ - 1) / W / p + 1) * grid_columns(FSEQ, W, p);
 }
 // first member of group g of the grid with `cols` columns
-__device__ inline int grid_first(int g, int W, int p, int cols) { return (g / cols) * p * W + (g % cols) * p; }
-__device__ inline bool grid_has(int g, int m, int FSEQ, int W, int p, int cols) {
+__host__ __device__ inline int grid_first(int g, int W, int p, int cols) { return (g / cols) * p * W + (g % cols) * p; }
+__host__ __device__ inline bool grid_has(int g, int m, int FSEQ, int W, int p, int cols) {
   const int x = (g % cols) * p + m % p;
   return x < W && ((g / cols) * p + m / p) * W + x < FSEQ;
+}
+// token that is read for member m of group g where the read does not wait for
+// the test whether the patch has it: the member, or a token of the frame that
+// is then not added (where a short last row opens a patch row, the groups past
+// its end have no member at all, and even their first token lies past the frame)
+__host__ __device__ inline int grid_read(int g, int m, int FSEQ, int W, int p, int cols) {
+  const int t = grid_first(g, W, p, cols) + (m / p) * W + m % p;
+  return t < FSEQ ? t : FSEQ - 1;
 }
 
 // group of token t on the arithmetic grid (y = t / W, x = t % W) in patches
@@ -1020,8 +1028,8 @@ __host__ __device__ inline int64_t merge_lds_words(int FSEQ, int MMA) {
 // Patch chunks of a merge tile's groups in every frame of a call, loaded
 // before the record is staged and the state machine run: the members of a
 // group on the grid of width W = min(spatial width, FSEQ) depend on nothing
-// else (members that an edge patch lacks load the group's first token, and
-// are not added).  merge_prefetch returns W, or 0 when the call does not
+// else (for members that an edge patch lacks another token of the frame is
+// loaded, grid_read, and not added).  merge_prefetch returns W, or 0 when the call does not
 // qualify (then nothing is loaded); frames whose lists turn out otherwise
 // load their members themselves.
 constexpr int kPreFrames = 3;
@@ -1055,11 +1063,9 @@ __device__ __forceinline__ int merge_prefetch(const UpdArgs &a, int h, int mt, M
   if (ln.own && ln.g < grid_groups(FSEQ, W, p)) {
     const uint16_t *src = ln.is_v ? a.src.v : a.src.k;
     const int gcols = grid_columns(FSEQ, W, p);
-    const int gbase = grid_first(ln.g, W, p, gcols);
     uint32_t off[kPreTok];
 #pragma unroll
-    for (int m = 0; m < kPreTok; ++m)
-      off[m] = (gbase + (grid_has(ln.g, m, FSEQ, W, p, gcols) ? (m / p) * W + m % p : 0)) * a.src_tb;
+    for (int m = 0; m < kPreTok; ++m) off[m] = grid_read(ln.g, m, FSEQ, W, p, gcols) * a.src_tb;
 #pragma unroll
     for (int f = 0; f < kPreFrames; ++f)
 #pragma unroll
@@ -2741,6 +2747,17 @@ int pkv_cache_update(const pkv_geometry *geo, const pkv_pools *pools, const pkv_
   hipLaunchKernelGGL(update_kernel, dim3(u.n_mh * u.n_merge + H * u.n_scat), dim3(kUpdThreads), smem, as_stream(stream),
                      u);
   return check_launch("update_kernel");
+}
+
+int32_t pkv_patch_grid(int32_t FSEQ, int32_t width, int32_t patch, int32_t *read, uint8_t *has) {
+  if (FSEQ <= 0 || FSEQ > kMaxMergeFseq || width <= 0 || patch <= 0 || patch > std::max(kPrePatch, FSEQ)) return 0;
+  const int W = std::min(width, FSEQ), cols = grid_columns(FSEQ, W, patch), n = grid_groups(FSEQ, W, patch);
+  for (int g = 0; g < n; ++g)
+    for (int m = 0; m < patch * patch; ++m) {
+      if (read) read[g * patch * patch + m] = grid_read(g, m, FSEQ, W, patch, cols);
+      if (has) has[g * patch * patch + m] = grid_has(g, m, FSEQ, W, patch, cols);
+    }
+  return n;
 }
 
 int pkv_evict_merge(uint8_t *states, int32_t H, int32_t F, int32_t FSEQ, int32_t D, int32_t MMA, int32_t MMB,

@@ -102,6 +102,8 @@ def lib():
             [_c_p] * 10
         L.pkv_evict_merge.argtypes = [_c_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_p, _c_p, _c_p,
                                       _c_i32, _c_p, _c_p, _c_p, _c_p, _c_p]
+        L.pkv_patch_grid.restype = _c_i32
+        L.pkv_patch_grid.argtypes = [_c_i32, _c_i32, _c_i32, _c_p, _c_p]
         L.pkv_evict_merge_workspace_size.restype = _c_i64
         L.pkv_evict_merge_workspace_size.argtypes = [_c_i32]
         L.pkv_ragged_attn_workspace_size.restype = _c_i64
@@ -115,7 +117,7 @@ def declared_symbols() -> list[str]:
     """Entry points declared in include/pyramidkv_hip.h."""
     with open(HEADER_PATH) as f:
         txt = f.read()
-    return sorted(set(re.findall(r"^\s*(?:int|int64_t|const char \*)\s*(pkv_\w+)\s*\(", txt, re.M)))
+    return sorted(set(re.findall(r"^\s*(?:int|int32_t|int64_t|const char \*)\s*(pkv_\w+)\s*\(", txt, re.M)))
 
 
 def check(rc: int, what: str) -> None:

@@ -226,3 +226,19 @@ def test_evict_short_patches_blocks_out_of_order_and_other_heads():
 
     _evict_run(H=3, FSEQ=21 * 33, W=33, calls=calls, seed=9, weighted=True, kinds=["merge", "merge", "cyclic"],
                tamper=tamper)
+
+
+# a short last row that opens a patch row: the groups past its end have no token
+@pytest.mark.parametrize("FSEQ,W", [(128, 52), (110, 52), (70, 34), (963, 37)])
+@pytest.mark.parametrize("F,D_", [(1, 16), (3, 16), (1, 128), (3, 128)])
+def test_evict_grids_with_groups_of_no_token(FSEQ, W, F, D_):
+    """head_dim 16 runs the update's merge tiles, 128 the eviction kernels, and
+    those tiles where a block's stored ids are another grid's."""
+    calls = [[2 + F * b + f for f in range(F)] for b in range(12 // F)]
+
+    def tamper(ci, acc, dacc):
+        if ci == len(calls) - 1:
+            acc["gid"][1] = acc["gid"][1][:, ::-1]
+            dacc["gid"].copy_(to_dev(acc["gid"]))
+
+    _evict_run(H=2, FSEQ=FSEQ, W=W, calls=calls, seed=FSEQ + F, weighted=F == 1, D=D_, tamper=tamper)

@@ -152,6 +152,26 @@ def test_megacache_rollout_bit_exact(seed, block_sizes, noisy_passes, FS, W, spl
         t0 += F
 
 
+@pytest.mark.parametrize("FS,W", [(128, 52), (110, 52), (70, 34), (67, 22)])
+def test_megacache_frames_with_a_short_last_row(FS, W):
+    """Frames that are no whole number of rows: Veil patches of the last rows
+    hold fewer tokens, or none where the short row opens a patch row."""
+    rng = np.random.default_rng(FS)
+    L, H, D = 1, 3, 128
+    print(f"megacache FS={FS} W={W}", flush=True)
+    caches, ref, g = _build(L, H, D, FS, W, [[2, -1, 2]], chunks=3)
+    t0 = 0
+    for F in (3, 1, 3, 2, 3):
+        k, v = _rand_bf16(rng, F * FS, H, D), _rand_bf16(rng, F * FS, H, D)
+        caches[0].update(to_dev(k).view(1, F * FS, H, D), to_dev(v).view(1, F * FS, H, D), t0 * FS,
+                         cache_update_mode="clean")
+        ref.update(0, k, v, t0 * FS, "clean")
+        torch.cuda.synchronize()
+        _compare_pools(caches, ref, f"t0={t0} F={F}")
+        _compare_attend(caches[0], ref, 0, t0 * FS, F, _rand_bf16(rng, F * FS, H, D), f"t0={t0} F={F}")
+        t0 += F
+
+
 @pytest.mark.parametrize("how", ["permuted", "other_width"])
 def test_megacache_continues_block_by_its_stored_group_ids(how):
     """A Veil block whose stored group ids are not the ids of the update's
