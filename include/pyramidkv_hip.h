@@ -426,7 +426,8 @@ int pkv_evict_merge(uint8_t *states, int32_t num_heads, int32_t frames, int32_t 
 /* The patch grid that the merges of a frame of frame_seqlen tokens in rows of
  * width walk (patches of patch x patch tokens; the last row may be short), by
  * the kernels' own arithmetic on the host.  Returns the group count (0: no
- * grid).  read and has (NULL or patch * patch entries per group): the token
+ * grid, or a patch of more places than the frame has tokens, whose members the
+ * merges find by the tokens' group ids).  read and has (NULL or patch * patch entries per group): the token
  * that a merge reads for each member place of a group, always one of the
  * frame's, and whether the patch has that member (others are not added). */
 int32_t pkv_patch_grid(int32_t frame_seqlen, int32_t width, int32_t patch, int32_t *read, uint8_t *has);

@@ -922,6 +922,12 @@ __host__ __device__ inline int grid_columns(int FSEQ, int W, int p) { return ((W
 __host__ __device__ inline int grid_groups(int FSEQ, int W, int p) {
   return ((FSEQ - 1) / W / p + 1) * grid_columns(FSEQ, W, p);
 }
+// Whether a group's members are walked place by place: records may name any
+// patch, and one of more places than the frame has tokens would take longer to
+// walk (or overflow) than the scan of the frame's ids, which merges it instead.
+__host__ __device__ inline bool grid_walked(int FSEQ, int p) {
+  return p > 0 && static_cast<int64_t>(p) * p <= (FSEQ > 4 ? FSEQ : 4);
+}
 // first member of group g of the grid with `cols` columns
 __host__ __device__ inline int grid_first(int g, int W, int p, int cols) { return (g / cols) * p * W + (g % cols) * p; }
 __host__ __device__ inline bool grid_has(int g, int m, int FSEQ, int W, int p, int cols) {
@@ -963,7 +969,7 @@ __device__ void upd_merge_plan(const UpdArgs &a, int h, UpdShared &sh) {
   const int we = maxx + 1;
   sh.grid_cols = cols;
   sh.grid_ng = min(rows * cols, MTPA);
-  sh.grid_w = (p > 0 && rows * cols <= MTPA) ? we : 0;
+  sh.grid_w = (grid_walked(FSEQ, p) && rows * cols <= MTPA) ? we : 0;
   for (int s = 0; s < a.MMA; ++s) {
     sh.s_src[s] = kSrcNone;
     sh.s_grid[s] = -1;
@@ -996,7 +1002,7 @@ __device__ void upd_merge_plan(const UpdArgs &a, int h, UpdShared &sh) {
 // its ids (group of token t = ((t / W) / p) * columns + (t % W) / p), else 0;
 // the same in every thread (a block-wide vote).
 __device__ int stored_grid_width(const int32_t *gids, int FSEQ, int W, int p, int ng) {
-  const bool ok = W > 0 && p > 0 && ng == grid_groups(FSEQ, W, p);
+  const bool ok = W > 0 && grid_walked(FSEQ, p) && ng == grid_groups(FSEQ, W, p);
   bool bad = false;
   if (ok) {
     const int cols = grid_columns(FSEQ, W, p);
@@ -1149,8 +1155,8 @@ __device__ void upd_merge_tile(const UpdArgs &a, int h, int mt, UpdShared &sh, i
   // and pf holds the patch's chunks, loaded up front.  Otherwise, on the
   // grid of width W the members are loaded here, and without one each thread
   // scans the block's group ids (staged in LDS) for its group's tokens in
-  // ascending order -- the path of grids of more groups than an anchor holds
-  // and of blocks begun with other positions.
+  // ascending order -- the path of grids of more groups than an anchor holds,
+  // of patches larger than the frame and of blocks begun with other positions.
   auto frame = [&](int f, const uint4 *pf, auto closed_tag) {
     constexpr bool kClosed = decltype(closed_tag)::value;
     const int src_kind = sh.f_src[f];
@@ -2750,7 +2756,7 @@ int pkv_cache_update(const pkv_geometry *geo, const pkv_pools *pools, const pkv_
 }
 
 int32_t pkv_patch_grid(int32_t FSEQ, int32_t width, int32_t patch, int32_t *read, uint8_t *has) {
-  if (FSEQ <= 0 || FSEQ > kMaxMergeFseq || width <= 0 || patch <= 0 || patch > std::max(kPrePatch, FSEQ)) return 0;
+  if (FSEQ <= 0 || FSEQ > kMaxMergeFseq || width <= 0 || !grid_walked(FSEQ, patch)) return 0;
   const int W = std::min(width, FSEQ), cols = grid_columns(FSEQ, W, patch), n = grid_groups(FSEQ, W, patch);
   for (int g = 0; g < n; ++g)
     for (int m = 0; m < patch * patch; ++m) {

@@ -242,3 +242,14 @@ def test_evict_grids_with_groups_of_no_token(FSEQ, W, F, D_):
             dacc["gid"].copy_(to_dev(acc["gid"]))
 
     _evict_run(H=2, FSEQ=FSEQ, W=W, calls=calls, seed=FSEQ + F, weighted=F == 1, D=D_, tamper=tamper)
+
+
+@pytest.mark.parametrize("F", [1, 3])
+def test_evict_records_with_large_patches(F):
+    """Patches of 3 and 31 tokens a side, of more places than the frame has
+    tokens, and whose square does not fit 32 bits."""
+    recs = [O.make_merge(2, 3) for _ in range(5)]
+    for r, patch in zip(recs, (3, 31, 45, 46341, 65536)):
+        r["patch_size"] = patch
+    _evict_run(H=5, FSEQ=30 * 52, W=52, calls=[[2 + F * b + f for f in range(F)] for b in range(9 // F)], seed=3,
+               weighted=False, recs=recs)

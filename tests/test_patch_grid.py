@@ -50,9 +50,18 @@ def test_reads_stay_in_the_frame_for_every_width():
     rng = np.random.default_rng(3)
     for _ in range(300):
         fseq = int(2 ** rng.uniform(0, 13))
-        _check(fseq, int(rng.integers(1, fseq + 2)), int(rng.integers(1, min(fseq, 4) + 1)))
+        _check(fseq, int(rng.integers(1, fseq + 2)), int(rng.integers(1, 3 if fseq < 16 else 5)))
 
 
 def test_no_grid():
     lib = A.lib()
     assert [lib.pkv_patch_grid(*a, None, None) for a in ((0, 4, 2), (16, 0, 2), (16, 4, 0), (8193, 4, 2))] == [0] * 4
+
+
+def test_a_patch_larger_than_the_frame_is_not_walked():
+    """Its places would number p * p whatever the frame holds: from 1560 ** 0.5
+    on, and at sizes whose square does not fit 32 bits."""
+    walked = lambda fseq, patch: A.lib().pkv_patch_grid(fseq, 52, patch, None, None) > 0
+    assert [p for p in range(1, 2000) if walked(1560, p)] == list(range(1, 40))
+    assert not any(walked(1560, p) for p in (46341, 65536, 100000, 2**31 - 1))
+    assert all(walked(fseq, 2) for fseq in range(1, 9)) and not walked(4, 3)
