@@ -6,10 +6,11 @@
 // never leaves the GPU (the reference builds it on the host after three
 // blocking device-to-host copies, mega_plan.cc:557-568).
 //
-// The pack kernel is a gather: each work item is (segment, 32-token tile); 16
-// lanes move one 256-byte K row with 16-byte loads, the same lanes rotate
-// their 4 complex pairs in registers, V and positions are copied alongside.
-// A segment that several query chunks of a call hold is read once.
+// The pack kernels are gathers: each work item is (segment, 64-token tile), or
+// (entry of the plan's list, 32-token tile); 16 lanes move one 256-byte K row
+// with 16-byte loads, the same lanes rotate their 4 complex pairs in registers,
+// V and positions are copied alongside.  A segment that several query chunks of
+// a listed call hold is read once.
 
 #include "pkv_common.h"
 
@@ -538,10 +539,12 @@ __device__ inline void st16_nt(uint16_t *p, uint4 v) {
 // ---------------------------------------------------------------------------
 // pack
 // ---------------------------------------------------------------------------
-constexpr int kPackTok = 32;
 constexpr int kPackThreads = 256;
+// tokens per workgroup and 16-byte chunks per thread per round, of single
+// segments and of a list's entries
+constexpr int kPackTok = 64, kPackPer = 4;
+constexpr int kListTok = 32, kListPer = 2;
 constexpr int kPackListGrid = 8192;
-constexpr int kPackPer = 2;  // 16-byte chunks per thread per round
 
 struct PackArgs {
   const uint16_t *k[4], *v[4];
@@ -551,30 +554,116 @@ struct PackArgs {
   int64_t *pos_out;
   const int32_t *kind, *sg, *len, *dst;
   const int64_t *tremap;
-  const char *list;  // the plan's PackEntry list (null: one entry per segment of the arrays above)
+  const char *list;  // the plan's PackEntry list (null: the segments of the arrays above)
   Rope rope;
   int fuse;  // rope tables + tremap present
   int n_seg, tiles_per_seg, FSEQ, MTPA, D;
   int64_t capacity;
 };
 
-// One workgroup per (entry, 32-token tile).  Bound by memory, by the stores
-// above all: each query chunk's flat copy is written, but most segments of a
-// call's chunks are the same frames (a head's sink and recent frames and its
-// Anchor and Veil segments in every chunk; a Wave head's middle frames differ
-// by phase), so the plan lists each once with the places it goes to (K rotated
-// anew where the remapped time differs).  One layer of 12 heads and 3 chunks
-// (117 MB read, 274 MB written): 74 us = 5.3 TB/s, against 99 us with every
-// chunk's segments read by themselves; a copy of one source to three places
-// runs at 6.6 TB/s.  Without the rotation it takes as long.  Tiles of 64
-// tokens hold 187 registers (88 us), of 16 tokens 71 (81 us).
-// kD: the head_dim, 0 for one known only at run time.
-template <int kD>
+// One workgroup per (segment, 64-token tile).  Bound by memory: 12 heads and 3
+// chunks of 1,560-token frames, 274 MB read and as many written, 86 us = 6.4
+// TB/s; 12 heads of 64 tokens and 8 chunks, where most of the 24,900
+// workgroups find no segment, 18 us.  A 16-byte chunk of K is rotated and stored before the thread's next one, so that 64 tokens' reads
+// are in flight on few registers (all of the chunks' table entries fetched
+// first: 138 registers, 112 us; 32-token tiles of pack_list_kernel's form 133).
 __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
   // clamped RoPE table rows (t, y, x) of the tile's tokens
-  __shared__ int s_rows[kPackTok * 3];
+  __shared__ int s_rows[kPackTok][3];
+  const int cpt = a.D / 8;
+  const int seg = blockIdx.x / a.tiles_per_seg, tile = blockIdx.x % a.tiles_per_seg;
+  // every descriptor field is read before the first test, by scalar loads in
+  // one round trip (the grid covers n_seg segments, so all of them are in
+  // bounds; the descriptors do not change while the kernel runs)
+  const int kind = ld_uniform(a.kind + seg);
+  const int len = ld_uniform(a.len + seg);
+  const int64_t sg = ld_uniform(a.sg + seg);
+  const int64_t dst = ld_uniform(a.dst + seg);
+  const int64_t tr_seg = a.fuse ? ld_uniform(a.tremap + seg) : -1;
+  if (kind < 0 || kind > 3) return;
+  if (len <= 0 || tile * kPackTok >= len) return;
+  const int stride = (kind == PKV_SEG_MERGE) ? a.MTPA : a.FSEQ;
+  // a segment starts at its slot and may run on through the following slots
+  // of the pool (the legacy plan's whole-pool segments), never past the
+  // pool's end
+  if (sg < 0 || sg * stride + len > a.slots[kind] * stride || dst < 0 || dst + len > a.capacity || !a.k[kind]) return;
+  const uint16_t *sk = a.k[kind] + sg * stride * a.D;
+  const uint16_t *sv = a.v[kind] + sg * stride * a.D;
+  const int64_t *sp = a.pos[kind] ? a.pos[kind] + sg * stride * 3 : nullptr;
+  uint16_t *ok = a.k_out + dst * a.D;
+  uint16_t *ov = a.v_out + dst * a.D;
+  const bool rope = a.fuse && sp;  // uniform over the workgroup
+  // segments up to tiles_per_seg tiles long (every frame or merge anchor)
+  // take one pass; longer ones are walked tiles_per_seg tiles at a time
+  for (int64_t tok0 = tile * kPackTok; tok0 < len; tok0 += static_cast<int64_t>(a.tiles_per_seg) * kPackTok) {
+    const int ntok = static_cast<int>(min<int64_t>(kPackTok, len - tok0));
+    const int n_items = ntok * cpt;
+    if (rope) {
+      // the tile's table rows, one thread per token (the positions are
+      // read once per token instead of once per chunk)
+      __syncthreads();  // the previous tile's readers are done
+      for (int i = threadIdx.x; i < ntok; i += blockDim.x) {
+        const int64_t *pp = sp + (tok0 + i) * 3;
+        s_rows[i][0] = clamp_row(tr_seg >= 0 ? tr_seg : pp[0], a.rope.ft_rows);
+        s_rows[i][1] = clamp_row(pp[1], a.rope.fy_rows);
+        s_rows[i][2] = clamp_row(pp[2], a.rope.fx_rows);
+      }
+      __syncthreads();
+    }
+    // all of this thread's chunks of a round are loaded before any store
+    // (up to kPackPer 16-byte K and V reads in flight per thread; one round
+    // covers the tile for head_dim <= 128)
+    for (int base = 0; base < n_items; base += kPackPer * kPackThreads) {
+      uint4 kk[kPackPer], vv[kPackPer];
+#pragma unroll
+      for (int u = 0; u < kPackPer; ++u) {
+        const int i = base + threadIdx.x + u * kPackThreads;
+        if (i < n_items) {
+          const int64_t e = (tok0 + i / cpt) * a.D + (i % cpt) * 8;
+          kk[u] = ld16(sk + e);
+          vv[u] = ld16(sv + e);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kPackPer; ++u) {
+        const int i = base + threadIdx.x + u * kPackThreads;
+        if (i >= n_items) continue;
+        const int tl = i / cpt, ch = i % cpt;
+        const int64_t e = (tok0 + tl) * a.D + ch * 8;
+        uint4 k4 = kk[u];
+        if (rope) {
+          float2 f[4];
+          rope_entries(f, ch, a.rope, s_rows[tl][0], s_rows[tl][1], s_rows[tl][2]);
+          k4 = rope_rotate(k4, f);
+        }
+        st16_nt(ok + e, k4);
+        st16_nt(ov + e, vv[u]);
+      }
+    }
+    if (a.pos_out && sp) {
+      int64_t *op = a.pos_out + dst * 3;
+      for (int i = threadIdx.x; i < ntok * 3; i += blockDim.x) op[tok0 * 3 + i] = sp[tok0 * 3 + i];
+    }
+  }  // tiles of a long segment
+}
+
+// The plan's list: one workgroup per (entry, 32-token tile).  Bound by memory,
+// by the stores above all: each query chunk's flat copy is written, but most
+// segments of a call's chunks are the same frames (a head's sink and recent
+// frames and its Anchor and Veil segments in every chunk; a Wave head's middle
+// frames differ by phase), so the plan lists each once with the places it goes
+// to (K rotated anew where the remapped time differs).  One layer of 12 heads
+// and 3 chunks (117 MB read, 274 MB written), plan included: 70 us, against 93
+// with every chunk's segments read by themselves (pack_kernel).  Without the
+// rotation it takes as long.  Tiles of 64 tokens hold 187 registers (14 us
+// more), of 16 tokens 71 (7 us more).
+// kD: the head_dim, 0 for one known only at run time.
+template <int kD>
+__global__ void __launch_bounds__(kPackThreads) pack_list_kernel(PackArgs a) {
+  // clamped RoPE table rows (t, y, x) of the tile's tokens
+  __shared__ int s_rows[kListTok * 3];
   const int D = kD ? kD : a.D, cpt = D / 8;
-  const int n_ent = a.list ? ld_uniform(reinterpret_cast<const int32_t *>(a.list)) : a.n_seg;
+  const int n_ent = ld_uniform(reinterpret_cast<const int32_t *>(a.list));
   const PackEntry *entries = reinterpret_cast<const PackEntry *>(a.list + kPackListHead);
   for (int64_t it = blockIdx.x;; it += gridDim.x) {
     const int ei = static_cast<int>(it / a.tiles_per_seg), tile = static_cast<int>(it % a.tiles_per_seg);
@@ -583,22 +672,13 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
     // trip (ei < n_seg, so all of them are in bounds, with whatever value past
     // the list's end; they do not change while the kernel runs)
     PackEntry en;
-    if (a.list) {
-      const int32_t *w = reinterpret_cast<const int32_t *>(entries + ei);
+    const int32_t *w = reinterpret_cast<const int32_t *>(entries + ei);
 #pragma unroll
-      for (int i = 0; i < 12; ++i) reinterpret_cast<int32_t *>(&en)[i] = ld_uniform(w + i);
-    } else {
-      en.kind = ld_uniform(a.kind + ei);
-      en.sg = ld_uniform(a.sg + ei);
-      en.len = ld_uniform(a.len + ei);
-      en.dst[0] = ld_uniform(a.dst + ei);
-      en.tr[0] = a.fuse ? remap32(ld_uniform(a.tremap + ei)) : -1;
-      en.n_to = 1;
-    }
+    for (int i = 0; i < 12; ++i) reinterpret_cast<int32_t *>(&en)[i] = ld_uniform(w + i);
     if (ei >= n_ent) return;
     const int kind = en.kind, len = en.len;
     if (kind < 0 || kind > 3) continue;
-    if (len <= 0 || tile * kPackTok >= len) continue;
+    if (len <= 0 || tile * kListTok >= len) continue;
     const int stride = (kind == PKV_SEG_MERGE) ? a.MTPA : a.FSEQ;
     const int64_t sg = en.sg;
     // a segment starts at its slot and may run on through the following
@@ -615,22 +695,22 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
     const bool rope = a.fuse && sp;  // uniform over the workgroup
     // segments up to tiles_per_seg tiles long (every frame or merge anchor)
     // take one pass; longer ones are walked tiles_per_seg tiles at a time
-    for (int64_t tok0 = tile * kPackTok; tok0 < len; tok0 += static_cast<int64_t>(a.tiles_per_seg) * kPackTok) {
-      const int ntok = static_cast<int>(min<int64_t>(kPackTok, len - tok0));
+    for (int64_t tok0 = tile * kListTok; tok0 < len; tok0 += static_cast<int64_t>(a.tiles_per_seg) * kListTok) {
+      const int ntok = static_cast<int>(min<int64_t>(kListTok, len - tok0));
       const int n_items = ntok * cpt;
       // the tile's positions: one word per thread, written on to every copy
       // and, clamped to the tables, kept for the rotation
-      static_assert(kPackTok * 3 <= kPackThreads, "one position word per thread");
+      static_assert(kListTok * 3 <= kPackThreads, "one position word per thread");
       int64_t pw = 0;
       const bool has_pos = sp && static_cast<int>(threadIdx.x) < ntok * 3;
       if (has_pos) pw = sp[tok0 * 3 + threadIdx.x];
-      for (int base = 0; base < n_items; base += kPackPer * kPackThreads) {
+      for (int base = 0; base < n_items; base += kListPer * kPackThreads) {
         // all of this thread's chunks of a round are loaded before any store
-        // (up to kPackPer 16-byte K and V reads in flight per thread; one round
+        // (up to kListPer 16-byte K and V reads in flight per thread; one round
         // covers the tile for head_dim <= 128)
-        uint4 kk[kPackPer], vv[kPackPer];
+        uint4 kk[kListPer], vv[kListPer];
 #pragma unroll
-        for (int u = 0; u < kPackPer; ++u) {
+        for (int u = 0; u < kListPer; ++u) {
           const int i = base + threadIdx.x + u * kPackThreads;
           if (i < n_items) {
             const int e = i / cpt * D + i % cpt * 8;
@@ -656,14 +736,14 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
           if (!to[w]) continue;
           uint16_t *ov = a.v_out + (en.dst[w] + tok0) * D;
 #pragma unroll
-          for (int u = 0; u < kPackPer; ++u) {
+          for (int u = 0; u < kListPer; ++u) {
             const int i = base + threadIdx.x + u * kPackThreads;
             if (i < n_items) st16_nt(ov + (i / cpt * D + i % cpt * 8), vv[u]);
           }
         }
         // K: the table entries of all of the thread's chunks are fetched
         // together, once for copies at the same time
-        float2 f[kPackPer][4];
+        float2 f[kListPer][4];
         int at = -2;
 #pragma unroll
         for (int w = 0; w < kPackShare; ++w) {
@@ -672,7 +752,7 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
           if (rope && en.tr[w] != at) {
             at = en.tr[w];
 #pragma unroll
-            for (int u = 0; u < kPackPer; ++u) {
+            for (int u = 0; u < kListPer; ++u) {
               const int i = min(base + static_cast<int>(threadIdx.x) + u * kPackThreads, n_items - 1);
               const int tl = i / cpt, ch = i % cpt;
               const int row_t = at >= 0 ? min(at, a.rope.ft_rows - 1) : s_rows[tl * 3];
@@ -680,7 +760,7 @@ __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
             }
           }
 #pragma unroll
-          for (int u = 0; u < kPackPer; ++u) {
+          for (int u = 0; u < kListPer; ++u) {
             const int i = base + threadIdx.x + u * kPackThreads;
             if (i < n_items) st16_nt(ok + (i / cpt * D + i % cpt * 8), rope ? rope_rotate(kk[u], f[u]) : kk[u]);
           }
@@ -846,15 +926,16 @@ static int pack_launch(const pkv_geometry *geo, const pkv_pools *pools, const in
   a.D = geo->head_dim;
   a.capacity = geo->max_pack_tokens;
   const int seg_max = geo->frame_seqlen > geo->max_merge_tokens ? geo->frame_seqlen : geo->max_merge_tokens;
-  a.tiles_per_seg = (seg_max + kPackTok - 1) / kPackTok;
+  const int tok = list ? kListTok : kPackTok;
+  a.tiles_per_seg = (seg_max + tok - 1) / tok;
   const int64_t items = static_cast<int64_t>(n_segments) * a.tiles_per_seg;
   if (items > 0x7fffffff) return fail(PKV_ERR_UNSUPPORTED, "pyramidkv_pack: too many segments");
   // one workgroup per (segment, tile), inactive ones exit at once; of a list
   // most segments are inactive or another's copy, so at most kPackListGrid
   // workgroups walk it (one layer of the production shape has about 4,500 items)
   const int grid = static_cast<int>(list && items > kPackListGrid ? kPackListGrid : items);
-  if (a.D == 128) hipLaunchKernelGGL(pack_kernel<128>, dim3(grid), dim3(kPackThreads), 0, stream, a);
-  else hipLaunchKernelGGL(pack_kernel<0>, dim3(grid), dim3(kPackThreads), 0, stream, a);
+  auto *k = !list ? pack_kernel : a.D == 128 ? pack_list_kernel<128> : pack_list_kernel<0>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(kPackThreads), 0, stream, a);
   return check_launch("pack_kernel");
 }
 
