@@ -258,7 +258,7 @@ int pkv_plan_pack(const pkv_geometry *geo, const pkv_pools *pools,
  * distinct segments of its query chunks: a segment that several chunks hold
  * is then read once and written to each of their places.  Same outputs.  A
  * NULL or smaller buffer, or a size of 0 (more chunks or heads than the plan
- * can list), packs every chunk's segments by themselves. */
+ * can list, or too few tokens for a list to pay), packs every chunk's segments by themselves. */
 int64_t pkv_plan_list_size(const pkv_geometry *geo, int32_t num_chunks);
 int pkv_plan_pack_list(const pkv_geometry *geo, const pkv_pools *pools,
                        const uint8_t *states_layer, int32_t layer,

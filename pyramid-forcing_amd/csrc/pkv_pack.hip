@@ -564,9 +564,10 @@ struct PackArgs {
 // One workgroup per (segment, 64-token tile).  Bound by memory: 12 heads and 3
 // chunks of 1,560-token frames, 274 MB read and as many written, 86 us = 6.4
 // TB/s; 12 heads of 64 tokens and 8 chunks, where most of the 24,900
-// workgroups find no segment, 18 us.  A 16-byte chunk of K is rotated and stored before the thread's next one, so that 64 tokens' reads
-// are in flight on few registers (all of the chunks' table entries fetched
-// first: 138 registers, 112 us; 32-token tiles of pack_list_kernel's form 133).
+// workgroups find no segment, 18 us.  A 16-byte chunk of K is rotated and
+// stored before the thread's next one, so that 64 tokens' reads are in flight
+// on few registers (all of the chunks' table entries fetched first: 138
+// registers, 112 us; 32-token tiles of pack_list_kernel's form 133).
 __global__ void __launch_bounds__(kPackThreads) pack_kernel(PackArgs a) {
   // clamped RoPE table rows (t, y, x) of the tile's tokens
   __shared__ int s_rows[kPackTok][3];
@@ -887,6 +888,20 @@ static bool plan_lists(const pkv_geometry *g, int64_t num_chunks) {
          (num_chunks + kPackShare - 1) / kPackShare * g->num_heads * S <= kPlanThreads;
 }
 
+// Whether the list pays: the plan takes 1-5 us more with it, the pack less by
+// what is read once and by the workgroups that find no segment.  Measured, plan
+// and pack together, with and without, 1-12 heads and 64-1,560 tokens: of one
+// chunk nothing is shared and only the second part is gained, up to about 4,000
+// tokens of all heads (6 heads of 390 tokens 12.3 us against 16.7, of 693 tokens
+// 15.7 and 15.4, 12 heads of 1,560 42.8 and 37.0); of C chunks the list pays
+// from about 256 C tokens of all heads on (3 heads: C = 3, 64 tokens 13.5 and
+// 12.4, 390 tokens 14.7 and 17.9; C = 4, 64 tokens 15.2 and 13.1, 390 tokens
+// 16.5 and 18.4; 12 heads of 1,560 tokens, C = 3, 69 and 92).
+static bool plan_list_pays(const pkv_geometry *g, int64_t num_chunks) {
+  const int64_t tokens = static_cast<int64_t>(g->num_heads) * g->frame_seqlen;
+  return num_chunks == 1 ? tokens < 4096 : tokens >= 256 * num_chunks;
+}
+
 // Pack of a segment list, or of the plan's entry list of those segments
 // (list non-null).
 static int pack_launch(const pkv_geometry *geo, const pkv_pools *pools, const int32_t *src_kind,
@@ -965,7 +980,7 @@ int pkv_plan_pack(const pkv_geometry *geo, const pkv_pools *pools, const uint8_t
 }
 
 int64_t pkv_plan_list_size(const pkv_geometry *geo, int32_t num_chunks) {
-  if (!geo || num_chunks <= 0 || !plan_lists(geo, num_chunks)) return 0;
+  if (!geo || num_chunks <= 0 || !plan_lists(geo, num_chunks) || !plan_list_pays(geo, num_chunks)) return 0;
   const int64_t S = geo->max_sink + geo->max_middle + geo->max_recent + geo->max_merge_blocks;
   return kPackListHead + num_chunks * geo->num_heads * S * static_cast<int64_t>(sizeof(PackEntry));
 }

@@ -102,6 +102,8 @@ def lib():
             [_c_p] * 10
         L.pkv_evict_merge.argtypes = [_c_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_p, _c_p, _c_p,
                                       _c_i32, _c_p, _c_p, _c_p, _c_p, _c_p]
+        L.pkv_plan_list_size.restype = _c_i64
+        L.pkv_plan_list_size.argtypes = [ctypes.POINTER(Geometry), _c_i32]
         L.pkv_patch_grid.restype = _c_i32
         L.pkv_patch_grid.argtypes = [_c_i32, _c_i32, _c_i32, _c_p, _c_p]
         L.pkv_evict_merge_workspace_size.restype = _c_i64

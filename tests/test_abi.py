@@ -30,3 +30,17 @@ def test_argument_errors_are_reported_without_touching_the_device():
     assert b"NULL" in lib.pkv_last_error()
     rc = lib.pkv_plan_multi(None, None, None, None, None, 0, None, None, None, None)
     assert rc == A.PKV_ERR_INVALID
+
+
+def test_plan_list_size_rule():
+    """A list is offered where it pays: one chunk below 4,096 tokens of all
+    heads, several from 256 tokens per chunk on, and never past what the plan
+    can list."""
+    size = lambda heads, fs, chunks: A.lib().pkv_plan_list_size(
+        ctypes.byref(A.make_geometry(2, heads, 128, fs, 3, 24, 4, 1 << 20)), chunks)
+    segs = 3 + 24 + 4 + 6
+    assert size(3, 64, 1) == 64 + 3 * segs * 48 and size(13, 315, 1) > 0 and size(16, 256, 1) == 0
+    for chunks in (2, 3, 4):
+        assert size(1, 256 * chunks, chunks) == 64 + chunks * segs * 48 and size(1, 256 * chunks - 1, chunks) == 0
+    assert size(12, 1560, 3) == 64 + 3 * 12 * segs * 48
+    assert size(12, 1560, 5) == 0 and size(20, 1560, 3) == 0 and size(12, 1560, 0) == 0

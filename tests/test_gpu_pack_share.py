@@ -18,7 +18,10 @@ pytestmark = pytest.mark.gpu
 # (chunk, head) pairs than the plan lists; head_dims with their own kernel and
 # without; frames of a few tokens and of several 32-token tiles with a remainder
 @pytest.mark.parametrize("chunks,heads,D,grid", [(1, 3, 128, (6, 9)), (2, 4, 128, (8, 16)), (4, 3, 64, (7, 9)),
-                                                 (6, 3, 128, (3, 5)), (6, 12, 128, (8, 8)), (3, 5, 40, (11, 13))])
+                                                 (6, 3, 128, (3, 5)), (6, 12, 128, (8, 8)), (3, 5, 40, (11, 13)),
+                                                 # the least tokens that are listed, and one token fewer per head
+                                                 (4, 3, 64, (18, 19)), (4, 3, 64, (11, 31)), (6, 2, 128, (24, 32)),
+                                                 (3, 4, 40, (12, 16)), (1, 13, 128, (15, 21)), (1, 16, 128, (16, 16))])
 def test_shared_segments_pack_as_each_chunk_by_itself(chunks, heads, D, grid):
     from pyramidkv import factory
     from pyramidkv._mega_cache import build_mega_caches
