@@ -63,14 +63,15 @@ __device__ inline float4 residual4(float4 a, uint2 b, const float *gate, int j) 
 // (one_plus ? 1 + mul : mul) and a = add, each optional (1 and 0).  kRes
 // first applies the residual update x[r, :] += float(y[r, :]) * gate in
 // registers and writes the updated row back, so the row is read once.  K
-// vectors of 4 values per lane, guarded unless kFull (the row is exactly K * 64
-// vectors long).  Bound by memory, and, since a launch of a few thousand rows
-// has all of its waves resident at once, by the chain of reads and sums of one
-// row: K fits the row (6 vectors at 1,536 columns), the row's y is read with
-// it, and the weights are read between the two sums.  4,680 rows of 1,536:
-// 14.9 us with the residual update (86 MB, 5.8 TB/s) and 9.3 us without,
-// against 17.2 and 11.4 with 8 guarded vectors and the weights read last.
-template <int K, bool kRes, bool kFull>
+// vectors of 4 values per lane, the first kSure of them in the row on every
+// lane, the others guarded (ln_instance).  Bound by memory, and, since a launch
+// of a few thousand rows has all of its waves resident at once, by the chain of
+// reads and sums of one row: K fits the row (6 vectors at 1,536 columns), the
+// row's y is read with it, and the weights are read between the two sums.
+// 4,680 rows of 1,536: 15.0 us with the residual update (86 MB, 5.7 TB/s) and
+// 8.8 us without, against 17.5 and 10.0 with 8 guarded vectors and the weights
+// read last; of 1,280: 12.2 and 7.4, against 16.5 and 9.2 with 6 guarded ones.
+template <int K, bool kRes, int kSure>
 __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x, int64_t rows, int C,
                                                                        const float *mul, const float *add,
                                                                        int one_plus, float eps, uint16_t *out,
@@ -86,7 +87,7 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    const bool in = kFull || j < nv;
+    const bool in = k < kSure || j < nv;
     v[k] = in ? ld_f4(xr + 4 * j) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (kRes && in) yv[k] = *reinterpret_cast<const uint2 *>(y + r * y_stride + 4 * j);
   }
@@ -94,7 +95,7 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    if (kRes && (kFull || j < nv)) {
+    if (kRes && (k < kSure || j < nv)) {
       v[k] = residual4(v[k], yv[k], gate, j);
       *reinterpret_cast<float4 *>(xr + 4 * j) = v[k];
     }
@@ -108,7 +109,7 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
   if constexpr (kEarly) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const int j = kFull ? lane + 64 * k : min(lane + 64 * k, nv - 1);
+      const int j = k < kSure ? lane + 64 * k : min(lane + 64 * k, nv - 1);
       if (mul) mv[k] = ld_f4(mul + 4 * j);
       if (add) av[k] = ld_f4(add + 4 * j);
     }
@@ -117,7 +118,7 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    if (kFull || j < nv) {
+    if (k < kSure || j < nv) {
       const float a = v[k].x - mean, b = v[k].y - mean, c = v[k].z - mean, d = v[k].w - mean;
       q += (a * a + b * b) + (c * c + d * d);
     }
@@ -127,7 +128,7 @@ __global__ void __launch_bounds__(64 * kDitRowsPerBlock) ln_mod_kernel(float *x,
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int j = lane + 64 * k;
-    if (!kFull && j >= nv) continue;
+    if (k >= kSure && j >= nv) continue;
     float y[4] = {(v[k].x - mean) * rstd, (v[k].y - mean) * rstd, (v[k].z - mean) * rstd, (v[k].w - mean) * rstd};
     if (mul) {
       const float4 m = kEarly ? mv[kEarly ? k : 0] : ld_f4(mul + 4 * j);
@@ -263,20 +264,32 @@ __global__ void __launch_bounds__(256) gelu_tanh_kernel(const uint16_t *x, int64
 static int row_grid(int64_t rows);
 
 // LayerNorm rows (kRes: after the residual update from y and gate)
+// the instance for rows of `vec` vectors per lane (ln_mod_kernel), full: the
+// last one too.  Up to 8 it is exact; beyond, registers decide more than guards
+// do, and with the residual 12 vectors all guarded are the fastest (3,072
+// columns 30.5 us, 37.3 with the first 8 unguarded; without it 19.8 and 19.7).
+template <bool kRes>
+static auto *ln_instance(int vec, bool full) {
+  switch (vec) {
+    case 1: return full ? ln_mod_kernel<1, kRes, 1> : ln_mod_kernel<1, kRes, 0>;
+    case 2: return full ? ln_mod_kernel<2, kRes, 2> : ln_mod_kernel<2, kRes, 1>;
+    case 3: return full ? ln_mod_kernel<3, kRes, 3> : ln_mod_kernel<3, kRes, 2>;
+    case 4: return full ? ln_mod_kernel<4, kRes, 4> : ln_mod_kernel<4, kRes, 3>;
+    case 5: return full ? ln_mod_kernel<5, kRes, 5> : ln_mod_kernel<5, kRes, 4>;
+    case 6: return full ? ln_mod_kernel<6, kRes, 6> : ln_mod_kernel<6, kRes, 5>;
+    case 7: return full ? ln_mod_kernel<7, kRes, 7> : ln_mod_kernel<7, kRes, 6>;
+    case 8: return full ? ln_mod_kernel<8, kRes, 8> : ln_mod_kernel<8, kRes, 7>;
+    default: return vec <= 12 ? ln_mod_kernel<12, kRes, kRes ? 0 : 8> : ln_mod_kernel<kMaxVec, kRes, 12>;
+  }
+}
+
 template <bool kRes>
 static int launch_ln_k(float *x, int64_t rows, int cols, const float *mul, const float *add, int mul_plus_one,
                        float eps, uint16_t *out, const uint16_t *y, int64_t y_stride, const float *gate, hipStream_t st,
                        const char *who) {
   const int vec = (cols / 4 + 63) / 64;
   if (vec > kMaxVec) return fail(PKV_ERR_UNSUPPORTED, "%s: cols (%d) above %d", who, cols, 64 * 4 * kMaxVec);
-  const bool full = cols % 256 == 0;
-  auto *k = vec <= 2              ? ln_mod_kernel<2, kRes, false>
-            : vec <= 4            ? ln_mod_kernel<4, kRes, false>
-            : vec == 6 && full    ? ln_mod_kernel<6, kRes, true>
-            : vec <= 6            ? ln_mod_kernel<6, kRes, false>
-            : vec <= 8            ? ln_mod_kernel<8, kRes, false>
-            : vec <= 12           ? ln_mod_kernel<12, kRes, false>
-                                  : ln_mod_kernel<kMaxVec, kRes, false>;
+  auto *k = ln_instance<kRes>(vec, cols % 256 == 0);
   hipLaunchKernelGGL(k, dim3(row_grid(rows)), dim3(64 * kDitRowsPerBlock), 0, st, x, rows, cols, mul, add, mul_plus_one,
                      eps, out, y, y_stride, gate);
   return check_launch("ln_mod_kernel");

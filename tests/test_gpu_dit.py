@@ -140,7 +140,8 @@ def test_dit_residual_layer_norm_equals_the_two_ops(rows, C, gated, one_plus):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
-@pytest.mark.parametrize("C", [8, 256, 264, 512, 520, 768, 1024, 1032, 1280, 1536, 1544, 2048, 2056, 3072, 3080, 4096])
+@pytest.mark.parametrize("C", [8, 256, 264, 512, 520, 768, 776, 1024, 1032, 1280, 1288, 1536, 1544, 1792, 1800,
+                               2048, 2056, 3072, 3080, 4096])
 def test_dit_norms_at_the_edges_of_their_widths(C):
     """The norms hold a row in as many vectors per lane as it needs: widths at,
     below and above the edges of each count, a weight that starts off a
