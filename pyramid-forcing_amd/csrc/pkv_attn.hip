@@ -2199,9 +2199,8 @@ static int64_t split_items(int64_t tiles) {
 // The workspace: an entry per query tile (of which there are at most 3/2 per
 // unit), then the items' partial results.
 static int64_t split_head_bytes() { return 2 * static_cast<int64_t>(device_cus()) * static_cast<int64_t>(sizeof(int4)); }
-static int64_t split_ws_bytes() {
-  return split_head_bytes() + 3 * static_cast<int64_t>(device_cus()) * kPartFloats * 4;
-}
+static int64_t split_ws_bytes(int64_t items) { return split_head_bytes() + items * kPartFloats * 4; }
+static int64_t split_ws_max() { return split_ws_bytes(3 * static_cast<int64_t>(device_cus())); }
 
 // Query tiles of a launch that may split its keys, 0 for one that may not:
 // head_dim 128, at most kSplitMaxSeqs sequences, and tiles on at most 9/10 of
@@ -2229,10 +2228,10 @@ static int64_t split_tiles(const pkv_attn_args *a, int64_t keys) {
 
 // Key-split launch: attn_pp_kernel<true> over as many workgroups as it may
 // have items, then attn_combine_kernel.  Returns -1 when the launch does not
-// qualify (the caller then runs the plain kernels).
+// qualify or ws_bytes are too few (the caller then runs the plain kernels).
 static int launch_split(const pkv_attn_args *a, void *ws, int64_t ws_bytes, hipStream_t st) {
   const int64_t tiles = split_tiles(a, 0), n = split_items(tiles);
-  if (!ws || tiles == 0 || ws_bytes < split_ws_bytes()) return -1;
+  if (!ws || tiles == 0 || ws_bytes < split_ws_bytes(n)) return -1;
   AttnParams p{};
   p.q = a->q; p.k = a->k; p.v = a->v; p.o = a->o;
   p.cu_q = a->cu_seqlens_q; p.cu_k = a->cu_seqlens_k;
@@ -2317,20 +2316,27 @@ static int attn_check(const pkv_attn_args *a) {
   return 0;
 }
 
-extern "C" int64_t pkv_ragged_attn_workspace_size(void) { return split_ws_bytes(); }
+extern "C" int64_t pkv_ragged_attn_workspace_size(void) { return split_ws_max(); }
 
 extern "C" int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *a, int64_t keys) {
   if (!a || a->num_batches <= 0 || a->num_heads_q <= 0 || a->max_seqlen_q <= 0) return 0;
-  return split_tiles(a, keys) ? split_ws_bytes() : 0;
+  const int64_t tiles = split_tiles(a, keys);
+  return tiles ? split_ws_bytes(split_items(tiles)) : 0;
 }
 
-extern "C" int pkv_ragged_attn_fwd_ws(const pkv_attn_args *a, void *workspace, int64_t workspace_bytes,
-                                      pkv_stream_t stream) {
+extern "C" int pkv_ragged_attn_fwd_for(const pkv_attn_args *a, void *workspace, int64_t workspace_bytes,
+                                       pkv_stream_t stream) {
   const int rc = attn_check(a);
   if (rc) return rc < 0 ? rc : PKV_OK;
   const int s = launch_split(a, workspace, workspace_bytes, as_stream(stream));
   if (s >= 0) return s;
   return pkv_ragged_attn_fwd(a, stream);
+}
+
+extern "C" int pkv_ragged_attn_fwd_ws(const pkv_attn_args *a, void *workspace, int64_t workspace_bytes,
+                                      pkv_stream_t stream) {
+  // (the size that it documents, whatever this launch would need)
+  return pkv_ragged_attn_fwd_for(a, workspace_bytes < split_ws_max() ? nullptr : workspace, workspace_bytes, stream);
 }
 
 extern "C" int pkv_ragged_attn_fwd(const pkv_attn_args *a, pkv_stream_t stream) {

@@ -721,15 +721,21 @@ static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q
     return out;
   }
   // a workspace of the stream's allocator for the launches that gain from one
-  // (k's rows are those of the sequences, or a buffer's that holds them)
+  // (k's rows are those of the sequences, or a buffer's that holds them); a
+  // device without room for it runs the launch unsplit
   const int64_t mean = k.size(0) / std::max<int64_t>(1, kv_per_head ? B * Hq : B);
   const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 && max_seqlen_k < mean ? max_seqlen_k : mean);
+  Tensor w;
   if (need > 0) {
-    const Tensor w = at::empty({need}, q.options().dtype(at::kByte));
-    pkv_check(pkv_ragged_attn_fwd_ws(&a, w.data_ptr(), need, stream_for(q)), "ragged_attention");
-  } else {
-    pkv_check(pkv_ragged_attn_fwd(&a, stream_for(q)), "ragged_attention");
+    try {
+      w = at::empty({need}, q.options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError &) {
+    }
   }
+  if (w.defined())
+    pkv_check(pkv_ragged_attn_fwd_for(&a, w.data_ptr(), need, stream_for(q)), "ragged_attention");
+  else
+    pkv_check(pkv_ragged_attn_fwd(&a, stream_for(q)), "ragged_attention");
   return out;
 }
 

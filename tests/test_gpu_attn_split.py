@@ -195,3 +195,42 @@ def test_split_rows_whose_scores_are_all_minus_infinity():
     for ws in (None, _ws()):
         got = O.bf16_to_f32(_run(q, k, v, cu_q, cu_k, 1, 3, ws))
         assert np.isnan(got[:, :2]).all() and np.isfinite(got[:, 2]).all()
+
+
+def _workspace_for(batches, heads, rows, keys=0, head_dim=D):
+    return int(A.lib().pkv_ragged_attn_workspace_for(
+        A.AttnArgs(num_batches=batches, num_heads_q=heads, max_seqlen_q=rows, head_dim=head_dim), keys))
+
+
+def test_workspace_is_sized_by_the_launch():
+    """One, two or three items per compute unit, by the query tiles of 256
+    rows; the full size serves the largest."""
+    full, cus = A.ragged_attn_workspace_size(), torch.cuda.get_device_properties(0).multi_processor_count
+    sizes = [_workspace_for(1, 1, 256 * t) for t in (1, cus * 3 // 8, cus * 3 // 8 + 1, cus * 9 // 10, cus + 1)]
+    assert sizes[0] == sizes[1] < sizes[2] == sizes[3] < sizes[4] == full
+    assert full // 3 <= sizes[0] < full // 3 + 65536
+    assert _workspace_for(1, 1, 256 * cus) == _workspace_for(1, 1, 512 * cus) == _workspace_for(1, 257, 1) == 0
+    assert _workspace_for(1, 1, 256, head_dim=64) == 0
+
+
+def test_no_room_for_the_workspace_runs_unsplit():
+    """A device whose memory would not hold the workspace attends all the same
+    (the limit is the allocator's own)."""
+    rng = np.random.default_rng(67)
+    q, k, v, cu_q, cu_k = _case(rng, [300], [[9000, 7000]], 2)
+    args = [to_dev(x) for x in (q, k, v, cu_q, cu_k)]
+    plain = _run(q, k, v, cu_q, cu_k, 1, 2, None)
+    split = _ops.ragged_attention(*args, 300)
+    assert not np.array_equal(to_np(split), plain)  # other chunks, other roundings
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + (8 << 20)
+    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(_workspace_for(1, 2, 300), dtype=torch.uint8, device=DEV)
+        out = _ops.ragged_attention(*args, 300)
+        assert np.array_equal(to_np(out), plain)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(_ops.ragged_attention(*args, 300), split)
