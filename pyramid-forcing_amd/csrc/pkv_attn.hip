@@ -471,6 +471,14 @@ __device__ inline SplitItem split_item(const SplitPlan &s, int c) {
   return r;
 }
 
+// The reference that a row's probabilities are taken against: while all of its
+// scores are -inf they weigh nothing, 0 and not 2^(inf - inf).
+__device__ inline float finite_ref(float m) { return m == -INFINITY ? 0.0f : m; }
+
+// What O is scaled by at the end: 1 / the row's sum l.  A row of keys whose
+// scores are all -inf is NaN (0 / 0, here 0 * inf), one of no keys 0.
+__device__ inline float row_scale(float l, int keys) { return l > 0.0f ? 1.0f / l : (keys > 0 ? INFINITY : 0.0f); }
+
 __device__ inline uint4 ldg16(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
 
 // Buffer resource word 3 for gfx9-family raw buffers (32-bit data format,
@@ -733,7 +741,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_fwd_kernel(AttnParams p) {
     if (wave_rows) {
       f32x16 sa0 = qk(0, 0), sa1 = qk(0, 1), sb0, sb1;
       mask(sa0, sa1, 0);
-      m = tile_max(sa0, sa1);  // finite: the first tile holds key 0
+      m = tile_max(sa0, sa1);  // (-inf where all of its scores are: the slow pass)
 
       // iteration j: Ks[(j+1)%2] = K(j+1), Vs[j%2] = V(j), (c0, c1) = S(j);
       // register set j%2 holds (K(j+2), V(j+1)), stored now, then refilled
@@ -760,6 +768,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_fwd_kernel(AttnParams p) {
         step(2 * pr, sa0, sa1, sb0, sb1, sk[0], sv[0]);
         step(2 * pr + 1, sb0, sb1, sa0, sa1, sk[1], sv[1]);
       }
+      ovf |= m == -INFINITY;  // the first tile gave the row no reference
     } else {
       // no query row in this wave: stage its share of every tile, with the
       // same barriers as the steps above
@@ -805,7 +814,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_fwd_kernel(AttnParams p) {
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
         bf16x8 pb[4];
-        l = l * alpha + probs(c0, c1, m, pb);
+        l = l * alpha + probs(c0, c1, finite_ref(m), pb);
         pv(0, pb);
       }
     }
@@ -814,7 +823,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_fwd_kernel(AttnParams p) {
   // ---- epilogue: O = O^T / l, rows of 4 consecutive dims per store
   uint16_t *op = p.o + static_cast<int64_t>(q_begin) * p.o_tok + h * p.o_head;
   const float lt = half_sum(l);
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const float inv = row_scale(lt, Lk);
   if (row_q < Lq) {
     uint16_t *orow = op + static_cast<int64_t>(row_q) * p.o_tok;
 #pragma unroll
@@ -1131,7 +1140,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
       load_k(Ka);
       gemm0(sa);
       mask(sa, 0);
-      m = tile_max(sa);  // finite: the first tile holds key 0
+      m = tile_max(sa);  // (-inf where all of its scores are: the slow pass)
       load_k(Kb);
     }
     dma_v(Vc, 2);
@@ -1224,9 +1233,9 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
     wait_vm<0>();  // no copy may land in LDS after the workgroup ends
     // every tile's sums were rebased below 2^kHeadroom (or flagged)
     ovf = ovf || !(l < exp2f(kHeadroom));
-    // a chunk whose first tile scores -inf in a row has no reference for it,
-    // while the row's other chunks may hold finite scores
-    if constexpr (SPLIT) ovf = ovf || (it.k > 1 && wave_rows && m == -INFINITY);
+    // a row whose first tile scores -inf has no reference, while later keys (or
+    // the row's other chunks) may score more
+    ovf = ovf || (wave_rows && m == -INFINITY);
     if (ovf) ovf_any = 1;
     __syncthreads();
     if (ovf_any) {
@@ -1258,9 +1267,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
           bf16x8 pq[2];
-          // (in a chunk such keys weigh nothing: 0, not 2^(inf - inf); a row
-          // that has all of its keys here is NaN, as unsplit)
-          l = l * alpha + probs(s, SPLIT && it.k > 1 && m == -INFINITY ? 0.0f : m, pq);
+          l = l * alpha + probs(s, finite_ref(m), pq);
           gemm1(pq);
         }
         __syncthreads();
@@ -1286,7 +1293,7 @@ __global__ void __launch_bounds__(kThreads, 1) attn_pp_kernel(AttnParams p) {
   // ---- epilogue: O = O^T / l
   uint16_t *op = p.o + static_cast<int64_t>(q_begin) * p.o_tok + h * p.o_head;
   const float lt = half_sum(l);
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const float inv = row_scale(lt, Lk);
   if (row_q < Lq) {
     uint16_t *orow = op + static_cast<int64_t>(row_q) * p.o_tok;
 #pragma unroll
@@ -1553,12 +1560,13 @@ __device__ __attribute__((always_inline)) inline void tail_item(const AttnParams
         l *= alpha;
         m = m_new;
       }
+      const float mr = finite_ref(m);
       bf16x8 pb[2];
 #pragma unroll
       for (int ks2 = 0; ks2 < 2; ++ks2)
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj)
-          pb[ks2][jj] = static_cast<__bf16>(__builtin_amdgcn_exp2f(fmaf(sc[8 * ks2 + jj], c, -m)));
+          pb[ks2][jj] = static_cast<__bf16>(__builtin_amdgcn_exp2f(fmaf(sc[8 * ks2 + jj], c, -mr)));
       l = bf16x8_acc(pb[1], bf16x8_acc(pb[0], l));
       int va = vaddr0;
       asm volatile("" : "+v"(va));
@@ -1623,7 +1631,7 @@ __device__ __attribute__((always_inline)) inline void tail_item(const AttnParams
   }
   if (qtr != 0 || !rows) return;
   const float lt = half_sum(l);
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const float inv = row_scale(lt, Lk);
   if (row_q < Lq) {
     uint16_t *orow = p.o + static_cast<int64_t>(q_begin + row_q) * p.o_tok + h * p.o_head;
 #pragma unroll
@@ -1847,7 +1855,7 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
       load_k_half(Ka, ic<1>());
       gemm0(s);
       mask(s, 0);
-      m = tile_max(s);  // finite: the first tile holds key 0
+      m = tile_max(s);  // (-inf where all of its scores are: the slow pass)
     }
     // P < 2^kHeadroom unless a later key scores that far above the row's
     // reference, which its sum shows after the tile (rebase)
@@ -1942,8 +1950,9 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
       step();
     }
     wait_vm<0>();  // no copy may land in LDS after the workgroup ends
-    // every tile's sums were rebased below 2^kHeadroom (or flagged)
-    ovf = ovf || !(l < exp2f(kHeadroom));
+    // every tile's sums were rebased below 2^kHeadroom (or flagged); a row
+    // whose first tile scores -inf has no reference
+    ovf = ovf || !(l < exp2f(kHeadroom)) || (wave_rows && m == -INFINITY);
     if (ovf) ovf_any = 1;
     __syncthreads();
     if (ovf_any) {
@@ -1978,7 +1987,7 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
           bf16x8 pq[2];
-          l = l * alpha + probs(s2, m, pq);
+          l = l * alpha + probs(s2, finite_ref(m), pq);
           asm volatile("" ::: "memory");
           load_v_half(Va, ic<0>());
           load_v_half(Va, ic<1>());
@@ -1992,7 +2001,7 @@ __device__ __attribute__((always_inline)) inline void p3_item(const AttnParams &
   // ---- epilogue: O = O^T / l
   uint16_t *op = p.o + static_cast<int64_t>(q_begin) * p.o_tok + h * p.o_head;
   const float lt = half_sum(l);
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const float inv = row_scale(lt, Lk);
   int rq = row_q;  // the row's offset computed again, not kept from the Q load through the key loop
   asm volatile("" : "+v"(rq));
   if (rq < Lq) {
