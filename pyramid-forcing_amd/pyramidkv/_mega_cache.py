@@ -146,6 +146,8 @@ class MegaCache:
         ctx, l = self.ctx, self.layer_idx
         mgr = ctx.mgr
         backup = ctx.recent_backup.get(l)
+        if restore and backup is None:
+            raise RuntimeError(f"MegaCache: layer {l} has a pending block but no copy of its committed recent FIFO")
         if backup is None:
             backup = tuple(torch.empty_like(t[l]) for t in (mgr.recent_k_pool(), mgr.recent_v_pool(),
                                                             mgr.recent_pos_pool()))

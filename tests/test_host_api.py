@@ -249,3 +249,27 @@ def test_megacache_keeps_and_restores_the_committed_recent_fifo():
         assert all(int(t.min()) == int(t.max()) == i + 1 for i, t in enumerate(pools())), (start, F)
         for t in pools():
             t.fill_(9)
+
+
+def _cpu_cache():
+    from pyramidkv import _ops, factory
+    from pyramidkv._mega_cache import build_mega_caches
+    from pyramidkv.base import HeadComposition
+    if not _ops.available():
+        pytest.skip("torch binding not built")
+    comps = [[HeadComposition("h", 0, sink_frames=1, recent_frames=3)]]
+    return build_mega_caches(1, 1, 16, 8, 1, 1, 3, comps, max_attend_chunks=1, device="cpu", spatial_width=4,
+                             spatial_height=2, **factory.PYRAMID_FORCING_REMAP)[0]
+
+
+def test_megacache_without_a_backup_restores_nothing():
+    """A pending block whose committed FIFO was never kept (state set from
+    outside) is an error before anything is written."""
+    cache = _cpu_cache()
+    mgr = cache.ctx.mgr
+    mgr.recent_k_pool().fill_(3)
+    cache.ctx.pending_block[0] = (5, 3)
+    kv = torch.zeros(1, 8, 1, 16, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="no copy of its committed recent FIFO"):
+        cache.update(kv, kv, 64, cache_update_mode="noisy")
+    assert not cache.ctx.recent_backup and bool((mgr.recent_k_pool() == 3).all())
