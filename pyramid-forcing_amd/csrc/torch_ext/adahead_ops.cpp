@@ -1141,8 +1141,7 @@ static Tensor attend_kv_layer(const Mgr &mgr, const Tensor &states, int64_t laye
 }
 
 // The layer's recent FIFO into (or, restore, from) tensors of its pools' shapes.
-static void recent_fifo_copy(const Mgr &mgr, int64_t layer, const Tensor &k, const Tensor &v, const Tensor &pos,
-                             bool restore) {
+static void recent_fifo_copy(Mgr mgr, int64_t layer, Tensor k, Tensor v, Tensor pos, bool restore) {
   TORCH_CHECK(layer >= 0 && layer < mgr->num_layers(), "recent_fifo_copy: layer out of range");
   const c10::Device dev = mgr->valid_count().device();
   if (!dev.is_cuda() || mgr->recent_k_pool().scalar_type() != at::kBFloat16) {  // pools that no kernel updates
@@ -1162,6 +1161,14 @@ static void recent_fifo_copy(const Mgr &mgr, int64_t layer, const Tensor &k, con
                                  reinterpret_cast<uint16_t *>(v.data_ptr()), pos.data_ptr<int64_t>(), restore ? 1 : 0,
                                  stream_for(k)),
             "recent_fifo_copy");
+}
+
+static void recent_fifo_copy_layer(const Mgr &mgr, int64_t layer, const Tensor &k, const Tensor &v, const Tensor &pos,
+                                   bool restore) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("adahead::recent_fifo_copy", "")
+                             .typed<decltype(recent_fifo_copy)>();
+  op.call(mgr, layer, k, v, pos, restore);
 }
 
 // attend_kv_layer, then the attention of q [num_chunks * frame_seqlen, H, D]
@@ -1228,6 +1235,7 @@ static Tensor dit_res_ln(Tensor x, Tensor, c10::optional<Tensor>, c10::optional<
 }
 static void cache_update(Mgr, Tensor, Tensor, Tensor, Tensor, Tensor, int64_t, int64_t, int64_t, int64_t, int64_t,
                          int64_t) {}
+static void recent_fifo_copy(Mgr, int64_t, Tensor, Tensor, Tensor, bool) {}
 static void scatter_copy(Tensor, Tensor, Tensor, Tensor, int64_t) {}
 static void pos_override(Tensor, Tensor, Tensor, Tensor) {}
 static void write_frames(Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor) {}
@@ -1296,7 +1304,7 @@ TORCH_LIBRARY(adahead, m) {
            })
       .def("recent_fifo_copy",
            [](const adahead::Mgr &m, int64_t layer, const at::Tensor &k, const at::Tensor &v, const at::Tensor &pos,
-              bool restore) { adahead::recent_fifo_copy(m, layer, k, v, pos, restore); })
+              bool restore) { adahead::recent_fifo_copy_layer(m, layer, k, v, pos, restore); })
       .def("attend_kv_layer", &adahead::attend_kv_layer)
       .def("attend_layer", &adahead::attend_layer);
 
@@ -1342,6 +1350,8 @@ TORCH_LIBRARY(adahead, m) {
   m.def("ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q, Tensor cu_seqlens_k, "
         "int max_seqlen_q, float softmax_scale, bool kv_per_head=True, bool causal=False, "
         "Tensor? workspace=None, int max_seqlen_k=0) -> Tensor");
+  m.def("recent_fifo_copy(__torch__.torch.classes.adahead.PyramidKVCacheManager mgr, int layer, Tensor(a!) k, "
+        "Tensor(b!) v, Tensor(c!) pos, bool restore) -> ()");
   m.def("ragged_attention_workspace_size() -> int");
   m.def("rope_apply(Tensor k, Tensor pos, Tensor freqs_ft_flat, Tensor freqs_fy_flat, Tensor freqs_fx_flat) "
         "-> Tensor");
@@ -1403,9 +1413,11 @@ TORCH_LIBRARY_IMPL(adahead, CompositeExplicitAutograd, m) {
   m.impl("update_descriptors", adahead::update_descriptors);
   m.impl("mega_attend_kv", adahead::mega_attend_kv);
   m.impl("pyramidkv_plan", adahead::pyramidkv_plan);
+  m.impl("recent_fifo_copy", adahead::recent_fifo_copy);
 }
 
 TORCH_LIBRARY_IMPL(adahead, Meta, m) {
+  m.impl("recent_fifo_copy", adahead_meta::recent_fifo_copy);
   m.impl("pyramidkv_pack", adahead_meta::pack);
   m.impl("pyramidkv_update", adahead_meta::update);
   m.impl("mega_state_update", adahead_meta::state_update);

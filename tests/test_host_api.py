@@ -273,3 +273,20 @@ def test_megacache_without_a_backup_restores_nothing():
     with pytest.raises(RuntimeError, match="no copy of its committed recent FIFO"):
         cache.update(kv, kv, 64, cache_update_mode="noisy")
     assert not cache.ctx.recent_backup and bool((mgr.recent_k_pool() == 3).all())
+
+
+def test_recent_fifo_copies_are_seen_by_dispatch_modes():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    cache = _cpu_cache()
+    with Seen():
+        cache._recent_fifo(restore=False)
+        cache._recent_fifo(restore=True)
+    assert sum("recent_fifo_copy" in s for s in seen) == 2, seen
