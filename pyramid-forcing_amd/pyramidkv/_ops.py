@@ -7,6 +7,7 @@ there is no CPU fallback.
 """
 from __future__ import annotations
 
+import numbers
 import os
 
 import torch
@@ -78,17 +79,22 @@ def attention_workspace(device) -> torch.Tensor:
     return ws
 
 
+def _key_hint(max_seqlen_k) -> int:
+    return max(0, min(int(max_seqlen_k), 2 ** 31 - 1)) if isinstance(max_seqlen_k, numbers.Integral) else 0
+
+
 def ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_scale=None, kv_per_head=True,
                      causal=False, workspace=None, max_seqlen_k=0):
     """flash_attn_varlen_func's arithmetic (non-causal) on the ragged layout.
     Launches of a few query tiles split their keys over the compute units,
     in a workspace of the allocator's or the one given (attention_workspace);
     max_seqlen_k, an upper bound of a sequence's keys, spares launches of
-    short sequences the attempt."""
+    short sequences the attempt.  It is a hint: anything but a whole number (a
+    tensor, whose value would have to be waited for) is taken as unknown."""
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
     return ops().ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), float(softmax_scale),
-                                  bool(kv_per_head), bool(causal), workspace, int(max_seqlen_k or 0))
+                                  bool(kv_per_head), bool(causal), workspace, _key_hint(max_seqlen_k))
 
 
 def scatter_copy(src_ptrs, lengths, offsets, dst, col_dim: int) -> None:

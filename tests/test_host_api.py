@@ -290,3 +290,16 @@ def test_recent_fifo_copies_are_seen_by_dispatch_modes():
         cache._recent_fifo(restore=False)
         cache._recent_fifo(restore=True)
     assert sum("recent_fifo_copy" in s for s in seen) == 2, seen
+
+
+@pytest.mark.parametrize("hint", [None, 512, np.int32(512), 0, -1, 2 ** 40, float("inf"), 512.0, "tensor"])
+def test_flash_attn_varlen_takes_any_key_bound(hint):
+    """max_seqlen_k decides nothing but whether a split may pay: every value
+    that was accepted when nothing read it still is, and a tensor's value is
+    never asked for (a meta tensor has none)."""
+    from pyramidkv._mega_attention import flash_attn_varlen_func
+    if hint == "tensor":
+        hint = torch.empty((), dtype=torch.int32, device="meta")
+    q = torch.empty(192, 4, 128, dtype=torch.bfloat16, device="meta")
+    cu = torch.empty(4, dtype=torch.int32, device="meta")
+    assert flash_attn_varlen_func(q, q, q, cu, cu, 64, hint).shape == q.shape
