@@ -661,8 +661,8 @@ static int64_t mega_evict_merge_workspace_size(int64_t num_heads) {
 // [total_k, D] (or [total_k, 1, D]) and cu_seqlens_k has num_batches*Hq+1
 // entries (sequence b*Hq+h); otherwise k/v are [total_k, Hq, D] with
 // cu_seqlens_k [num_batches+1].  max_seqlen_k bounds a sequence's keys (0 =
-// unknown): with k's rows it tells which launches may gain from splitting
-// their keys, nothing else.  Returns the output shaped like q.
+// unknown): it tells which launches may gain from splitting their keys, nothing
+// else.  Returns the output shaped like q.
 static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q, Tensor cu_seqlens_k,
                                int64_t max_seqlen_q, double softmax_scale, bool kv_per_head, bool causal,
                                c10::optional<Tensor> workspace, int64_t max_seqlen_k) {
@@ -720,11 +720,12 @@ static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q
               "ragged_attention");
     return out;
   }
-  // a workspace of the stream's allocator for the launches that gain from one
-  // (k's rows are those of the sequences, or a buffer's that holds them); a
-  // device without room for it runs the launch unsplit
+  // a workspace of the stream's allocator for the launches that gain from one:
+  // a launch takes as long as its longest sequence, whose keys max_seqlen_k
+  // says, whatever buffer k lies in; without it k's rows per sequence stand in.
+  // A device without room for it runs the launch unsplit
   const int64_t mean = k.size(0) / std::max<int64_t>(1, kv_per_head ? B * Hq : B);
-  const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 && max_seqlen_k < mean ? max_seqlen_k : mean);
+  const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 ? max_seqlen_k : mean);
   Tensor w;
   if (need > 0) {
     try {

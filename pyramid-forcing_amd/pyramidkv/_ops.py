@@ -88,9 +88,10 @@ def ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_
     """flash_attn_varlen_func's arithmetic (non-causal) on the ragged layout.
     Launches of a few query tiles split their keys over the compute units,
     in a workspace of the allocator's or the one given (attention_workspace);
-    max_seqlen_k, an upper bound of a sequence's keys, spares launches of
-    short sequences the attempt.  It is a hint: anything but a whole number (a
-    tensor, whose value would have to be waited for) is taken as unknown."""
+    max_seqlen_k, an upper bound of a sequence's keys (without it, the rows of
+    k per sequence), spares launches of short sequences the attempt.  It is a
+    hint: anything but a whole number (a tensor, whose value would have to be
+    waited for) is taken as unknown."""
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
     return ops().ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), float(softmax_scale),

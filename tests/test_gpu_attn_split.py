@@ -234,3 +234,19 @@ def test_no_room_for_the_workspace_runs_unsplit():
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(_ops.ragged_attention(*args, 300), split)
+
+
+def test_split_by_the_longest_sequence_whatever_buffer_holds_the_keys():
+    """With max_seqlen_k the rule reads that alone: one long sequence beside
+    short ones splits, and the bits are the same where K is part of a larger
+    buffer."""
+    rng = np.random.default_rng(71)
+    H = 10
+    q, k, v, cu_q, cu_k = _case(rng, [300], [[2500] + [10 + h for h in range(H - 1)]], H)
+    plain = _run(q, k, v, cu_q, cu_k, 1, H, None)
+    room = lambda a: np.concatenate([a, np.zeros((40000, D), np.uint16)])
+    runs = [to_np(_ops.ragged_attention(to_dev(q), to_dev(kk), to_dev(vv), to_dev(cu_q), to_dev(cu_k), 300,
+                                        max_seqlen_k=2500)) for kk, vv in ((k, v), (room(k), room(v)))]
+    assert np.array_equal(*runs)
+    assert not np.array_equal(runs[0], plain)  # split: other roundings
+    _check(runs[0], q, k, v, cu_q, cu_k, H)
