@@ -223,7 +223,7 @@ class MegaCache:
         if cu_q is None or cu_q.device != q.device:
             cu_q = ctx.cu_q[L_q] = torch.arange(0, L_q + 1, FSEQ, dtype=torch.int32, device=q.device)
         qb = q[0] if q.dtype == torch.bfloat16 else q[0].to(torch.bfloat16)
-        max_keys = ctx.layer_max_keys[self.layer_idx] if ctx.layer_max_keys else 0
+        max_keys = self._max_keys(int(current_start // FSEQ) + C)
         if C <= int(ctx.mgr.max_attend_chunks()):
             scale = float(softmax_scale) if softmax_scale is not None else D ** -0.5
             out = ctx.mgr.attend_layer(*self._attend_args(current_start, C, freqs), qb, cu_q, scale, bool(causal),
@@ -234,6 +234,13 @@ class MegaCache:
                                         cu_k, FSEQ, softmax_scale, kv_per_head=True, causal=causal,
                                         workspace=self._split_workspace(q.device), max_seqlen_k=max_keys)
         return out.view(1, L_q, H, D).to(q.dtype)
+
+    def _max_keys(self, frames: int) -> int:
+        """The most keys that a head can hold once `frames` frames have come: a
+        rollout's first chunks hold fewer than the policy keeps (0 = unknown)."""
+        ctx = self.ctx
+        kept = ctx.layer_max_keys[self.layer_idx] if ctx.layer_max_keys else 0
+        return min(kept, frames * ctx.frame_seqlen)
 
 
     def _split_workspace(self, device):

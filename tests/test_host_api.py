@@ -303,3 +303,13 @@ def test_flash_attn_varlen_takes_any_key_bound(hint):
     q = torch.empty(192, 4, 128, dtype=torch.bfloat16, device="meta")
     cu = torch.empty(4, dtype=torch.int32, device="meta")
     assert flash_attn_varlen_func(q, q, q, cu, cu, 64, hint).shape == q.shape
+
+
+def test_megacache_key_bound_of_a_rollouts_first_chunks():
+    """The bound that the attention's split rule reads: the frames that have
+    come, up to what the policy keeps."""
+    cache = _cpu_cache()  # 1 sink and 3 recent frames of 8 tokens per head
+    kept = cache.ctx.layer_max_keys[0]
+    assert kept >= 4 * 8 and [cache._max_keys(n) for n in (1, 3, 1000)] == [8, 24, kept]
+    cache.ctx.layer_max_keys = []
+    assert cache._max_keys(3) == 0
