@@ -153,7 +153,8 @@ def test_split_through_the_torch_op_on_strided_views():
 ])
 def test_split_by_the_op_vs_float64(Lq, Lk, H, kv_per_head):
     """The op without a workspace, which splits by its own rule: against
-    float64, and twice with the same bits."""
+    float64, and twice with the same bits, other ones than the unsplit kernels'
+    (a chunk rounds its probabilities against its own reference)."""
     rng = np.random.default_rng(61)
     B = len(Lq)
     cu_q = np.concatenate([[0], np.cumsum(Lq)]).astype(np.int32)
@@ -164,8 +165,13 @@ def test_split_by_the_op_vs_float64(Lq, Lk, H, kv_per_head):
     print(f"attention split by the op: {B} x {H} sequences, up to {np.max(Lq)} x {np.max(Lk)}", flush=True)
     run = lambda: to_np(_ops.ragged_attention(to_dev(q), to_dev(k), to_dev(v), to_dev(cu_q), to_dev(cu_k),
                                               int(np.max(Lq)), kv_per_head=kv_per_head))
+    assert _workspace_for(B, H, int(np.max(Lq)), shape[0] // (B * H if kv_per_head else B)) > 0
     got = run()
     assert np.array_equal(got, run())
+    qd, plain = to_dev(q), torch.empty_like(to_dev(q))
+    A.ragged_attn_fwd(qd, to_dev(k), to_dev(v), plain, to_dev(cu_q), to_dev(cu_k), B, H, kv_per_head,
+                      int(np.max(Lq)), D ** -0.5)
+    assert not np.array_equal(got, to_np(plain)), "the launch did not split"
     got = O.bf16_to_f32(got).astype(np.float64)
     want = O.ragged_attention_ref(O.bf16_to_f32(q), O.bf16_to_f32(k), O.bf16_to_f32(v), cu_q, cu_k, H, kv_per_head)
     err = np.abs(got - want)
