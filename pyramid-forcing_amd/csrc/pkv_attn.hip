@@ -464,8 +464,8 @@ __device__ inline SplitItem split_item(const SplitPlan &s, int c) {
       r.j = static_cast<int>(static_cast<unsigned>(c - base) / static_cast<unsigned>(r.nq));
       r.qt = c - base - r.j * r.nq;
       r.first = base + r.qt;
-      r.u_lo = static_cast<int>(static_cast<unsigned>(r.j * nu) / static_cast<unsigned>(r.k));
-      r.u_hi = static_cast<int>(static_cast<unsigned>((r.j + 1) * nu) / static_cast<unsigned>(r.k));
+      r.u_lo = static_cast<int>(static_cast<unsigned>(r.j) * nu / static_cast<unsigned>(r.k));
+      r.u_hi = static_cast<int>(static_cast<unsigned>(r.j + 1) * nu / static_cast<unsigned>(r.k));
     }
   }
   return r;
