@@ -91,6 +91,17 @@ __device__ inline uint32_t pack_bf16x2(float lo, float hi) {
          (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
 }
 
+// The same by the hardware's round-to-nearest-even conversion, with any NaN
+// half replaced by 0x7fc0: the same bits.
+__device__ inline uint32_t cvt_bf16x2(float lo, float hi) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  if ((u & 0x7fffu) > 0x7f80u) u = (u & 0xffff0000u) | 0x7fc0u;
+  if ((u & 0x7fff0000u) > 0x7f800000u) u = (u & 0xffffu) | 0x7fc00000u;
+  return u;
+}
+
 // Read of a workgroup-uniform value that no thread writes while the kernel
 // runs (written by an earlier launch), through the constant address space:
 // the compiler issues it as a scalar load, which keeps it out of the vector

@@ -25,17 +25,6 @@ __device__ inline float wave_sum(float x) {
   return x;
 }
 
-// f32 pair -> bf16x2 by the hardware round-to-nearest-even conversion (NaN
-// halves to 0x7fc0, as pack_bf16x2)
-__device__ inline uint32_t cvt_bf16x2(float lo, float hi) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  const bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-  uint32_t u = __builtin_bit_cast(uint32_t, v);
-  if ((u & 0x7fffu) > 0x7f80u) u = (u & 0xffff0000u) | 0x7fc0u;
-  if ((u & 0x7fff0000u) > 0x7f800000u) u = (u & 0xffffu) | 0x7fc00000u;
-  return u;
-}
-
 __device__ inline float4 ld_f4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 
 // 16 bytes at any 4-byte boundary (gfx950 loads need no more)

@@ -488,17 +488,6 @@ __device__ inline PairTab pair_tab(int chunk, int e, const Rope &r) {
   return PairTab{r.fx + 2 * (pidx - fy_end), 2 * r.fx_cols, 2};
 }
 
-// f32 pair -> bf16x2 by the hardware round-to-nearest-even conversion, with
-// any NaN half replaced by 0x7fc0: the same bits as pack_bf16x2
-__device__ inline uint32_t cvt_bf16x2(float lo, float hi) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  const bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-  uint32_t u = __builtin_bit_cast(uint32_t, v);
-  if ((u & 0x7fffu) > 0x7f80u) u = (u & 0xffff0000u) | 0x7fc0u;
-  if ((u & 0x7fff0000u) > 0x7f800000u) u = (u & 0xffffu) | 0x7fc00000u;
-  return u;
-}
-
 // Table entries (cos, sin) of the 4 complex pairs of a chunk for a token's
 // clamped rows.
 __device__ inline void rope_entries(float2 (&f)[4], int chunk, const Rope &r, int row_t, int row_y, int row_x) {
