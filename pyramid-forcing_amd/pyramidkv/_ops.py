@@ -79,8 +79,10 @@ def attention_workspace(device) -> torch.Tensor:
     return ws
 
 
-def _key_hint(max_seqlen_k) -> int:
-    return max(0, min(int(max_seqlen_k), 2 ** 31 - 1)) if isinstance(max_seqlen_k, numbers.Integral) else 0
+def _key_hint(n) -> int:
+    if type(n) is not int:
+        n = int(n) if isinstance(n, numbers.Integral) else 0
+    return n if 0 <= n < 0x80000000 else (0 if n < 0 else 0x7fffffff)
 
 
 def ragged_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_scale=None, kv_per_head=True,
