@@ -998,7 +998,7 @@ def config1_entry(args):
                      "avg_launch_ms": round(at_ms, 4)},
         "roofline_pack": {"bound": "hbm", "achieved": round(pk_gbs, 2), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                           "frac": round(pk_gbs / PEAK_HBM_GBS, 4), "traffic": None,
-                          "kernel": "plan_kernel + pack_kernel", "avg_ms": round(pk_ms, 4)},
+                          "kernel": "plan_kernel + pack_list_kernel", "avg_ms": round(pk_ms, 4)},
     }
     if not args.no_cpu_baseline:
         cpu, parity = config1_cpu_and_parity(r)
@@ -1043,7 +1043,8 @@ def secondary(args):
         "packed_tokens": c3["pack_tok"], "layers": L, "heads": H, "step": 40, "policy": "shipped best_labels.csv",
         "roofline": {"bound": "hbm", "achieved": round(gbs, 2), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None,
-                     "dominant_kernel": "pack_kernel", "dominant_kernel_traffic": traffic_bytes("pack_kernel")},
+                     "dominant_kernel": "pack_list_kernel",
+                     "dominant_kernel_traffic": traffic_bytes("pack_list_kernel")},
         "plan_pack_layer0": {"ms": round(c3["plan_pack_ms_l0"], 4), "GB/s": round(pk_gbs, 2),
                              "frac": round(pk_gbs / PEAK_HBM_GBS, 4)},
         "parity_layer0_bit_exact": ok, "cpu_baseline": cpu}

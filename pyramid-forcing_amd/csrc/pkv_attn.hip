@@ -327,7 +327,7 @@ __device__ void queue_done(int *queue) {
 // into chunks, one workgroup of attn_pp_kernel<true> per (query tile, chunk);
 // attn_combine_kernel then merges a tile's chunks in chunk order.  What
 // bounds such a launch is its longest workgroup, not the chip: 42 tiles of
-// 3,000-8,000 keys took 163 us on 42 of 256 units, 49 us split over 219.
+// 5,544-6,930 keys take 154 us on 42 of 256 units, 43 + 9 us split over 219.
 //
 // Every wave of the first launch computes the same plan from cu_q / cu_k in
 // registers (no LDS, no barrier; lane i holds sequences i, i + 64, ...); the

@@ -2839,8 +2839,8 @@ int pkv_evict_merge(uint8_t *states, int32_t H, int32_t F, int32_t FSEQ, int32_t
   // tile for heads their path does not cover.  Grids that tile into 2 x 2
   // patches, with slots' ids 16-byte aligned, take the instances without
   // members to leave out (40 frames of 12 heads: 107 us on 30 x 52 tokens; on
-  // 29 x 51 108 us, against 3,708 in update_kernel, whose threads scanned the
-  // frame's ids for their group's members; one frame 12 against 108 us).
+  // 29 x 51 108 us, against 3,706 in update_kernel, whose threads scanned the
+  // frame's ids for their group's members; one frame 10.9 against 99 us).
   auto al16 = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   const int W = std::min(spatial_width, FSEQ);
   const bool grid = MMA <= 2 && grid_groups(FSEQ, W, kPrePatch) <= MTPA && FSEQ <= kEvMaxFseq && D >= 8 * kPreTok &&
