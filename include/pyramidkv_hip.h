@@ -370,8 +370,10 @@ int pkv_ragged_attn_fwd(const pkv_attn_args *args, pkv_stream_t stream);
  * these arguments in pkv_ragged_attn_fwd_for (a third of the full size for a
  * launch of one item per compute unit), 0 where none would be used or gain
  * anything; keys is the number of keys a sequence is expected to have (0 =
- * unknown). */
+ * unknown).  pkv_ragged_attn_workspace_bound: the same where no sequence has
+ * more than max_keys. */
 int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *args, int64_t keys);
+int64_t pkv_ragged_attn_workspace_bound(const pkv_attn_args *args, int64_t max_keys);
 int64_t pkv_ragged_attn_workspace_size(void);
 int pkv_ragged_attn_fwd_ws(const pkv_attn_args *args, void *workspace, int64_t workspace_bytes,
                            pkv_stream_t stream);

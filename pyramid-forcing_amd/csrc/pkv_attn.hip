@@ -2333,6 +2333,15 @@ extern "C" int64_t pkv_ragged_attn_workspace_for(const pkv_attn_args *a, int64_t
   return tiles ? split_ws_bytes(split_items(tiles)) : 0;
 }
 
+// Where no sequence has more than a shortest chunk and the fixed part of units,
+// split_plan splits none (each of its estimates is longer), so the second
+// launch is saved: 126 tiles, one sequence of 1,016 keys, the others of 63: 32
+// us, 36 with it.
+extern "C" int64_t pkv_ragged_attn_workspace_bound(const pkv_attn_args *a, int64_t max_keys) {
+  if (max_keys > 0 && max_keys <= (kSplitMinUnits + kSplitFixedUnits) * 32 * kSplitUnit) return 0;
+  return pkv_ragged_attn_workspace_for(a, max_keys);
+}
+
 extern "C" int pkv_ragged_attn_fwd_for(const pkv_attn_args *a, void *workspace, int64_t workspace_bytes,
                                        pkv_stream_t stream) {
   const int rc = attn_check(a);

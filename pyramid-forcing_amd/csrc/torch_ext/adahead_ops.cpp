@@ -725,7 +725,8 @@ static Tensor ragged_attention(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens_q
   // says, whatever buffer k lies in; without it k's rows per sequence stand in.
   // A device without room for it runs the launch unsplit
   const int64_t mean = k.size(0) / std::max<int64_t>(1, kv_per_head ? B * Hq : B);
-  const int64_t need = pkv_ragged_attn_workspace_for(&a, max_seqlen_k > 0 ? max_seqlen_k : mean);
+  const int64_t need =
+      max_seqlen_k > 0 ? pkv_ragged_attn_workspace_bound(&a, max_seqlen_k) : pkv_ragged_attn_workspace_for(&a, mean);
   Tensor w;
   if (need > 0) {
     try {

@@ -112,6 +112,8 @@ def lib():
         L.pkv_ragged_attn_workspace_size.argtypes = []
         L.pkv_ragged_attn_workspace_for.restype = _c_i64
         L.pkv_ragged_attn_workspace_for.argtypes = [ctypes.POINTER(AttnArgs), _c_i64]
+        L.pkv_ragged_attn_workspace_bound.restype = _c_i64
+        L.pkv_ragged_attn_workspace_bound.argtypes = [ctypes.POINTER(AttnArgs), _c_i64]
         L.pkv_ragged_attn_fwd_ws.argtypes = [_c_p, _c_p, _c_i64, _c_p]
         L.pkv_ragged_attn_fwd_for.argtypes = [_c_p, _c_p, _c_i64, _c_p]
         _lib = L

@@ -217,6 +217,10 @@ def test_workspace_is_sized_by_the_launch():
     assert full // 3 <= sizes[0] < full // 3 + 65536
     assert _workspace_for(1, 1, 256 * cus) == _workspace_for(1, 1, 512 * cus) == _workspace_for(1, 257, 1) == 0
     assert _workspace_for(1, 1, 256, head_dim=64) == 0
+    # no sequence long enough for two chunks and what a second launch costs
+    bound = lambda keys: int(A.lib().pkv_ragged_attn_workspace_bound(
+        A.AttnArgs(num_batches=1, num_heads_q=3, max_seqlen_q=256, head_dim=D), keys))
+    assert bound(1024) == 0 and bound(1025) == bound(0) == sizes[0] == _workspace_for(1, 3, 256, 1024)
 
 
 def test_no_room_for_the_workspace_runs_unsplit():
